@@ -176,17 +176,27 @@ __device__ __forceinline__ float row_sum16(float s) {
   return s;
 }
 
+// The same sum added in the order of the one-query kernels' shuffles (lanes 8, then 4, 2
+// and 1 apart: rotations by that much reach the same partner sums), for their bits.
+__device__ __forceinline__ float row_sum16_apart(float s) {
+  s += dpp_f32<0x128>(s);  // row_ror:8
+  s += dpp_f32<0x124>(s);  // row_ror:4
+  s += dpp_f32<0x122>(s);  // row_ror:2
+  s += dpp_f32<0x121>(s);  // row_ror:1
+  return s;
+}
+
 // Document end of the shared-tile kernels: NB query blocks of two 16-token halves, each
 // half's running max rmax[j][h] in the MFMA accumulator layout (lane (c, g): the max over
 // its rows of query token c). The row swaps move two accumulators at a time: register P
-// holds blocks 2P and 2P + 1 (block 0 alone when NB == 1), and its 16-lane row k ends with
-// the document's max of accumulator (2P + (k & 1), k >> 1) (of (0, k >> 1) when NB == 1),
+// holds blocks 2P and 2P + 1 (the last block alone when NB is odd), and its 16-lane row k
+// ends with the document's max of accumulator (2P + (k & 1), k >> 1) (of (2P, k >> 1) alone),
 // so the query masks and scales of each lane's row are picked once, by init(). Each block
-// sums (0 + half 0) + half 1 per query token and then its 16 tokens by row_sum16: the bits
-// of reducing every accumulator on its own.
+// sums (0 + half 0) + half 1 per query token and then its 16 tokens by row_sum16_apart: the
+// bits of the one-query kernels.
 template <int NB, bool QSCALE>
 struct DocEnd {
-  static constexpr int NPK = NB == 1 ? 1 : NB / 2;
+  static constexpr int NPK = (NB + 1) / 2;
   bool qv_pk[NPK];
   float qinv_pk[QSCALE ? NPK : 1];
 
@@ -198,7 +208,7 @@ struct DocEnd {
       if constexpr (QSCALE) qinv_pk[P] = 1.f;
 #pragma unroll
       for (int k = 0; k < 4; k++) {
-        const int j = NB == 1 ? 0 : 2 * P + (k & 1), h = k >> 1;
+        const int j = 2 * P + 1 < NB ? 2 * P + (k & 1) : 2 * P, h = k >> 1;
         if (krow == k) {
           qv_pk[P] = qv[j][h];
           if constexpr (QSCALE) qinv_pk[P] = qinv[j][h];
@@ -224,23 +234,24 @@ struct DocEnd {
 #pragma unroll
     for (int P = 0; P < NPK; P++) {
       float x;
-      if constexpr (NB == 1) {
-        const float p0 = swap_max32(rmax[0][0], rmax[0][1]);
-        x = swap_max16(p0, p0);
-      } else {
-        const float p0 = swap_max32(rmax[2 * P][0], rmax[2 * P][1]);
-        const float p1 = swap_max32(rmax[2 * P + 1][0], rmax[2 * P + 1][1]);
+      const float p0 = swap_max32(rmax[2 * P][0], rmax[2 * P][1]);
+      if (2 * P + 1 < NB) {
+        const int last = 2 * P + 1 < NB ? 2 * P + 1 : 0;  // in range also where the branch is not taken
+        const float p1 = swap_max32(rmax[last][0], rmax[last][1]);
         x = swap_max16(p0, p1);
+      } else {
+        x = swap_max16(p0, p0);
       }
       if constexpr (QSCALE) x *= qinv_pk[P];  // exact: a power of two
       if (padded) x = fmaxf(x, 0.f);
       x = 0.f + (qv_pk[P] ? x : 0.f);
       const auto q = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, x), __builtin_bit_cast(unsigned, x),
                                                       false, false);
-      const float sm = row_sum16(__builtin_bit_cast(float, (unsigned)q[0]) + __builtin_bit_cast(float, (unsigned)q[1]));
+      const float sm = row_sum16_apart(__builtin_bit_cast(float, (unsigned)q[0]) + __builtin_bit_cast(float, (unsigned)q[1]));
 #pragma unroll
-      for (int b = 0; b < (NB == 1 ? 1 : 2); b++) {
-        const int j = NB == 1 ? 0 : 2 * P + b;
+      for (int b = 0; b < 2; b++) {
+        const int j = 2 * P + b;
+        if (j >= NB) break;
         const float v = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, sm), 16 * b));
         pend[j] = lane == doc_lane ? v : pend[j];
       }

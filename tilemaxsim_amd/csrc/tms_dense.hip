@@ -18,7 +18,7 @@ int run_stream(const void* Q, int64_t nQ, int64_t nq, int64_t d, const void* D, 
                const int64_t* offsets, const uint8_t* mask, int64_t T, int64_t pad_len, int dtype, float* out,
                hipStream_t st);
 constexpr int64_t kMaskedStreamMaxTokens = 1024;  // masked: a wave's 64 lanes hold a document's tile masks
-// Variable-length documents, d in {32, 64, 96, 128}, several query blocks (tms_stream.hip).
+// Variable-length documents, d in {32, 64, 96, 128}, several query blocks (tms_batched.hip).
 int run_varlen_batched(const void* Q, int64_t nQ, int64_t nq, int64_t d, const void* D, int64_t T,
                        const int64_t* offsets, int64_t nd, int64_t B, int64_t pad_len, int dtype, float* out,
                        hipStream_t st, bool q32);
@@ -153,7 +153,9 @@ static int dense_entry(const char* fn, const void* Q, int64_t nQ, int64_t nq, in
   if (qreg && nQ * a.nbq <= 3 && rerank_fits(B, hint))
     return run_rerank(Q, nQ, nq, d, D, B, nd, total_tokens, offsets, mask, pad_len, mode, dtype, out, st);
   if (mode == MODE_FIXED && qreg) return run_stream(Q, nQ, nq, d, D, B, nd, nullptr, nullptr, 0, 0, dtype, out, st);
-  if (mode == MODE_VARLEN && qreg && a.nbq <= 4 && nQ * a.nbq >= 4)  // one pass for up to 32 blocks
+  // one pass for up to 32 blocks, from three queries on (one or two blocks a pass is the
+  // stream kernel's; 50,000 x 180 tokens, three queries: two passes 707 us, one 430)
+  if (mode == MODE_VARLEN && qreg && a.nbq <= 4 && (nQ * a.nbq >= 4 || nQ == 3))
     return run_varlen_batched(Q, nQ, nq, d, D, total_tokens, offsets, 0, B, pad_len, dtype, out, st, false);
   // variable-length documents against one or two query blocks per pass: the stream kernel,
   // whose walk reads each wave's document bounds from its lanes (no rows: the general kernel)
