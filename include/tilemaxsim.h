@@ -28,6 +28,7 @@ extern "C" {
 #define TMS_ERR_INVALID 1     /* bad argument (shape, pointer, offsets) */
 #define TMS_ERR_UNSUPPORTED 2 /* valid but not implemented (dtype, size limit) */
 #define TMS_ERR_HIP 3         /* the HIP runtime reported an error */
+#define TMS_ERR_BOUNDS 4      /* a *_checked call: document bounds or ids out of range */
 
 #define TMS_DTYPE_F16 0
 #define TMS_DTYPE_BF16 1
@@ -301,6 +302,35 @@ int tms_maxsim_residual_batched(const void* Qs, int64_t nQ, int64_t nq, int64_t 
                                 int64_t ncent, const void* bucket_weights, int nbits, const int32_t* codes,
                                 const uint8_t* residuals, int64_t total_tokens, const int64_t* offsets, int64_t ndocs,
                                 const int64_t* pids, int64_t B, int64_t pad_len, float* out, void* stream);
+
+/*
+ * The calls above with their document bounds checked on the device: a check kernel, then the
+ * scoring kernels, then the host waits for the check's verdict (not for the scores) and
+ * returns TMS_ERR_BOUNDS when offsets decrease or leave [0, total_tokens], or a pid leaves
+ * [0, ndocs); the scores of such a call are not to be used. zero_pad != 0 scores as if
+ * zero-padded to the longest scored document, whose length the check finds. B >= 1.
+ *   parts    device memory, TMS_CHECK_PARTS int64, any content; may be NULL without zero_pad
+ *   verdict  pinned host memory (hipHostMalloc), TMS_CHECK_PARTS int64, used by one call at a
+ *            time; NULL: nothing is waited for or refused (invalid documents score NaN). With
+ *            a verdict the stream must not be under capture (TMS_ERR_HIP).
+ * tms_maxsim_packed_checked takes lengths (1 <= B <= TMS_PACKED_SCAN_MAX) and writes their
+ * offsets (B + 1). tms_maxsim_residual_checked scores as tms_maxsim_residual (nQ = 1), or as
+ * tms_maxsim_residual_batched when `batched` is not 0. They replace the reference's host-side
+ * length handling before its PLAID scorer (src/plaid_integration_benchmark.py:162-174).
+ */
+#define TMS_CHECK_PARTS 64
+#define TMS_PACKED_SCAN_MAX 16384
+int tms_maxsim_varlen_checked(const void* Qs, int64_t nQ, int64_t nq, int64_t d, const void* D_flat,
+                              int64_t total_tokens, const int64_t* offsets, int64_t B, int zero_pad, int dtype,
+                              float* out, int64_t* parts, int64_t* verdict, void* stream);
+int tms_maxsim_packed_checked(const void* Q, int64_t nq, int64_t d, const void* D_packed, int64_t total_tokens,
+                              const int64_t* lengths, int64_t B, int zero_pad, int dtype, float* out, int64_t* offsets,
+                              int64_t* parts, int64_t* verdict, void* stream);
+int tms_maxsim_residual_checked(const void* Qs, int64_t nQ, int64_t nq, int64_t d, const void* centroids,
+                                int64_t ncent, const void* bucket_weights, int nbits, const int32_t* codes,
+                                const uint8_t* residuals, int64_t total_tokens, const int64_t* offsets, int64_t ndocs,
+                                const int64_t* pids, int64_t B, int zero_pad, int batched, float* out, int64_t* parts,
+                                int64_t* verdict, void* stream);
 
 /*
  * Measurement helper, not part of the scoring path and with no counterpart in the

@@ -18,6 +18,7 @@ TMS_OK = 0
 TMS_ERR_INVALID = 1
 TMS_ERR_UNSUPPORTED = 2
 TMS_ERR_HIP = 3
+TMS_ERR_BOUNDS = 4
 
 TMS_DTYPE_F16 = 0
 TMS_DTYPE_BF16 = 1
@@ -29,6 +30,8 @@ TMS_READ_PROBE_SINK_WORDS = 524288  # words of the sink tms_read_probe writes
 TMS_LDS_PROBE_WAVES = 4096  # waves of one tms_lds_probe launch (one cycle count each)
 TMS_MAXSIM_TOPK_COUNTER_WORDS = 144  # 32-bit words of tms_maxsim_topk's zeroed ticket block
 TMS_MFMA_PROBE_SINK_WORDS = 131072  # words of the sink tms_mfma_probe writes
+TMS_CHECK_PARTS = 64  # words of a *_checked call's parts (device) and verdict (pinned host)
+TMS_PACKED_SCAN_MAX = 16384  # documents tms_maxsim_packed_checked takes
 
 _c_void_p = ctypes.c_void_p
 _i64 = ctypes.c_int64
@@ -66,6 +69,13 @@ SIGNATURES = {
                              _c_void_p, _c_void_p],
     "tms_maxsim_residual_batched": [_c_void_p, _i64, _i64, _i64, _c_void_p, _i64, _c_void_p, _int, _c_void_p,
                                     _c_void_p, _i64, _c_void_p, _i64, _c_void_p, _i64, _i64, _c_void_p, _c_void_p],
+    "tms_maxsim_varlen_checked": [_c_void_p, _i64, _i64, _i64, _c_void_p, _i64, _c_void_p, _i64, _int, _int, _c_void_p,
+                                  _c_void_p, _c_void_p, _c_void_p],
+    "tms_maxsim_packed_checked": [_c_void_p, _i64, _i64, _c_void_p, _i64, _c_void_p, _i64, _int, _int, _c_void_p,
+                                  _c_void_p, _c_void_p, _c_void_p, _c_void_p],
+    "tms_maxsim_residual_checked": [_c_void_p, _i64, _i64, _i64, _c_void_p, _i64, _c_void_p, _int, _c_void_p, _c_void_p,
+                                    _i64, _c_void_p, _i64, _c_void_p, _i64, _int, _int, _c_void_p, _c_void_p, _c_void_p,
+                                    _c_void_p],
 }
 RESTYPES = {"tms_topk_workspace_size": ctypes.c_int64, "tms_set_rerank_limit": ctypes.c_int64}
 
@@ -119,11 +129,31 @@ def check(status: int) -> None:
     if status == TMS_OK:
         return
     msg = load().tms_last_error().decode(errors="replace")
-    if status == TMS_ERR_INVALID:
+    if status in (TMS_ERR_INVALID, TMS_ERR_BOUNDS):
         raise ValueError(msg)
     if status == TMS_ERR_UNSUPPORTED:
         raise NotImplementedError(msg)
     raise TileMaxSimError(msg)
+
+
+_thread = threading.local()
+
+
+def verdict_ptr() -> int:
+    """Address of the calling thread's verdict words (pinned host memory). A ``*_checked``
+    call waits for its own verdicts before it returns, so a thread's words are never
+    shared; they go back to torch's pinned-memory pool when the thread ends."""
+    v = getattr(_thread, "verdict", None)
+    if v is None:
+        v = _thread.verdict = torch.zeros(TMS_CHECK_PARTS, dtype=torch.int64, pin_memory=True)
+    return v.data_ptr()
+
+
+def check_bounds(status: int, msg: str) -> None:
+    """:func:`check`, with ``msg`` for the bounds a ``*_checked`` call refused."""
+    if status == TMS_ERR_BOUNDS:
+        raise ValueError(msg)
+    check(status)
 
 
 def dtype_code(dt: torch.dtype) -> int:

@@ -11,7 +11,7 @@ int run_batched_q32(const BatchedArgs& a, int64_t nQ, int64_t tokens_per_doc, in
 // D, queries of at most 4 blocks (2 for fp32 queries; q32: fp32 queries against 16-bit
 // rows). offsets null: documents of nd tokens back to back.
 int run_varlen_batched(const void* Q, int64_t nQ, int64_t nq, int64_t d, const void* D, int64_t T,
-                       const int64_t* offsets, int64_t nd, int64_t B, int64_t pad_len, int dtype, float* out,
+                       const int64_t* offsets, int64_t nd, int64_t B, PadLen pad, int dtype, float* out,
                        hipStream_t st, bool q32) {
   BatchedArgs a;
   memset(&a, 0, sizeof(a));
@@ -21,7 +21,7 @@ int run_varlen_batched(const void* Q, int64_t nQ, int64_t nq, int64_t d, const v
   a.out = out;
   a.B = B;
   a.T = T;
-  a.pad_len = pad_len;
+  a.pad = pad;
   a.nd = nd;
   a.nq = (int32_t)nq;
   a.nbq = (int32_t)((nq + 31) / 32);

@@ -9,7 +9,7 @@
 // scores tile i. The MFMA cluster runs at raised wave priority, so a wave that has its
 // operands keeps the matrix pipe fed ahead of the other wave's bookkeeping; the running
 // max takes two v_max3 per fragment and each document's reduction uses the row swaps and
-// DPP. pad_len > 0 gives the zero-padding semantics of tms_maxsim_varlen_padded; invalid
+// DPP. pad > 0 gives the zero-padding semantics of tms_maxsim_varlen_padded; invalid
 // offsets score NaN.
 //
 // Workgroup forms. Bound by the matrix cores (a step's MFMA time is the blocks a SIMD's
@@ -40,7 +40,8 @@ struct BatchedArgs {
   const int64_t* offsets;   // (B + 1), or null: document b is rows [b * nd, (b + 1) * nd)
   const uint8_t* codebook;  // PQ: (M, K, dsub) elements of the input dtype
   float* out;               // (nQ, B)
-  int64_t B, T, pad_len, nd;
+  int64_t B, T, nd;
+  PadLen pad;
   int32_t nq, nbq, blk0, blk_end, d, docs_per_wg, M, K;
   int32_t nblk_l, nblk_x;  // blocks of each wave 0-3 and of each wave 4-7 (whole queries)
 };
@@ -202,6 +203,7 @@ __device__ __forceinline__ void batched_body(const BatchedArgs& a, BatchedRing<S
       dlen = (int32_t)(e0 - s0);
     }
   }
+  const int64_t pad_len = pad_length(a.pad, lane);
   float pend[NB];  // lane j: scores of document b_begin + j
 #pragma unroll
   for (int j = 0; j < NB; j++) pend[j] = NEG_INF;
@@ -231,7 +233,7 @@ __device__ __forceinline__ void batched_body(const BatchedArgs& a, BatchedRing<S
         return;
       }
       if (record) {  // invalid offsets (len < 0): the final store writes NaN for the lane
-        const float v = a.pad_len > 0 ? 0.f : NEG_INF;
+        const float v = pad_len > 0 ? 0.f : NEG_INF;
 #pragma unroll
         for (int j = 0; j < NB; j++) pend[j] = lane == (int)(b - b_begin) ? v : pend[j];
       }
@@ -347,7 +349,7 @@ __device__ __forceinline__ void batched_body(const BatchedArgs& a, BatchedRing<S
         for (int h = 0; h < 2; h++)
           rmax[j][h] = fmaxf(fmaxf(fmaxf(fmaxf(rmax[j][h], acc[j][h][0]), acc[j][h][1]), acc[j][h][2]), acc[j][h][3]);
       if (wc.t0 + 16 >= wc.len) {  // document wc.b ends with this tile
-        const bool padded = wc.len < a.pad_len;
+        const bool padded = wc.len < pad_len;
         doc_end.finish(rmax, padded, lane, (int)(wc.b - b_begin), pend);
       }
       advance(wc, true);

@@ -262,6 +262,24 @@ struct DocEnd {
   }
 };
 
+// The zero-padding length of a call (0: none): a number, or the largest of up to 64 numbers
+// that an earlier kernel on the stream left in device memory.
+struct PadLen {
+  int64_t len;
+  const int64_t* parts;
+  int32_t nparts;
+};
+__device__ __forceinline__ int64_t pad_length(const PadLen& p, int lane) {
+  if (p.parts == nullptr) return p.len;  // uniform
+  int64_t m = lane < p.nparts ? p.parts[lane] : 0;
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) {
+    const int64_t x = __shfl_xor(m, o);
+    m = x > m ? x : m;
+  }
+  return wave_uniform(m);
+}
+
 // Per-thread last-error text behind tms_last_error().
 void set_error(const char* fmt, ...);
 int fail(int code, const char* fmt, ...);

@@ -8,6 +8,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include "tms_check.h"
 #include "tms_dense_kernel.h"
 
 namespace tms {
@@ -15,17 +16,17 @@ namespace tms {
 // Fixed-length documents (offsets null) or documents at offsets into T >= 1 rows, d in
 // {32, 64, 96, 128} (tms_stream.hip).
 int run_stream(const void* Q, int64_t nQ, int64_t nq, int64_t d, const void* D, int64_t B, int64_t nd,
-               const int64_t* offsets, const uint8_t* mask, int64_t T, int64_t pad_len, int dtype, float* out,
+               const int64_t* offsets, const uint8_t* mask, int64_t T, PadLen pad, int dtype, float* out,
                hipStream_t st);
 constexpr int64_t kMaskedStreamMaxTokens = 1024;  // masked: a wave's 64 lanes hold a document's tile masks
 // Variable-length documents, d in {32, 64, 96, 128}, several query blocks (tms_batched.hip).
 int run_varlen_batched(const void* Q, int64_t nQ, int64_t nq, int64_t d, const void* D, int64_t T,
-                       const int64_t* offsets, int64_t nd, int64_t B, int64_t pad_len, int dtype, float* out,
+                       const int64_t* offsets, int64_t nd, int64_t B, PadLen pad, int dtype, float* out,
                        hipStream_t st, bool q32);
 // Small batches (candidate reranking), documents split over several waves (tms_rerank.hip).
 bool rerank_fits(int64_t B, int64_t tokens_per_doc);
 int run_rerank(const void* Q, int64_t nQ, int64_t nq, int64_t d, const void* D, int64_t B, int64_t nd, int64_t T,
-               const int64_t* offsets, const uint8_t* mask, int64_t pad_len, int mode, int dtype, float* out,
+               const int64_t* offsets, const uint8_t* mask, PadLen pad, int mode, int dtype, float* out,
                hipStream_t st);
 // fp32 queries against fp16 / bf16 documents (tms_dense_q32.hip).
 int run_dense_q32(DenseArgs a, int64_t nQ, int dtype, int mode, bool aligned, hipStream_t st);
@@ -94,12 +95,12 @@ static int pick_docs_per_wave(int64_t B, int64_t tokens_per_doc_hint, bool f32, 
 
 static int dense_entry(const char* fn, const void* Q, int64_t nQ, int64_t nq, int64_t d, const void* D, int64_t B,
                        int64_t nd, int64_t total_tokens, const int64_t* offsets, const uint8_t* mask, int mode,
-                       int dtype, float* out, void* stream, int64_t pad_len = 0) {
+                       int dtype, float* out, void* stream, PadLen pad = PadLen{0, nullptr, 0}) {
   const bool q32 = (dtype & TMS_QUERY_F32) != 0;  // fp32 queries (implied for fp32 documents)
   dtype &= ~TMS_QUERY_F32;
   if (dtype != TMS_DTYPE_F16 && dtype != TMS_DTYPE_BF16 && dtype != TMS_DTYPE_F32)
     return fail(TMS_ERR_UNSUPPORTED, "%s: unsupported dtype %d", fn, dtype);
-  if (pad_len < 0) return fail(TMS_ERR_INVALID, "%s: negative pad_len %lld", fn, (long long)pad_len);
+  if (pad.len < 0) return fail(TMS_ERR_INVALID, "%s: negative pad_len %lld", fn, (long long)pad.len);
   if (nQ < 0 || nq < 0 || d < 0 || B < 0 || nd < 0 || total_tokens < 0)
     return fail(TMS_ERR_INVALID, "%s: negative size (nQ=%lld nq=%lld d=%lld B=%lld nd=%lld T=%lld)", fn, (long long)nQ,
                 (long long)nq, (long long)d, (long long)B, (long long)nd, (long long)total_tokens);
@@ -135,7 +136,7 @@ static int dense_entry(const char* fn, const void* Q, int64_t nQ, int64_t nq, in
   if (a.nkg < 1) a.nkg = 1;
   int64_t hint = (mode == MODE_VARLEN) ? (B > 0 ? total_tokens / B : 0) : nd;
   a.docs_per_wave = pick_docs_per_wave(B, hint, dtype == TMS_DTYPE_F32, d);
-  a.pad_len = pad_len;
+  a.pad = pad;
   a.mask4 = (nd % 4 == 0 && ((uintptr_t)mask & 3) == 0) ? 1 : 0;
   const bool aligned = (d % 8 == 0) && (((uintptr_t)Q & 15) == 0) && (((uintptr_t)D & 15) == 0);
   const bool qreg = aligned && d > 0 && d <= 128 && d % 32 == 0;
@@ -144,31 +145,38 @@ static int dense_entry(const char* fn, const void* Q, int64_t nQ, int64_t nq, in
   // two blocks
   if ((dtype == TMS_DTYPE_F32 || q32) && mode != MODE_MASKED && qreg && a.nbq <= 2 && nQ * a.nbq > 2)
     return run_varlen_batched(Q, nQ, nq, d, D, mode == MODE_VARLEN ? total_tokens : B * nd,
-                              mode == MODE_VARLEN ? offsets : nullptr, nd, B, pad_len, dtype, out, st,
+                              mode == MODE_VARLEN ? offsets : nullptr, nd, B, pad, dtype, out, st,
                               dtype != TMS_DTYPE_F32);
   if (dtype == TMS_DTYPE_F32) return run_dense<TMS_DTYPE_F32, TMS_DTYPE_F32>(a, nQ, mode, aligned, st);
   if (q32) return run_dense_q32(a, nQ, dtype, mode, aligned, st);
   // a few thousand documents or fewer against one or two query blocks: each document split
   // over up to four waves, so that small calls still fill the chip
   if (qreg && nQ * a.nbq <= 3 && rerank_fits(B, hint))
-    return run_rerank(Q, nQ, nq, d, D, B, nd, total_tokens, offsets, mask, pad_len, mode, dtype, out, st);
-  if (mode == MODE_FIXED && qreg) return run_stream(Q, nQ, nq, d, D, B, nd, nullptr, nullptr, 0, 0, dtype, out, st);
+    return run_rerank(Q, nQ, nq, d, D, B, nd, total_tokens, offsets, mask, pad, mode, dtype, out, st);
+  if (mode == MODE_FIXED && qreg) return run_stream(Q, nQ, nq, d, D, B, nd, nullptr, nullptr, 0, pad, dtype, out, st);
   // one pass for up to 32 blocks, from three queries on (one or two blocks a pass is the
   // stream kernel's; 50,000 x 180 tokens, three queries: two passes 707 us, one 430)
   if (mode == MODE_VARLEN && qreg && a.nbq <= 4 && (nQ * a.nbq >= 4 || nQ == 3))
-    return run_varlen_batched(Q, nQ, nq, d, D, total_tokens, offsets, 0, B, pad_len, dtype, out, st, false);
+    return run_varlen_batched(Q, nQ, nq, d, D, total_tokens, offsets, 0, B, pad, dtype, out, st, false);
   // variable-length documents against one or two query blocks per pass: the stream kernel,
   // whose walk reads each wave's document bounds from its lanes (no rows: the general kernel)
   if (mode == MODE_VARLEN && qreg && total_tokens > 0)
-    return run_stream(Q, nQ, nq, d, D, B, 0, offsets, nullptr, total_tokens, pad_len, dtype, out, st);
+    return run_stream(Q, nQ, nq, d, D, B, 0, offsets, nullptr, total_tokens, pad, dtype, out, st);
   // masked documents of up to 1,024 tokens (64 tiles, one lane each): the stream kernel walks
   // the tiles that hold a real token (2,000 x 180 tokens: 15 us against 22 for the general
   // kernel; 20,000: 93 against 183); longer ones: the general kernel
   if (mode == MODE_MASKED && qreg && nd > 0 && nd <= kMaskedStreamMaxTokens)
-    return run_stream(Q, nQ, nq, d, D, B, nd, nullptr, mask, 0, 0, dtype, out, st);
+    return run_stream(Q, nQ, nq, d, D, B, nd, nullptr, mask, 0, pad, dtype, out, st);
   if (dtype == TMS_DTYPE_F16) return run_dense<TMS_DTYPE_F16, TMS_DTYPE_F16>(a, nQ, mode, aligned, st);
   return run_dense<TMS_DTYPE_BF16, TMS_DTYPE_BF16>(a, nQ, mode, aligned, st);
 }
+
+int varlen_scores(const char* fn, const void* Qs, int64_t nQ, int64_t nq, int64_t d, const void* D_flat, int64_t T,
+                  const int64_t* offsets, int64_t B, PadLen pad, int dtype, float* out, void* stream) {
+  return dense_entry(fn, Qs, nQ, nq, d, D_flat, B, 0, T, offsets, nullptr, MODE_VARLEN, dtype, out, stream, pad);
+}
+
+void keep_error(char* to, int n) { snprintf(to, (size_t)n, "%s", g_err); }
 
 }  // namespace tms
 
@@ -199,14 +207,14 @@ int tms_maxsim_varlen(const void* Q, int64_t nq, int64_t d, const void* D_flat, 
 int tms_maxsim_varlen_padded(const void* Q, int64_t nq, int64_t d, const void* D_flat, int64_t total_tokens,
                              const int64_t* offsets, int64_t B, int64_t pad_len, int dtype, float* out, void* stream) {
   return tms::dense_entry("tms_maxsim_varlen_padded", Q, 1, nq, d, D_flat, B, 0, total_tokens, offsets, nullptr,
-                          tms::MODE_VARLEN, dtype, out, stream, pad_len);
+                          tms::MODE_VARLEN, dtype, out, stream, tms::PadLen{pad_len, nullptr, 0});
 }
 
 int tms_maxsim_varlen_batched(const void* Qs, int64_t nQ, int64_t nq, int64_t d, const void* D_flat,
                               int64_t total_tokens, const int64_t* offsets, int64_t B, int64_t pad_len, int dtype,
                               float* out, void* stream) {
   return tms::dense_entry("tms_maxsim_varlen_batched", Qs, nQ, nq, d, D_flat, B, 0, total_tokens, offsets, nullptr,
-                          tms::MODE_VARLEN, dtype, out, stream, pad_len);
+                          tms::MODE_VARLEN, dtype, out, stream, tms::PadLen{pad_len, nullptr, 0});
 }
 
 int tms_maxsim_dense_batched(const void* Qs, int64_t nQ, int64_t nq, int64_t d, const void* D, int64_t B, int64_t nd,

@@ -56,7 +56,7 @@ struct DenseArgs {
   int32_t nblk;            // blocks in this launch (<= NQB template)
   int32_t d, nchunk, nstep, nkg;
   int32_t docs_per_wave;
-  int64_t pad_len;         // varlen: score as if zero-padded to this many tokens (0 = off)
+  PadLen pad;              // varlen: score as if zero-padded to this many tokens (0 = off)
   int32_t mask4;           // masked: nd % 4 == 0 and a 4-byte aligned mask (word loads)
 };
 
@@ -157,6 +157,8 @@ __global__ void __launch_bounds__(NT, 1) dense_maxsim_kernel(DenseArgs a) {
     if constexpr (LINES32) return load_chunk_f32_lines(a.Q, row, S, gg, a.d);
     else return load_chunk<QDT, ALIGNED>(a.Q, row, 4 * S + gg, a.d, a.nchunk);
   };
+
+  const int64_t pad_len = MODE == MODE_VARLEN ? pad_length(a.pad, lane) : 0;
 
   // Query blocks of this launch: [my_blk0, my_blk0 + my_nblk).
   const int my_blk0 = a.blk0, my_nblk = a.nblk;
@@ -335,7 +337,7 @@ __global__ void __launch_bounds__(NT, 1) dense_maxsim_kernel(DenseArgs a) {
       }
       // an empty document zero-padded to pad_len > 0 tokens has every max equal to 0
       if (bad) write_bad(b);
-      else write_empty(b, a.pad_len > 0 ? 0.f : NEG_INF);
+      else write_empty(b, pad_len > 0 ? 0.f : NEG_INF);
     }
     c.b = b_end;
   };
@@ -467,7 +469,7 @@ __global__ void __launch_bounds__(NT, 1) dense_maxsim_kernel(DenseArgs a) {
 
   auto finish_doc = [&](int64_t b, int64_t len) {
     // zero padding up to pad_len adds dot products equal to 0 to a shorter document
-    const bool padded = (MODE == MODE_VARLEN) && len < a.pad_len;
+    const bool padded = (MODE == MODE_VARLEN) && len < pad_len;
     float blk[NQB];
 #pragma unroll
     for (int j = 0; j < NQB; j++) {

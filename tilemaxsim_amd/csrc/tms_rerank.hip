@@ -31,7 +31,8 @@ struct RerankArgs {
   const int64_t* offsets;  // varlen: (B + 1)
   const uint8_t* mask;     // masked: (B, nd), non-zero = real token
   float* out;              // (nQ, B)
-  int64_t B, nd, T, pad_len;
+  int64_t B, nd, T;
+  PadLen pad;
   int32_t nq, nbq;         // tokens per query, 32-token blocks per query
   int32_t blk0, nblk;      // query blocks [blk0, blk0 + nblk) of this launch, nblk <= NB
   int32_t d;               // 32 * KS
@@ -78,6 +79,7 @@ __device__ __forceinline__ void rerank_body(const RerankArgs& a) {
     qtmp[i] = v ? *(const u32x4*)(a.Q + (row * a.d + 8 * (4 * s + (fl >> 4))) * 2) : u32x4{0u, 0u, 0u, 0u};
   }
 
+  const int64_t pad_len = MODE == RR_VARLEN ? pad_length(a.pad, lane) : 0;
   // the document's rows [base, base + len); invalid offsets mark it bad
   int64_t base = 0, len = 0;
   bool bad = false;
@@ -219,7 +221,7 @@ __device__ __forceinline__ void rerank_body(const RerankArgs& a) {
     return;
   }
   // zero padding up to pad_len adds dot products equal to 0 to a shorter document
-  const bool padded_doc = MODE == RR_VARLEN && len < a.pad_len;
+  const bool padded_doc = MODE == RR_VARLEN && len < pad_len;
   float blk[NB];
 #pragma unroll
   for (int j = 0; j < NB; j++) {
@@ -360,9 +362,9 @@ bool rerank_fits(int64_t B, int64_t tokens_per_doc) {
 
 // Entry used by tms_dense.hip: nQ queries of nq tokens (at most 3 blocks in all, two per
 // launch), d in {32, 64, 96, 128}, 16-byte aligned Q and D, fp16 / bf16. mode: 0 fixed,
-// 1 variable-length (offsets, pad_len), 2 masked (mask). out is (nQ, B).
+// 1 variable-length (offsets, pad), 2 masked (mask). out is (nQ, B).
 int run_rerank(const void* Q, int64_t nQ, int64_t nq, int64_t d, const void* D, int64_t B, int64_t nd, int64_t T,
-               const int64_t* offsets, const uint8_t* mask, int64_t pad_len, int mode, int dtype, float* out,
+               const int64_t* offsets, const uint8_t* mask, PadLen pad, int mode, int dtype, float* out,
                hipStream_t st) {
   RerankArgs a;
   memset(&a, 0, sizeof(a));
@@ -374,7 +376,7 @@ int run_rerank(const void* Q, int64_t nQ, int64_t nq, int64_t d, const void* D, 
   a.B = B;
   a.nd = nd;
   a.T = T;
-  a.pad_len = pad_len;
+  a.pad = pad;
   a.nq = (int32_t)nq;
   a.nbq = (int32_t)((nq + 31) / 32);
   a.d = (int32_t)d;

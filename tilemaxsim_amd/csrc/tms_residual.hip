@@ -25,7 +25,7 @@
 // rounding x to fp16 first (differences ~1e-4 relative on unit-norm data).
 #include <string.h>
 
-#include "tms_common.h"
+#include "tms_check.h"
 
 namespace tms {
 
@@ -49,7 +49,8 @@ struct ResArgs {
   const int64_t* pids;       // (B) documents to score, or null for 0 .. B-1
   const uint16_t* weights;   // (2^nbits) fp16 bucket weights
   float* out;                // (B) scores, or (T, d) fp16 for the decompression kernel
-  int64_t B, ndocs, T, ncent, pad_len;
+  int64_t B, ndocs, T, ncent;
+  PadLen pad;
   int32_t nq, nbq, blk0, d, rb, docs_per_wave;
   int32_t nblk, blk_end;  // batched kernel: blocks per wave, one past the launch's last block
   int32_t wpd;            // fused kernel: waves per document (1: each wave walks whole documents)
@@ -270,6 +271,7 @@ __global__ void __launch_bounds__(256) residual_maxsim_kernel(ResArgs a) {
   // The wave's documents (at most 64) are read once, lane j holding document
   // b_begin + j: base row and length (-1 for an invalid pid or offsets). The walk
   // below takes them with readlane, so crossing a document never waits for memory.
+  const int64_t pad_len = pad_length(a.pad, lane);
   int64_t dbase = 0;
   int32_t dlen = -1;
   if (b_begin + lane < b_end) {
@@ -315,7 +317,7 @@ __global__ void __launch_bounds__(256) residual_maxsim_kernel(ResArgs a) {
       } else if (len < 0) {  // invalid pid or offsets: NaN, written as an integer by every launch
         if (lane == 0) store_nan_score(a.out + b);
       } else {
-        write(b, a.pad_len > 0 ? 0.f : NEG_INF);
+        write(b, pad_len > 0 ? 0.f : NEG_INF);
       }
     }
     c.b = b_end;
@@ -366,7 +368,7 @@ __global__ void __launch_bounds__(256) residual_maxsim_kernel(ResArgs a) {
       }
       return;
     }
-    const bool padded = len < a.pad_len;
+    const bool padded = len < pad_len;
     float s = 0.f;
 #pragma unroll
     for (int h = 0; h < 2; h++) {
@@ -470,7 +472,7 @@ __global__ void __launch_bounds__(256) residual_maxsim_kernel(ResArgs a) {
     __syncthreads();
     const int32_t len0 = __builtin_amdgcn_readlane(dlen, 0);  // lane 0 holds document b_begin
     if (part == 0 && b_begin < b_end && len0 > 0) {
-      const bool padded = len0 < a.pad_len;
+      const bool padded = len0 < pad_len;
       float s = 0.f;
 #pragma unroll
       for (int h = 0; h < 2; h++) {
@@ -545,6 +547,7 @@ __global__ void __launch_bounds__(64 * kResBatchedWaves, 1) residual_batched_ker
 
   // The workgroup's documents (at most 64): lane j holds document b_begin + j's first
   // index row and length (-1 for an invalid pid or offsets).
+  const int64_t pad_len = pad_length(a.pad, lane);
   int64_t dbase = 0;
   int32_t dlen = -1;
   if (lane < ndocs) {
@@ -588,7 +591,7 @@ __global__ void __launch_bounds__(64 * kResBatchedWaves, 1) residual_batched_ker
         return;
       }
       if (record) {  // invalid pid or offsets (len < 0): the final store writes NaN for the lane
-        const float v = a.pad_len > 0 ? 0.f : NEG_INF;
+        const float v = pad_len > 0 ? 0.f : NEG_INF;
 #pragma unroll
         for (int j = 0; j < NB; j++) pend[j] = lane == (int)(b - b_begin) ? v : pend[j];
       }
@@ -717,7 +720,7 @@ __global__ void __launch_bounds__(64 * kResBatchedWaves, 1) residual_batched_ker
       doc_end.init(qv, no_scale, lane);
     }
     auto finish = [&]() {  // the document of wc ends with this tile
-      doc_end.finish(rmax, wc.len < a.pad_len, lane, (int)(wc.b - b_begin), pend);
+      doc_end.finish(rmax, wc.len < pad_len, lane, (int)(wc.b - b_begin), pend);
     };
     auto step = [&](auto slot) -> bool {
       constexpr int i = decltype(slot)::value;  // step index mod 6
@@ -905,8 +908,8 @@ static int launch_batched_ks(const ResArgs& a, int nbits, int nb, int64_t grid, 
 static int prep_maxsim(const char* fn, const void* Q, int64_t nQ, int64_t nq, int64_t d, const void* centroids,
                        int64_t ncent, const void* bucket_weights, int nbits, const int32_t* codes,
                        const uint8_t* residuals, int64_t total_tokens, const int64_t* offsets, int64_t ndocs,
-                       const int64_t* pids, int64_t B, int64_t pad_len, float* out, hipStream_t st, ResArgs& a) {
-  if (nQ < 0 || nq < 0 || d < 0 || ncent < 0 || total_tokens < 0 || ndocs < 0 || B < 0 || pad_len < 0)
+                       const int64_t* pids, int64_t B, PadLen pad, float* out, hipStream_t st, ResArgs& a) {
+  if (nQ < 0 || nq < 0 || d < 0 || ncent < 0 || total_tokens < 0 || ndocs < 0 || B < 0 || pad.len < 0)
     return fail(TMS_ERR_INVALID, "%s: negative size", fn);
   int rc = check_format(fn, d, nbits, ncent, centroids, bucket_weights);
   if (rc) return rc;
@@ -940,12 +943,116 @@ static int prep_maxsim(const char* fn, const void* Q, int64_t nQ, int64_t nq, in
   a.ndocs = ndocs;
   a.T = total_tokens;
   a.ncent = ncent;
-  a.pad_len = pad_len;
+  a.pad = pad;
   a.nq = (int32_t)nq;
   a.nbq = (int32_t)((nq + 31) / 32);
   a.d = (int32_t)d;
   a.rb = (int32_t)(d * nbits / 8);
   return TMS_OK;
+}
+
+static int residual_one(const char* fn, const void* Q, int64_t nq, int64_t d, const void* centroids, int64_t ncent,
+                        const void* bucket_weights, int nbits, const int32_t* codes, const uint8_t* residuals,
+                        int64_t total_tokens, const int64_t* offsets, int64_t ndocs, const int64_t* pids, int64_t B,
+                        PadLen pad, float* out, void* stream) {
+  hipStream_t st = (hipStream_t)stream;
+  ResArgs a;
+  int rc = prep_maxsim(fn, Q, 1, nq, d, centroids, ncent, bucket_weights, nbits, codes, residuals,
+                       total_tokens, offsets, ndocs, pids, B, pad, out, st, a);
+  if (rc) return rc < 0 ? TMS_OK : rc;
+  // about TMS_RES_TOKENS_PER_WAVE tokens per wave (whole documents), at least two rounds
+  // of the chip's resident waves
+  const int64_t hint = ndocs > 0 ? total_tokens / ndocs : 1;
+  int64_t dpw = hint > 0 ? TMS_RES_TOKENS_PER_WAVE / hint : 1;
+  if (dpw > 1 && B / dpw < (int64_t)256 * 16 * 2) dpw = B / ((int64_t)256 * 16 * 2);
+  if (dpw < 1) dpw = 1;
+  if (dpw > 64) dpw = 64;  // one lane per document holds its bounds
+  a.docs_per_wave = (int32_t)dpw;
+  // Small calls (PLAID's final stage scores about 64 .. 1,024 candidates per query):
+  // documents split over up to four waves while the call still fits the waves the chip
+  // holds at once (three per SIMD at this kernel's registers), at most one wave per
+  // tile of an average document.
+  a.wpd = 1;
+  const int64_t tiles = (hint + 15) / 16;
+  if (rerank_fits(B, hint))  // the dense entry points' small-batch limit (tms_set_rerank_limit)
+    while (a.wpd < 4 && B * a.wpd * 2 <= TMS_RES_SPLIT_WAVES && 2 * a.wpd <= tiles) a.wpd *= 2;
+  if (a.wpd > 1) a.docs_per_wave = 1;
+  const int64_t grid = a.wpd > 1 ? (B * a.wpd + 3) / 4 : ((B + dpw - 1) / dpw + 3) / 4;
+  for (int blk = 0; blk < a.nbq; blk++) {
+    a.blk0 = blk;
+    switch (d / 32) {
+      case 1: rc = launch_fused_ks<1>(a, nbits, grid, st); break;
+      case 2: rc = launch_fused_ks<2>(a, nbits, grid, st); break;
+      case 3: rc = launch_fused_ks<3>(a, nbits, grid, st); break;
+      default: rc = launch_fused_ks<4>(a, nbits, grid, st); break;
+    }
+    if (rc) return rc;
+  }
+  return TMS_OK;
+}
+
+static int residual_many(const char* fn, const void* Qs, int64_t nQ, int64_t nq, int64_t d, const void* centroids,
+                         int64_t ncent, const void* bucket_weights, int nbits, const int32_t* codes,
+                         const uint8_t* residuals, int64_t total_tokens, const int64_t* offsets, int64_t ndocs,
+                         const int64_t* pids, int64_t B, PadLen pad, float* out, void* stream) {
+  hipStream_t st = (hipStream_t)stream;
+  ResArgs a;
+  int rc = prep_maxsim(fn, Qs, nQ, nq, d, centroids, ncent, bucket_weights, nbits, codes, residuals, total_tokens,
+                       offsets, ndocs, pids, B, pad, out, st, a);
+  if (rc) return rc < 0 ? TMS_OK : rc;
+  const int64_t nblocks = nQ * (int64_t)a.nbq;
+  if (a.nbq > kResMaxBlocksPerWave || nblocks < 2) {  // one query at a time
+    for (int64_t qi = 0; qi < nQ; qi++) {
+      rc = residual_one(fn, (const uint8_t*)Qs + qi * nq * d * 2, nq, d, centroids, ncent, bucket_weights, nbits,
+                               codes, residuals, total_tokens, offsets, ndocs, pids, B, pad, out + qi * B, stream);
+      if (rc) return rc;
+    }
+    return TMS_OK;
+  }
+  if (nblocks > ((int64_t)1 << 30)) return fail(TMS_ERR_UNSUPPORTED, "%s: too many queries", fn);
+  // Blocks per wave: the smallest of 1, 2, 4 whose launch covers every block in one pass
+  // (a wave computes all of its slots, used or not), else 4. A wave holds whole queries.
+  int nb = kResMaxBlocksPerWave;
+  for (int c = 1; c < kResMaxBlocksPerWave; c *= 2)
+    if (c >= a.nbq && nblocks <= (int64_t)kResBatchedWaves * ((c / a.nbq) * a.nbq)) {
+      nb = c;
+      break;
+    }
+  a.nblk = (nb / a.nbq) * a.nbq;
+  // about TMS_RES_BATCHED_TOKENS tokens per workgroup (whole documents, at most 64), at
+  // least four rounds of one workgroup per CU
+  const int64_t hint = ndocs > 0 ? total_tokens / ndocs : 1;
+  int64_t dpw = hint > 0 ? TMS_RES_BATCHED_TOKENS / hint : 1;
+  if (dpw > 1 && B / dpw < (int64_t)256 * 4) dpw = B / ((int64_t)256 * 4);
+  if (dpw < 1) dpw = 1;
+  if (dpw > 64) dpw = 64;
+  a.docs_per_wave = (int32_t)dpw;
+  const int64_t grid = (B + dpw - 1) / dpw;
+  if (grid > 0x7fffffff) return fail(TMS_ERR_UNSUPPORTED, "%s: too many documents", fn);
+  const int64_t per_launch = (int64_t)kResBatchedWaves * a.nblk;
+  for (int64_t b0 = 0; b0 < nblocks; b0 += per_launch) {
+    a.blk0 = (int32_t)b0;
+    a.blk_end = (int32_t)(nblocks - b0 < per_launch ? nblocks : b0 + per_launch);
+    switch (d / 32) {
+      case 1: rc = launch_batched_ks<1>(a, nbits, nb, grid, st); break;
+      case 2: rc = launch_batched_ks<2>(a, nbits, nb, grid, st); break;
+      case 3: rc = launch_batched_ks<3>(a, nbits, nb, grid, st); break;
+      default: rc = launch_batched_ks<4>(a, nbits, nb, grid, st); break;
+    }
+    if (rc) return rc;
+  }
+  return TMS_OK;
+}
+
+int residual_scores(const char* fn, const void* Qs, int64_t nQ, int64_t nq, int64_t d, const void* centroids,
+                    int64_t ncent, const void* bucket_weights, int nbits, const int32_t* codes,
+                    const uint8_t* residuals, int64_t total_tokens, const int64_t* offsets, int64_t ndocs,
+                    const int64_t* pids, int64_t B, PadLen pad, bool batched, float* out, void* stream) {
+  if (batched)
+    return residual_many(fn, Qs, nQ, nq, d, centroids, ncent, bucket_weights, nbits, codes, residuals, total_tokens,
+                         offsets, ndocs, pids, B, pad, out, stream);
+  return residual_one(fn, Qs, nq, d, centroids, ncent, bucket_weights, nbits, codes, residuals, total_tokens, offsets,
+                      ndocs, pids, B, pad, out, stream);
 }
 
 }  // namespace tms
@@ -987,96 +1094,18 @@ int tms_maxsim_residual(const void* Q, int64_t nq, int64_t d, const void* centro
                         const void* bucket_weights, int nbits, const int32_t* codes, const uint8_t* residuals,
                         int64_t total_tokens, const int64_t* offsets, int64_t ndocs, const int64_t* pids, int64_t B,
                         int64_t pad_len, float* out, void* stream) {
-  using namespace tms;
-  hipStream_t st = (hipStream_t)stream;
-  ResArgs a;
-  int rc = prep_maxsim("tms_maxsim_residual", Q, 1, nq, d, centroids, ncent, bucket_weights, nbits, codes, residuals,
-                       total_tokens, offsets, ndocs, pids, B, pad_len, out, st, a);
-  if (rc) return rc < 0 ? TMS_OK : rc;
-  // about TMS_RES_TOKENS_PER_WAVE tokens per wave (whole documents), at least two rounds
-  // of the chip's resident waves
-  const int64_t hint = ndocs > 0 ? total_tokens / ndocs : 1;
-  int64_t dpw = hint > 0 ? TMS_RES_TOKENS_PER_WAVE / hint : 1;
-  if (dpw > 1 && B / dpw < (int64_t)256 * 16 * 2) dpw = B / ((int64_t)256 * 16 * 2);
-  if (dpw < 1) dpw = 1;
-  if (dpw > 64) dpw = 64;  // one lane per document holds its bounds
-  a.docs_per_wave = (int32_t)dpw;
-  // Small calls (PLAID's final stage scores about 64 .. 1,024 candidates per query):
-  // documents split over up to four waves while the call still fits the waves the chip
-  // holds at once (three per SIMD at this kernel's registers), at most one wave per
-  // tile of an average document.
-  a.wpd = 1;
-  const int64_t tiles = (hint + 15) / 16;
-  if (rerank_fits(B, hint))  // the dense entry points' small-batch limit (tms_set_rerank_limit)
-    while (a.wpd < 4 && B * a.wpd * 2 <= TMS_RES_SPLIT_WAVES && 2 * a.wpd <= tiles) a.wpd *= 2;
-  if (a.wpd > 1) a.docs_per_wave = 1;
-  const int64_t grid = a.wpd > 1 ? (B * a.wpd + 3) / 4 : ((B + dpw - 1) / dpw + 3) / 4;
-  for (int blk = 0; blk < a.nbq; blk++) {
-    a.blk0 = blk;
-    switch (d / 32) {
-      case 1: rc = launch_fused_ks<1>(a, nbits, grid, st); break;
-      case 2: rc = launch_fused_ks<2>(a, nbits, grid, st); break;
-      case 3: rc = launch_fused_ks<3>(a, nbits, grid, st); break;
-      default: rc = launch_fused_ks<4>(a, nbits, grid, st); break;
-    }
-    if (rc) return rc;
-  }
-  return TMS_OK;
+  return tms::residual_scores("tms_maxsim_residual", Q, 1, nq, d, centroids, ncent, bucket_weights, nbits, codes,
+                              residuals, total_tokens, offsets, ndocs, pids, B, tms::PadLen{pad_len, nullptr, 0}, false,
+                              out, stream);
 }
 
 int tms_maxsim_residual_batched(const void* Qs, int64_t nQ, int64_t nq, int64_t d, const void* centroids,
                                 int64_t ncent, const void* bucket_weights, int nbits, const int32_t* codes,
                                 const uint8_t* residuals, int64_t total_tokens, const int64_t* offsets, int64_t ndocs,
                                 const int64_t* pids, int64_t B, int64_t pad_len, float* out, void* stream) {
-  using namespace tms;
-  const char* fn = "tms_maxsim_residual_batched";
-  hipStream_t st = (hipStream_t)stream;
-  ResArgs a;
-  int rc = prep_maxsim(fn, Qs, nQ, nq, d, centroids, ncent, bucket_weights, nbits, codes, residuals, total_tokens,
-                       offsets, ndocs, pids, B, pad_len, out, st, a);
-  if (rc) return rc < 0 ? TMS_OK : rc;
-  const int64_t nblocks = nQ * (int64_t)a.nbq;
-  if (a.nbq > kResMaxBlocksPerWave || nblocks < 2) {  // one query at a time
-    for (int64_t qi = 0; qi < nQ; qi++) {
-      rc = tms_maxsim_residual((const uint8_t*)Qs + qi * nq * d * 2, nq, d, centroids, ncent, bucket_weights, nbits,
-                               codes, residuals, total_tokens, offsets, ndocs, pids, B, pad_len, out + qi * B, stream);
-      if (rc) return rc;
-    }
-    return TMS_OK;
-  }
-  if (nblocks > ((int64_t)1 << 30)) return fail(TMS_ERR_UNSUPPORTED, "%s: too many queries", fn);
-  // Blocks per wave: the smallest of 1, 2, 4 whose launch covers every block in one pass
-  // (a wave computes all of its slots, used or not), else 4. A wave holds whole queries.
-  int nb = kResMaxBlocksPerWave;
-  for (int c = 1; c < kResMaxBlocksPerWave; c *= 2)
-    if (c >= a.nbq && nblocks <= (int64_t)kResBatchedWaves * ((c / a.nbq) * a.nbq)) {
-      nb = c;
-      break;
-    }
-  a.nblk = (nb / a.nbq) * a.nbq;
-  // about TMS_RES_BATCHED_TOKENS tokens per workgroup (whole documents, at most 64), at
-  // least four rounds of one workgroup per CU
-  const int64_t hint = ndocs > 0 ? total_tokens / ndocs : 1;
-  int64_t dpw = hint > 0 ? TMS_RES_BATCHED_TOKENS / hint : 1;
-  if (dpw > 1 && B / dpw < (int64_t)256 * 4) dpw = B / ((int64_t)256 * 4);
-  if (dpw < 1) dpw = 1;
-  if (dpw > 64) dpw = 64;
-  a.docs_per_wave = (int32_t)dpw;
-  const int64_t grid = (B + dpw - 1) / dpw;
-  if (grid > 0x7fffffff) return fail(TMS_ERR_UNSUPPORTED, "%s: too many documents", fn);
-  const int64_t per_launch = (int64_t)kResBatchedWaves * a.nblk;
-  for (int64_t b0 = 0; b0 < nblocks; b0 += per_launch) {
-    a.blk0 = (int32_t)b0;
-    a.blk_end = (int32_t)(nblocks - b0 < per_launch ? nblocks : b0 + per_launch);
-    switch (d / 32) {
-      case 1: rc = launch_batched_ks<1>(a, nbits, nb, grid, st); break;
-      case 2: rc = launch_batched_ks<2>(a, nbits, nb, grid, st); break;
-      case 3: rc = launch_batched_ks<3>(a, nbits, nb, grid, st); break;
-      default: rc = launch_batched_ks<4>(a, nbits, nb, grid, st); break;
-    }
-    if (rc) return rc;
-  }
-  return TMS_OK;
+  return tms::residual_scores("tms_maxsim_residual_batched", Qs, nQ, nq, d, centroids, ncent, bucket_weights, nbits,
+                              codes, residuals, total_tokens, offsets, ndocs, pids, B,
+                              tms::PadLen{pad_len, nullptr, 0}, true, out, stream);
 }
 
 }  // extern "C"

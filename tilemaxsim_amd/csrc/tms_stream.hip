@@ -31,7 +31,8 @@ struct StreamArgs {
   const int64_t* offsets;    // variable length: (B + 1)
   const uint8_t* mask;       // masked: (B, nd), non-zero = real token
   float* out;                // (nQ, B)
-  int64_t B, nd, T, pad_len;  // pad_len > 0 (variable length): score as if zero-padded to it
+  int64_t B, nd, T;
+  PadLen pad;                // > 0 (variable length): score as if zero-padded to it
   int32_t nq, nbq;           // tokens per query, 32-token blocks per query
   int32_t blk0;              // first global query block of this launch
   int32_t blk_end;           // one past the last block of this launch
@@ -150,6 +151,7 @@ __global__ void __launch_bounds__(256, 1) stream_maxsim_kernel(StreamArgs a) {
   auto doc_live = [&](int64_t dd) -> uint64_t {  // MASKED: bit t: tile t holds a real token
     return (mlive >> (dd * mtiles)) & (~0ull >> (64 - mtiles));
   };
+  const int64_t pad_len = VARLEN ? pad_length(a.pad, lane) : 0;
   auto doc_len = [&](int64_t dd) -> int64_t {
     if constexpr (VARLEN) return (int32_t)__builtin_amdgcn_readlane((uint32_t)dlen, (int)dd);
     else return a.nd;
@@ -323,7 +325,7 @@ __global__ void __launch_bounds__(256, 1) stream_maxsim_kernel(StreamArgs a) {
         }
       }
       // document done: max over the 64 rows of each column, sum over query tokens
-      const bool padded = VARLEN && len < a.pad_len;  // zero padding adds dot products of 0
+      const bool padded = VARLEN && len < pad_len;  // zero padding adds dot products of 0
       float blk[NB];
 #pragma unroll
       for (int j = 0; j < NB; j++) {
@@ -342,7 +344,7 @@ __global__ void __launch_bounds__(256, 1) stream_maxsim_kernel(StreamArgs a) {
         s += __shfl_xor(s, 2);
         s += __shfl_xor(s, 1);
         if (MASKED && doc_live(dd) == 0) s = NEG_INF;  // no real token (the tiles read row 0)
-        if (VARLEN && len <= 0) s = a.pad_len > 0 ? 0.f : NEG_INF;  // no rows (the tiles read row 0)
+        if (VARLEN && len <= 0) s = pad_len > 0 ? 0.f : NEG_INF;  // no rows (the tiles read row 0)
         blk[j] = s;
       }
       const bool mine = lane == (int)dd;
@@ -408,16 +410,16 @@ static int stream_ks(const StreamArgs& a, int64_t grid, hipStream_t st) {
 
 // Batched queries (tms_batched.hip).
 int run_varlen_batched(const void* Q, int64_t nQ, int64_t nq, int64_t d, const void* D, int64_t T,
-                       const int64_t* offsets, int64_t nd, int64_t B, int64_t pad_len, int dtype, float* out,
+                       const int64_t* offsets, int64_t nd, int64_t B, PadLen pad, int dtype, float* out,
                        hipStream_t st, bool q32);
 
 // Entry used by tms_dense.hip for d in {32, 64, 96, 128}, 16-byte aligned Q and D:
 // fixed-length documents (offsets and mask null), padded ones with a (B, nd) token mask
 // (1 <= nd <= kMaskedStreamMaxTokens), or documents at offsets into T >= 1 rows
-// (pad_len > 0: scored as if zero-padded to pad_len tokens). nQ queries of nq tokens;
+// (pad > 0: scored as if zero-padded to that many tokens). nQ queries of nq tokens;
 // out is (nQ, B).
 int run_stream(const void* Q, int64_t nQ, int64_t nq, int64_t d, const void* D, int64_t B, int64_t nd,
-               const int64_t* offsets, const uint8_t* mask, int64_t T, int64_t pad_len, int dtype, float* out,
+               const int64_t* offsets, const uint8_t* mask, int64_t T, PadLen pad, int dtype, float* out,
                hipStream_t st) {
   StreamArgs a;
   memset(&a, 0, sizeof(a));
@@ -430,13 +432,13 @@ int run_stream(const void* Q, int64_t nQ, int64_t nq, int64_t d, const void* D, 
   a.B = B;
   a.nd = offsets ? 0 : nd;
   a.T = T;
-  a.pad_len = pad_len;
+  a.pad = pad;
   a.nq = (int32_t)nq;
   a.nbq = (int32_t)((nq + 31) / 32);
   a.d = (int32_t)d;
   const int64_t nblocks = nQ * (int64_t)a.nbq;
   if (!offsets && !mask && a.nbq <= 4 && (nblocks >= 4 || nQ == 3))  // batched: documents at implicit offsets b * nd
-    return run_varlen_batched(Q, nQ, nq, d, D, B * nd, nullptr, nd, B, 0, dtype, out, st, false);
+    return run_varlen_batched(Q, nQ, nq, d, D, B * nd, nullptr, nd, B, PadLen{0, nullptr, 0}, dtype, out, st, false);
   const int64_t hint = offsets ? (B > 0 ? T / B : 1) : nd;  // tokens per document
   int64_t dpw = hint > 0 ? TMS_STREAM_TOKENS_PER_WAVE / hint : 1;
   const int64_t min_waves = TMS_STREAM_MIN_WAVES;

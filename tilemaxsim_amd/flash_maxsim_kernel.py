@@ -61,9 +61,9 @@ def flash_maxsim_multi_doc(Q: torch.Tensor, D_flat: torch.Tensor, doc_offsets: t
         D_flat: (total_tokens, d) all document tokens, float16, bfloat16 or float32, contiguous.
         doc_offsets: (num_docs + 1,) integer start offsets (any device; moved to Q's
             device as int64).
-        validate: check on the host that offsets are non-decreasing within
-            [0, total_tokens] (one device-to-host copy); with ``validate=False`` a
-            document with invalid offsets scores NaN instead of raising.
+        validate: check that offsets are non-decreasing within
+            [0, total_tokens] (a check on the device whose verdict the host waits for); with
+            ``validate=False`` a document with invalid offsets scores NaN instead of raising.
 
     Returns:
         (num_docs,) float32 scores; an empty document scores -inf.
@@ -88,15 +88,17 @@ def flash_maxsim_multi_doc(Q: torch.Tensor, D_flat: torch.Tensor, doc_offsets: t
     Q, code = _check.query_for(Q, D_flat.dtype)
     offsets = doc_offsets.to(device=Q.device, dtype=torch.int64).contiguous()
     num_docs = offsets.shape[0] - 1
-    if validate and num_docs > 0:
-        bad = (offsets[0] < 0) | (offsets[-1] > T) | (offsets[1:] < offsets[:-1]).any()
-        if bool(bad):
-            raise ValueError("flash_maxsim_multi_doc: doc_offsets must be non-decreasing within [0, total_tokens]")
     scores = torch.empty(num_docs, dtype=torch.float32, device=Q.device)
     if num_docs == 0:
         return scores
     lib = _lib.load()
     with _lib.on_device(Q.device):
+        if validate:  # the check runs on the device before the scoring kernel; its verdict is waited for
+            _lib.check_bounds(
+                lib.tms_maxsim_varlen_checked(Q.data_ptr(), 1, Nq, d, D_flat.data_ptr(), T, offsets.data_ptr(), num_docs, 0,
+                                              code, scores.data_ptr(), None, _lib.verdict_ptr(), _lib.stream_of(Q)),
+                "flash_maxsim_multi_doc: doc_offsets must be non-decreasing within [0, total_tokens]")
+            return scores
         _lib.check(lib.tms_maxsim_varlen(Q.data_ptr(), Nq, d, D_flat.data_ptr(), T, offsets.data_ptr(), num_docs,
                                          code, scores.data_ptr(), _lib.stream_of(Q)))
     return scores
@@ -124,19 +126,21 @@ def _varlen_batched(fn: str, Qs: torch.Tensor, D_flat: torch.Tensor, doc_offsets
     Qs, code = _check.query_for(Qs, D_flat.dtype)
     offsets = doc_offsets.to(device=Qs.device, dtype=torch.int64).contiguous()
     B = offsets.shape[0] - 1
-    if (validate or zero_pad) and B > 0:
-        bad = (offsets[0] < 0) | (offsets[-1] > T) | (offsets[1:] < offsets[:-1]).any()
-        if bool(bad):
-            raise ValueError(f"{fn}: doc_offsets must be non-decreasing within [0, total_tokens]")
-    pad_len = int((offsets[1:] - offsets[:-1]).max()) if zero_pad and B > 0 else 0
     out = torch.empty(nQ, B, dtype=torch.float32, device=Qs.device)
-    if B == 0 or nQ == 0:
+    if B == 0 or (nQ == 0 and not (validate or zero_pad)):
         return out
     lib = _lib.load()
     with _lib.on_device(Qs.device):
+        if validate or zero_pad:
+            parts = torch.empty(_lib.TMS_CHECK_PARTS, dtype=torch.int64, device=Qs.device) if zero_pad else None
+            _lib.check_bounds(
+                lib.tms_maxsim_varlen_checked(Qs.data_ptr(), nQ, Nq, d, D_flat.data_ptr(), T, offsets.data_ptr(), B,
+                                              int(zero_pad), code, out.data_ptr(), _lib.ptr(parts), _lib.verdict_ptr(),
+                                              _lib.stream_of(Qs)),
+                f"{fn}: doc_offsets must be non-decreasing within [0, total_tokens]")
+            return out
         _lib.check(lib.tms_maxsim_varlen_batched(Qs.data_ptr(), nQ, Nq, d, D_flat.data_ptr(), T, offsets.data_ptr(), B,
-                                                 pad_len, code, out.data_ptr(),
-                                                 _lib.stream_of(Qs)))
+                                                 0, code, out.data_ptr(), _lib.stream_of(Qs)))
     return out
 
 

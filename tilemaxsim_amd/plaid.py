@@ -71,23 +71,33 @@ def flashmaxsim_score_packed(Q: torch.Tensor, D_packed: torch.Tensor, D_lengths:
     _check.on_gpu("D_packed", D_packed)
     dev = D_packed.device
     Q2 = Q2.to(dev).half().contiguous()
-    offsets = lengths_to_offsets(D_lengths, dev)
     if padding == "mask":
-        return flash_maxsim_multi_doc(Q2, D_packed, offsets)
-    B = offsets.numel() - 1
+        return flash_maxsim_multi_doc(Q2, D_packed, lengths_to_offsets(D_lengths, dev))
+    B = D_lengths.numel()
     T, d = D_packed.shape
     assert Q2.shape[1] == d, f"flashmaxsim_score_packed: Q width {Q2.shape[1]} != D width {d}"
-    if B > 0 and (bool((offsets[1:] < offsets[:-1]).any()) or int(offsets[-1]) > T):
-        raise ValueError("flashmaxsim_score_packed: D_lengths must be >= 0 and sum to at most D_packed.shape[0]")
-    pad_len = int(D_lengths.max()) if B > 0 else 0
     scores = torch.empty(B, dtype=torch.float32, device=dev)
     if B == 0:
         return scores
+    # the lengths' sums, their checks and the longest one (the zero padding's length) are
+    # taken on the device, before the scoring kernel that uses them
+    parts = torch.empty(_lib.TMS_CHECK_PARTS, dtype=torch.int64, device=dev)
+    scan = B <= _lib.TMS_PACKED_SCAN_MAX  # longer lists: torch's prefix sum
+    lengths = D_lengths.to(device=dev, dtype=torch.int64).contiguous()
+    offsets = torch.empty(B + 1, dtype=torch.int64, device=dev) if scan else lengths_to_offsets(lengths, dev)
     lib = _lib.load()
     with _lib.on_device(dev):
-        _lib.check(lib.tms_maxsim_varlen_padded(Q2.data_ptr(), Q2.shape[0], d, D_packed.data_ptr(), T,
-                                                offsets.data_ptr(), B, pad_len, _lib.TMS_DTYPE_F16,
-                                                scores.data_ptr(), _lib.stream_of(Q2)))
+        if scan:
+            status = lib.tms_maxsim_packed_checked(Q2.data_ptr(), Q2.shape[0], d, D_packed.data_ptr(), T,
+                                                   lengths.data_ptr(), B, 1, _lib.TMS_DTYPE_F16, scores.data_ptr(),
+                                                   offsets.data_ptr(), parts.data_ptr(), _lib.verdict_ptr(),
+                                                   _lib.stream_of(Q2))
+        else:
+            status = lib.tms_maxsim_varlen_checked(Q2.data_ptr(), 1, Q2.shape[0], d, D_packed.data_ptr(), T,
+                                                   offsets.data_ptr(), B, 1, _lib.TMS_DTYPE_F16, scores.data_ptr(),
+                                                   parts.data_ptr(), _lib.verdict_ptr(), _lib.stream_of(Q2))
+        _lib.check_bounds(status,
+                          "flashmaxsim_score_packed: D_lengths must be >= 0 and sum to at most D_packed.shape[0]")
     return scores
 
 

@@ -76,8 +76,8 @@ def decompress_residual(codes: torch.Tensor, residuals: torch.Tensor, centroids:
     return out
 
 
-def _prep_docs(fn: str, doc_offsets, pids, dev, T: int, padding: str, validate: bool):
-    """Offsets, pids, B and pad_len for the MaxSim entry points (shared checks)."""
+def _prep_docs(doc_offsets, pids, dev, padding: str):
+    """Offsets, pids, ndocs and B for the MaxSim entry points (shared checks)."""
     if padding not in ("zeros", "mask"):
         raise ValueError(f"padding must be 'zeros' or 'mask', got {padding!r}")
     _check.tensor("doc_offsets", doc_offsets)
@@ -95,21 +95,32 @@ def _prep_docs(fn: str, doc_offsets, pids, dev, T: int, padding: str, validate: 
         B = pids.numel()
     else:
         B = ndocs
-    if B == 0:
-        return offsets, pids, ndocs, B, 0
-    if validate:
-        bad = bool((offsets[1:] < offsets[:-1]).any()) or int(offsets[0]) < 0 or int(offsets[-1]) > T
-        if pids is not None:
-            bad = bad or bool(((pids < 0) | (pids >= ndocs)).any())
-        if bad:
-            raise ValueError(f"{fn}: doc_offsets must be non-decreasing within [0, T] and pids within [0, ndocs)")
-    pad_len = 0
-    if padding == "zeros" and ndocs > 0:  # the longest scored document (one host sync)
-        lengths = offsets[1:] - offsets[:-1]
-        if pids is not None:
-            lengths = lengths[pids.clamp(0, ndocs - 1)]
-        pad_len = max(int(lengths.max()), 0)
-    return offsets, pids, ndocs, B, pad_len
+    return offsets, pids, ndocs, B
+
+
+def _score(fn: str, Qs, nQ: int, Nq: int, d: int, batched: bool, index, offsets, pids, ndocs: int, B: int, padding: str,
+           validate: bool, out: torch.Tensor) -> torch.Tensor:
+    """One scoring call into ``out``; the bounds and the longest scored document are found
+    on the device before the scoring kernel, and with ``validate`` the bounds' verdict is
+    waited for."""
+    codes, residuals, centroids, bucket_weights, nbits = index
+    zeros = padding == "zeros"
+    parts = torch.empty(_lib.TMS_CHECK_PARTS, dtype=torch.int64, device=out.device) if zeros else None
+    lib = _lib.load()
+    with _lib.on_device(out.device):
+        args = (Nq, d, centroids.data_ptr(), centroids.shape[0], bucket_weights.data_ptr(), nbits, codes.data_ptr(),
+                residuals.data_ptr(), codes.shape[0], offsets.data_ptr(), ndocs, _lib.ptr(pids), B)
+        stream = _lib.stream_of(out)
+        if validate or zeros:
+            _lib.check_bounds(
+                lib.tms_maxsim_residual_checked(Qs.data_ptr(), nQ, *args, int(zeros), int(batched), out.data_ptr(),
+                                                _lib.ptr(parts), _lib.verdict_ptr() if validate else None, stream),
+                f"{fn}: doc_offsets must be non-decreasing within [0, T] and pids within [0, ndocs)")
+        elif batched:
+            _lib.check(lib.tms_maxsim_residual_batched(Qs.data_ptr(), nQ, *args, 0, out.data_ptr(), stream))
+        else:
+            _lib.check(lib.tms_maxsim_residual(Qs.data_ptr(), *args, 0, out.data_ptr(), stream))
+    return out
 
 
 def flashmaxsim_score_residual(Q: torch.Tensor, codes: torch.Tensor, residuals: torch.Tensor,
@@ -127,8 +138,8 @@ def flashmaxsim_score_residual(Q: torch.Tensor, codes: torch.Tensor, residuals: 
             zero-padded to the longest scored one, so a shorter document's per-token max
             is at least 0 (``src/plaid_integration_benchmark.py:167-171``); "mask" --
             plain MaxSim, padding never wins (an empty document scores -inf).
-        validate: check pids and offsets on the device first (one host sync); without
-            it an invalid document scores NaN.
+        validate: check pids and offsets on the device before scoring, and wait for the
+            verdict; without it an invalid document scores NaN.
 
     Returns:
         (B,) float32 scores, equal to MaxSim over :func:`decompress_residual`'s output up
@@ -143,21 +154,13 @@ def flashmaxsim_score_residual(Q: torch.Tensor, codes: torch.Tensor, residuals: 
     if Q2.dim() != 2:
         raise ValueError(f"Q must be (1, Nq, d) or (Nq, d), got {tuple(Q.shape)}")
     assert Q2.shape[1] == d, f"flashmaxsim_score_residual: Q width {Q2.shape[1]} != centroid width {d}"
-    T = codes.shape[0]
-    offsets, pids, ndocs, B, pad_len = _prep_docs("flashmaxsim_score_residual", doc_offsets, pids, dev, T, padding,
-                                                  validate)
+    offsets, pids, ndocs, B = _prep_docs(doc_offsets, pids, dev, padding)
     Q2 = _check.query_like(Q2.to(dev), torch.float16)
     scores = torch.empty(B, dtype=torch.float32, device=dev)
     if B == 0:
         return scores
-    lib = _lib.load()
-    with _lib.on_device(dev):
-        _lib.check(lib.tms_maxsim_residual(Q2.data_ptr(), Q2.shape[0], d, centroids.data_ptr(), centroids.shape[0],
-                                           bucket_weights.data_ptr(), nbits, codes.data_ptr(), residuals.data_ptr(),
-                                           T, offsets.data_ptr(), ndocs,
-                                           pids.data_ptr() if pids is not None else None, B, pad_len,
-                                           scores.data_ptr(), _lib.stream_of(Q2)))
-    return scores
+    return _score("flashmaxsim_score_residual", Q2, 1, Q2.shape[0], d, False,
+                  (codes, residuals, centroids, bucket_weights, nbits), offsets, pids, ndocs, B, padding, validate, scores)
 
 
 def flashmaxsim_score_residual_batched(Qs: torch.Tensor, codes: torch.Tensor, residuals: torch.Tensor,
@@ -182,19 +185,11 @@ def flashmaxsim_score_residual_batched(Qs: torch.Tensor, codes: torch.Tensor, re
     if Qs.dim() != 3:
         raise ValueError(f"Qs must be (nQ, Nq, d), got {tuple(Qs.shape)}")
     assert Qs.shape[2] == d, f"flashmaxsim_score_residual_batched: Q width {Qs.shape[2]} != centroid width {d}"
-    T = codes.shape[0]
-    offsets, pids, ndocs, B, pad_len = _prep_docs("flashmaxsim_score_residual_batched", doc_offsets, pids, dev, T,
-                                                  padding, validate)
+    offsets, pids, ndocs, B = _prep_docs(doc_offsets, pids, dev, padding)
     Qs = _check.query_like(Qs.to(dev), torch.float16)
     nQ, Nq = Qs.shape[0], Qs.shape[1]
     scores = torch.empty(nQ, B, dtype=torch.float32, device=dev)
-    if B == 0 or nQ == 0:
+    if B == 0 or (nQ == 0 and not validate):
         return scores
-    lib = _lib.load()
-    with _lib.on_device(dev):
-        _lib.check(lib.tms_maxsim_residual_batched(Qs.data_ptr(), nQ, Nq, d, centroids.data_ptr(), centroids.shape[0],
-                                                   bucket_weights.data_ptr(), nbits, codes.data_ptr(),
-                                                   residuals.data_ptr(), T, offsets.data_ptr(), ndocs,
-                                                   pids.data_ptr() if pids is not None else None, B, pad_len,
-                                                   scores.data_ptr(), _lib.stream_of(Qs)))
-    return scores
+    return _score("flashmaxsim_score_residual_batched", Qs, nQ, Nq, d, True,
+                  (codes, residuals, centroids, bucket_weights, nbits), offsets, pids, ndocs, B, padding, validate, scores)
