@@ -70,9 +70,69 @@ int topk_checks(const char* fn, const float* scores, int64_t nrows, int64_t n, i
   return TMS_OK;
 }
 
+// Group maxima (tms_topk_kernel.h): the groups' size for k, or 0 where the tournament takes
+// the row. k groups of a span's or of g scores have to fit the selection's keys (4,096 up to
+// k = 128, 16,384 up to 512), the spans its first stage, and the maxima the workspace the
+// tournament would use (which leaves it k < 8 and a few k above a power of two). Rows of few
+// groups for their k stay too: their maxima bound little (5,000 scores, k = 200: 17 us, by
+// groups 51).
+constexpr int64_t kGroupMaxSpans = 16384;
+static int group_lanes_log2(int64_t nrows, int64_t n, int k) {
+  const int64_t keys = k <= kFilterMaxK ? 4096 : 16384;
+  if (n <= kChunk || k > keys / 32 || (k > kFilterMaxK && n < (int64_t)64 * k)) return 0;
+  int lg = 3;
+  // the largest group of which k fit, with twice k groups in the row
+  while (lg < 6 && ((int64_t)8 << lg) * k <= keys && n >= 2 * ((int64_t)8 << lg) * k) lg++;
+  const int64_t spans = ceil_div(n, kSpan), per = kSpan >> (lg + 2);
+  const bool direct = spans * per <= keys;
+  if (!direct && (spans > kGroupMaxSpans || per * k > keys || spans < k)) return 0;
+  const int64_t need = nrows * spans * (per + (direct ? 0 : 1)) * (int64_t)sizeof(uint32_t);
+  return need <= topk_workspace_bytes(nrows, n, k) ? lg : 0;
+}
+
+template <int CH1, int CHS>
+static void group_last(int64_t nrows, hipStream_t st, const float* scores, int64_t n, int64_t spans, int lg,
+                       const uint32_t* groups, const uint32_t* spans_in, float* out_values, int64_t* out_indices, int k) {
+  hipLaunchKernelGGL((topk_group_last_kernel<CH1, CHS>), dim3((unsigned)nrows), dim3(kLastThreads), 0, st, scores, n,
+                     spans, lg, groups, spans_in, out_values, out_indices, k);
+}
+
+static int group_run(const float* scores, int64_t nrows, int64_t n, int k, int lg, uint32_t* ws, float* out_values,
+                     int64_t* out_indices, hipStream_t st) {
+  const int64_t keys = k <= kFilterMaxK ? 4096 : 16384;
+  const int64_t spans = ceil_div(n, kSpan), per = kSpan >> (lg + 2), total = nrows * spans;
+  uint32_t* groups = ws;
+  uint32_t* spans_out = spans * per <= keys ? nullptr : ws + total * per;
+  // one span a wave while that leaves the chip room (2,048 workgroups), else up to four
+  int64_t per_row = ceil_div(spans, kGroupWaves);
+  if (per_row * nrows > 2048) per_row = ceil_div(spans, kGroupWaves * (per_row * nrows > 8192 ? 4 : 2));
+  const dim3 grid((unsigned)per_row, (unsigned)nrows);
+  switch (lg) {
+    case 3: hipLaunchKernelGGL(topk_group_max_kernel<3>, grid, dim3(64 * kGroupWaves), 0, st, scores, n, spans, groups, spans_out); break;
+    case 4: hipLaunchKernelGGL(topk_group_max_kernel<4>, grid, dim3(64 * kGroupWaves), 0, st, scores, n, spans, groups, spans_out); break;
+    case 5: hipLaunchKernelGGL(topk_group_max_kernel<5>, grid, dim3(64 * kGroupWaves), 0, st, scores, n, spans, groups, spans_out); break;
+    default: hipLaunchKernelGGL(topk_group_max_kernel<6>, grid, dim3(64 * kGroupWaves), 0, st, scores, n, spans, groups, spans_out); break;
+  }
+  int rc = check_launch("topk_group_max_kernel");
+  if (rc) return rc;
+  const bool big = spans_out && spans > 4096, mid = spans_out && spans > 1024;
+  if (keys == 4096) {
+    if (big) group_last<16384, 4096>(nrows, st, scores, n, spans, lg, groups, spans_out, out_values, out_indices, k);
+    else if (mid) group_last<4096, 4096>(nrows, st, scores, n, spans, lg, groups, spans_out, out_values, out_indices, k);
+    else group_last<1024, 4096>(nrows, st, scores, n, spans, lg, groups, spans_out, out_values, out_indices, k);
+  } else {
+    if (big) group_last<16384, 16384>(nrows, st, scores, n, spans, lg, groups, spans_out, out_values, out_indices, k);
+    else if (mid) group_last<4096, 16384>(nrows, st, scores, n, spans, lg, groups, spans_out, out_values, out_indices, k);
+    else group_last<1024, 16384>(nrows, st, scores, n, spans, lg, groups, spans_out, out_values, out_indices, k);
+  }
+  return check_launch("topk_group_last_kernel");
+}
+
 // The levels of one call; `workspace` holds topk_workspace_bytes(nrows, n, k) bytes.
 int topk_run(const float* scores, int64_t nrows, int64_t n, int64_t k, void* workspace, float* out_values,
              int64_t* out_indices, hipStream_t st) {
+  if (const int lg = group_lanes_log2(nrows, n, (int)k))
+    return group_run(scores, nrows, n, (int)k, lg, (uint32_t*)workspace, out_values, out_indices, st);
   int64_t sizes[64];
   const int64_t lv = level_sizes(n, (int)k, sizes, 64);
   int64_t amax = 0;

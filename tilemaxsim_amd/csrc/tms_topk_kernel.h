@@ -7,6 +7,9 @@
 // so descending key order is "value descending, then index ascending" -- deterministic,
 // and compared as integers (no float NaN semantics involved).
 //
+// Rows past one chunk at 8 <= k <= 512 go by group maxima (end of this file), the others by
+// the tournament.
+//
 // Tournament: a workgroup selects the best k of a chunk of kChunk keys and each level
 // shrinks a row by kChunk / k until one chunk holds it; the last level sorts its k keys
 // (a last level of at most kShortRow keys runs a chunk of that size over four waves).
@@ -121,16 +124,85 @@ __device__ __forceinline__ uint32_t wave_inclusive_sum(uint32_t x) {
   return x;
 }
 
-// One workgroup of NT threads selects the best k keys of chunk `chunk` of row `row`. The
-// values written by the LAST level are read back from the scores (vals, row stride
-// val_stride) at the selected indices, so they keep the input's bits (-0.0, NaN payloads).
-// Every thread of the workgroup calls it (it synchronises the workgroup).
-template <bool FIRST, bool LAST, int NT, int CH = kChunk>
-__device__ __forceinline__ void topk_chunk(const float* __restrict__ vals, int64_t val_stride,
-                                           const uint64_t* __restrict__ keys_in, int64_t n_in, int64_t in_stride,
-                                           uint64_t* __restrict__ keys_out, int64_t out_stride,
-                                           float* __restrict__ out_vals, int64_t* __restrict__ out_idx, int k,
-                                           int64_t row, int64_t chunk) {
+// The last level's ordering: each of the m distinct keys in sel[0, m) counts the keys
+// above it among sel[0, m8) (m rounded up to a multiple of 8; slots [m, m8 + kRankPad)
+// hold 0, below every real key), and a key of rank < k is written at its rank. S = 8, 4 or 2
+// lanes share a key when the threads allow: lane part p counts among slots
+// [p * m8 / S, (p + 1) * m8 / S), and DPP steps add the S counts.
+constexpr int kRankPad = 48;  // zero slots past m8 that the one-lane-per-key loop may read
+static_assert(kRankSortMaxK + kRankPad <= kMaxK, "the rank step's read ahead stays inside sel");
+template <bool FIRST, int NT>
+__device__ __forceinline__ void topk_rank_out(const uint64_t* sel, const uint32_t* sel_bits, int m, int m8,
+                                              const float* __restrict__ vals, int64_t val_stride,
+                                              float* __restrict__ out_vals, int64_t* __restrict__ out_idx, int k,
+                                              int64_t row) {
+  const int tid = threadIdx.x;
+  const int lg = m * 8 <= NT ? 3 : (m * 4 <= NT ? 2 : (m * 2 <= NT ? 1 : 0));
+  const int S = 1 << lg;
+  const int per = m8 >> lg;
+  for (int t = tid; t < (S > 1 ? S * m8 : m); t += NT) {
+    const int i = t >> lg;
+    const uint64_t me = sel[i];
+    const int j0 = (t & (S - 1)) * per;
+    uint32_t rank = 0u;
+    int j = j0;
+    const int end = j0 + per;
+    if (S == 1) {
+      // One lane per key, the whole range [0, m8) in steps of 32 with the next 16 keys
+      // read ahead, so the LDS latency hides behind the compares (one wave per SIMD has
+      // nothing else to run meanwhile). No exit between a read and its use, so the
+      // compiler keeps the reads ahead. Reads run up to 40 slots past m8 and counts up
+      // to 24, into slots that hold 0 (set with the keys): a 0 key is above nothing.
+      uint64_t xa[16], xb[16];
+      auto load16 = [&](uint64_t(&x)[16], int at) {
+#pragma unroll
+        for (int q = 0; q < 16; q++) x[q] = sel[at + q];
+      };
+      auto count16 = [&](const uint64_t(&x)[16]) {
+#pragma unroll
+        for (int q = 0; q < 16; q++) rank += x[q] > me ? 1u : 0u;
+      };
+      load16(xa, 0);
+      for (j = 0; j < m8; j += 32) {
+        load16(xb, j + 16);
+        count16(xa);
+        load16(xa, j + 32);
+        count16(xb);
+      }
+      j = end;
+    }
+    for (; j + 8 <= end; j += 8) {  // eight reads in flight per step
+      uint64_t x[8];
+#pragma unroll
+      for (int q = 0; q < 8; q++) x[q] = sel[j + q];
+#pragma unroll
+      for (int q = 0; q < 8; q++) rank += x[q] > me ? 1u : 0u;
+    }
+    for (; j < end; j++) rank += sel[j] > me ? 1u : 0u;
+    if (S > 1) {
+      rank += dpp_u32<0xB1>(rank);                 // quad_perm [1,0,3,2]: pairs
+      if (S > 2) rank += dpp_u32<0x4E>(rank);      // quad_perm [2,3,0,1]: quads
+      if (S > 4) rank += dpp_u32<0x141>(rank);     // row_half_mirror: the other quad of the eight
+      if ((t & (S - 1)) != 0) continue;
+    }
+    if (i >= m || rank >= (uint32_t)k) continue;
+    const int64_t idx = (int64_t)(0xffffffffu - (uint32_t)me);
+    if constexpr (FIRST) out_vals[row * k + rank] = __builtin_bit_cast(float, sel_bits[i]);
+    else out_vals[row * k + rank] = vals[row * val_stride + (idx < val_stride ? idx : val_stride - 1)];
+    out_idx[row * k + rank] = idx;
+  }
+}
+
+// One workgroup of NT threads selects the best k of its CH / NT keys a thread (0: padding).
+// FIRST && LAST: v holds the keys' scores, whose own bits are written up to k =
+// kRankSortMaxK; otherwise LAST reads the values back from the scores (vals, row stride
+// val_stride) at the selected indices. Both keep the input's bits (-0.0, NaN payloads). Not LAST: the keys go to keys_out (memory
+// or LDS). Every thread of the workgroup calls it (it synchronises the workgroup).
+template <bool FIRST, bool LAST, int NT, int CH>
+__device__ __forceinline__ void topk_core(uint64_t (&key)[CH / NT], const float (&v)[CH / NT],
+                                          const float* __restrict__ vals, int64_t val_stride, int64_t n_in,
+                                          uint64_t* keys_out, int64_t out_stride, float* __restrict__ out_vals,
+                                          int64_t* __restrict__ out_idx, int k, int64_t row, int64_t chunk) {
   constexpr int kPerThread = CH / NT;
   constexpr int kTopkWaves = NT / 64;
   static_assert(NT % 256 == 0 && NT <= kHistCopies * 256, "histogram clearing and the per-wave copies");
@@ -147,117 +219,8 @@ __device__ __forceinline__ void topk_chunk(const float* __restrict__ vals, int64
   // the loads so the output needs no second read of the scores.
   __shared__ uint32_t sel_bits[(FIRST && LAST) ? kMaxK : 1];
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  const int64_t c0 = chunk * CH;
-  // All loads are issued before any key is formed (one memory round trip, not one per
-  // element). A chunk inside the row reads from one uniform base at 32-bit offsets and
-  // every key is real; in the row's last chunk, positions past the row read its last
-  // element and become padding.
-  uint64_t key[kPerThread];
-  float v[kPerThread];
-  const bool inside = c0 + CH <= n_in;  // uniform
-  if constexpr (FIRST) {
-    if (inside) {
-      const float* __restrict__ base = vals + row * val_stride + c0;
-#pragma unroll
-      for (int e = 0; e < kPerThread; e++) v[e] = base[e * NT + tid];
-      const uint32_t inv = 0xffffffffu - (uint32_t)c0 - (uint32_t)tid;  // inverted index of element 0
-#pragma unroll
-      for (int e = 0; e < kPerThread; e++)
-        key[e] = ((uint64_t)order_key(v[e]) << 32) | (uint64_t)(inv - (uint32_t)(e * NT));
-    } else {
-#pragma unroll
-      for (int e = 0; e < kPerThread; e++) {
-        const int64_t p = c0 + e * NT + tid;
-        v[e] = vals[row * val_stride + (p < n_in ? p : n_in - 1)];
-      }
-#pragma unroll
-      for (int e = 0; e < kPerThread; e++) {
-        const int64_t p = c0 + e * NT + tid;
-        key[e] = p < n_in ? ((uint64_t)order_key(v[e]) << 32) | (uint64_t)(0xffffffffu - (uint32_t)p)
-                          : 0ull;  // below every real element
-      }
-    }
-  } else {
-    if (inside) {
-      const uint64_t* __restrict__ base = keys_in + row * in_stride + c0;
-#pragma unroll
-      for (int e = 0; e < kPerThread; e++) key[e] = base[e * NT + tid];
-    } else {
-#pragma unroll
-      for (int e = 0; e < kPerThread; e++) {
-        const int64_t p = c0 + e * NT + tid;
-        key[e] = keys_in[row * in_stride + (p < n_in ? p : n_in - 1)];
-      }
-#pragma unroll
-      for (int e = 0; e < kPerThread; e++) {
-        const int64_t p = c0 + e * NT + tid;
-        key[e] = p < n_in ? key[e] : 0ull;
-      }
-    }
-  }
-
-  // The last level's ordering: each of the m distinct keys in sel[0, m) counts the keys
-  // above it among sel[0, m8) (m rounded up to a multiple of 8; slots [m, m8 + kRankPad)
-  // hold 0, below every real key), and a key of rank < k is written at its rank. S = 8, 4 or 2
-  // lanes share a key when the threads allow: lane part p counts among slots
-  // [p * m8 / S, (p + 1) * m8 / S), and DPP steps add the S counts.
-  constexpr int kRankPad = 48;  // zero slots past m8 that the one-lane-per-key loop may read
-  static_assert(kRankSortMaxK + kRankPad <= kMaxK, "the rank step's read ahead stays inside sel");
   auto rank_out = [&](int m, int m8) {
-    const int lg = m * 8 <= NT ? 3 : (m * 4 <= NT ? 2 : (m * 2 <= NT ? 1 : 0));
-    const int S = 1 << lg;
-    const int per = m8 >> lg;
-    for (int t = tid; t < (S > 1 ? S * m8 : m); t += NT) {
-      const int i = t >> lg;
-      const uint64_t me = sel[i];
-      const int j0 = (t & (S - 1)) * per;
-      uint32_t rank = 0u;
-      int j = j0;
-      const int end = j0 + per;
-      if (S == 1) {
-        // One lane per key, the whole range [0, m8) in steps of 32 with the next 16 keys
-        // read ahead, so the LDS latency hides behind the compares (one wave per SIMD has
-        // nothing else to run meanwhile). No exit between a read and its use, so the
-        // compiler keeps the reads ahead. Reads run up to 40 slots past m8 and counts up
-        // to 24, into slots that hold 0 (set with the keys): a 0 key is above nothing.
-        uint64_t xa[16], xb[16];
-        auto load16 = [&](uint64_t(&x)[16], int at) {
-#pragma unroll
-          for (int q = 0; q < 16; q++) x[q] = sel[at + q];
-        };
-        auto count16 = [&](const uint64_t(&x)[16]) {
-#pragma unroll
-          for (int q = 0; q < 16; q++) rank += x[q] > me ? 1u : 0u;
-        };
-        load16(xa, 0);
-        for (j = 0; j < m8; j += 32) {
-          load16(xb, j + 16);
-          count16(xa);
-          load16(xa, j + 32);
-          count16(xb);
-        }
-        j = end;
-      }
-      for (; j + 8 <= end; j += 8) {  // eight reads in flight per step
-        uint64_t x[8];
-#pragma unroll
-        for (int q = 0; q < 8; q++) x[q] = sel[j + q];
-#pragma unroll
-        for (int q = 0; q < 8; q++) rank += x[q] > me ? 1u : 0u;
-      }
-      for (; j < end; j++) rank += sel[j] > me ? 1u : 0u;
-      if (S > 1) {
-        rank += dpp_u32<0xB1>(rank);                 // quad_perm [1,0,3,2]: pairs
-        if (S > 2) rank += dpp_u32<0x4E>(rank);      // quad_perm [2,3,0,1]: quads
-        if (S > 4) rank += dpp_u32<0x141>(rank);     // row_half_mirror: the other quad of the eight
-        if ((t & (S - 1)) != 0) continue;
-      }
-      if (i >= m || rank >= (uint32_t)k) continue;
-      const int64_t idx = (int64_t)(0xffffffffu - (uint32_t)me);
-      if constexpr (FIRST) out_vals[row * k + rank] = __builtin_bit_cast(float, sel_bits[i]);
-      else out_vals[row * k + rank] = vals[row * val_stride + (idx < val_stride ? idx : val_stride - 1)];
-      out_idx[row * k + rank] = idx;
-    }
+    topk_rank_out<FIRST, NT>(sel, sel_bits, m, m8, vals, val_stride, out_vals, out_idx, k, row);
   };
 
   if constexpr (FIRST && LAST) {
@@ -563,6 +526,68 @@ __device__ __forceinline__ void topk_chunk(const float* __restrict__ vals, int64
   }
 }
 
+
+// topk_core over chunk `chunk` of row `row`.
+template <bool FIRST, bool LAST, int NT, int CH = kChunk>
+__device__ __forceinline__ void topk_chunk(const float* __restrict__ vals, int64_t val_stride,
+                                           const uint64_t* __restrict__ keys_in, int64_t n_in, int64_t in_stride,
+                                           uint64_t* __restrict__ keys_out, int64_t out_stride,
+                                           float* __restrict__ out_vals, int64_t* __restrict__ out_idx, int k,
+                                           int64_t row, int64_t chunk) {
+  constexpr int kPerThread = CH / NT;
+  const int tid = threadIdx.x;
+  const int64_t c0 = chunk * CH;
+  // All loads are issued before any key is formed (one memory round trip, not one per
+  // element). A chunk inside the row reads from one uniform base at 32-bit offsets and
+  // every key is real; in the row's last chunk, positions past the row read its last
+  // element and become padding.
+  uint64_t key[kPerThread];
+  float v[kPerThread] = {};
+  const bool inside = c0 + CH <= n_in;  // uniform
+  if constexpr (FIRST) {
+    if (inside) {
+      const float* __restrict__ base = vals + row * val_stride + c0;
+#pragma unroll
+      for (int e = 0; e < kPerThread; e++) v[e] = base[e * NT + tid];
+      const uint32_t inv = 0xffffffffu - (uint32_t)c0 - (uint32_t)tid;  // inverted index of element 0
+#pragma unroll
+      for (int e = 0; e < kPerThread; e++)
+        key[e] = ((uint64_t)order_key(v[e]) << 32) | (uint64_t)(inv - (uint32_t)(e * NT));
+    } else {
+#pragma unroll
+      for (int e = 0; e < kPerThread; e++) {
+        const int64_t p = c0 + e * NT + tid;
+        v[e] = vals[row * val_stride + (p < n_in ? p : n_in - 1)];
+      }
+#pragma unroll
+      for (int e = 0; e < kPerThread; e++) {
+        const int64_t p = c0 + e * NT + tid;
+        key[e] = p < n_in ? ((uint64_t)order_key(v[e]) << 32) | (uint64_t)(0xffffffffu - (uint32_t)p)
+                          : 0ull;  // below every real element
+      }
+    }
+  } else {
+    if (inside) {
+      const uint64_t* __restrict__ base = keys_in + row * in_stride + c0;
+#pragma unroll
+      for (int e = 0; e < kPerThread; e++) key[e] = base[e * NT + tid];
+    } else {
+#pragma unroll
+      for (int e = 0; e < kPerThread; e++) {
+        const int64_t p = c0 + e * NT + tid;
+        key[e] = keys_in[row * in_stride + (p < n_in ? p : n_in - 1)];
+      }
+#pragma unroll
+      for (int e = 0; e < kPerThread; e++) {
+        const int64_t p = c0 + e * NT + tid;
+        key[e] = p < n_in ? key[e] : 0ull;
+      }
+    }
+  }
+
+  topk_core<FIRST, LAST, NT, CH>(key, v, vals, val_stride, n_in, keys_out, out_stride, out_vals, out_idx, k, row, chunk);
+}
+
 template <bool FIRST, bool LAST, int NT, int CH = kChunk>
 __global__ void __launch_bounds__(NT) topk_level_kernel(const float* __restrict__ vals, int64_t val_stride,
                                                         const uint64_t* __restrict__ keys_in, int64_t n_in,
@@ -571,6 +596,311 @@ __global__ void __launch_bounds__(NT) topk_level_kernel(const float* __restrict_
                                                         int64_t* __restrict__ out_idx, int k) {
   topk_chunk<FIRST, LAST, NT, CH>(vals, val_stride, keys_in, n_in, in_stride, keys_out, out_stride, out_vals, out_idx, k,
                                   blockIdx.y, blockIdx.x);
+}
+
+// Long rows by group maxima. One pass over the scores writes the largest key of every group
+// of g = 4 << LG consecutive scores, and of every 1,024 (a span). The top k then lie in the
+// k best groups, and those in the k best spans (compared by maximum, then by position): an
+// element outside them has k maxima above it. So one workgroup a row selects spans, then
+// their groups, then the scores of those groups, from at most CHS keys at a time, and reads
+// g k scores again instead of sorting every chunk. The first pass is bound by the read of the
+// scores; the tournament's first level was bound by its issue (VALUBusy 71-81 %).
+constexpr int kSpan = 1024;
+constexpr int kGroupWaves = 4;  // waves per workgroup of the first pass
+
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // rows start at any score
+
+// Largest key over the 1 << LG consecutive lanes of a group (every lane gets it).
+template <int LG>
+__device__ __forceinline__ uint32_t lanes_max_u32(uint32_t x, int lane) {
+  auto mx = [](uint32_t a, uint32_t b) { return a > b ? a : b; };
+  x = mx(x, dpp_u32<0xB1>(x));                       // quad_perm [1,0,3,2]
+  x = mx(x, dpp_u32<0x4E>(x));                       // quad_perm [2,3,0,1]
+  x = mx(x, dpp_u32<0x141>(x));                      // row_half_mirror
+  if constexpr (LG >= 4) x = mx(x, dpp_u32<0x140>(x));  // row_mirror
+  if constexpr (LG >= 5) x = mx(x, swap16_u32(x, lane));
+  if constexpr (LG >= 6) x = mx(x, swap32_u32(x, lane));
+  return x;
+}
+
+// LG = 3..6: 8 to 64 lanes of four scores a group (g = 32 to 256). Each wave walks spans of
+// row blockIdx.y; lane l reads scores 256 j + 4 l .. + 4 of a span, j = 0..3. groups:
+// (nrows, spans * kSpan / g), spans_out (or null): (nrows, spans); 0 for a group past the row.
+template <int LG>
+__global__ void __launch_bounds__(64 * kGroupWaves) topk_group_max_kernel(const float* __restrict__ vals, int64_t n,
+                                                                          int64_t spans,
+                                                                          uint32_t* __restrict__ groups,
+                                                                          uint32_t* __restrict__ spans_out) {
+  constexpr int LPG = 1 << LG;               // lanes per group
+  constexpr int GPL = 64 / LPG;              // groups per 256 scores
+  const int lane = threadIdx.x & 63;
+  const int64_t stride = (int64_t)gridDim.x * kGroupWaves;
+  const int64_t row = blockIdx.y;
+  for (int64_t sp = (int64_t)blockIdx.x * kGroupWaves + (threadIdx.x >> 6); sp < spans; sp += stride) {
+    const float* __restrict__ p = vals + row * n + sp * kSpan;
+    const int64_t left = n - sp * kSpan;  // scores of the row from the span on
+    uint32_t m[4];
+    if (left >= kSpan) {  // uniform
+      f32x4 x[4];
+#pragma unroll
+      for (int j = 0; j < 4; j++) x[j] = __builtin_nontemporal_load((const f32x4u*)(p + 256 * j + 4 * lane));
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        // the float maximum's key, or the NaN key when some score's bits (sign shifted out)
+        // are a NaN's, about two operations a score
+        const float f = fmaxf(fmaxf(x[j][0], x[j][1]), fmaxf(x[j][2], x[j][3]));
+        uint32_t nan = 0u;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          const float xq = x[j][q];
+          const uint32_t b = __builtin_bit_cast(uint32_t, xq) << 1;
+          nan = b > nan ? b : nan;
+        }
+        const uint32_t fb = __builtin_bit_cast(uint32_t, f);
+        const uint32_t o = (int32_t)fb < 0 ? 0u - fb : (fb | 0x80000000u);
+        m[j] = nan > 0xff000000u ? 0xffffffffu : o;
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        float x[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          const int64_t i = 256 * j + 4 * lane + q;
+          x[q] = p[i < left ? i : left - 1];
+        }
+        m[j] = 0u;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          const uint32_t b = 256 * j + 4 * lane + q < left ? order_key(x[q]) : 0u;
+          m[j] = b > m[j] ? b : m[j];
+        }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) m[j] = lanes_max_u32<LG>(m[j], lane);
+    // lane j of a group's lanes keeps the j-th 256 scores' maximum
+    const int j = lane & (LPG - 1);
+    const uint32_t mine = j == 0 ? m[0] : (j == 1 ? m[1] : (j == 2 ? m[2] : m[3]));
+    if (j < 4) groups[(row * spans + sp) * (4 * GPL) + j * GPL + lane / LPG] = mine;
+    if (spans_out) {
+      uint32_t a = m[0] > m[1] ? m[0] : m[1], b = m[2] > m[3] ? m[2] : m[3];
+      a = wave_max_u32(a > b ? a : b, lane);
+      if (lane == 0) spans_out[row * spans + sp] = a;
+    }
+  }
+}
+
+// The selection of one row: spans (when spans_in is given: at most CH1 of them), their
+// groups, their scores. lg: groups of 4 << lg scores, at most CHS / k of them in a span and
+// at most CHS / k scores in a group; without spans_in, at most CHS groups a row.
+//
+// First the fast way: the k-th largest maximum T is a bound on the k-th largest score, so
+// after one selection among the maxima only what reaches T is kept: the k best spans' groups,
+// those groups' scores (on continuous scores a few more than k), and the scores kept are
+// ordered by rank. Lists that outgrow kFastCap (sorted rows, ties) take the selection level
+// by level. 32 rows of 1M scores, k = 100: 32 us with the first pass, against 58 for the
+// tournament and 41 selecting level by level throughout.
+constexpr int kFastCap = 2048;
+template <int CH1, int CHS>
+__global__ void __launch_bounds__(kLastThreads) topk_group_last_kernel(const float* __restrict__ vals, int64_t n,
+                                                                       int64_t spans, int lg,
+                                                                       const uint32_t* __restrict__ groups,
+                                                                       const uint32_t* __restrict__ spans_in,
+                                                                       float* __restrict__ out_vals,
+                                                                       int64_t* __restrict__ out_idx, int k) {
+  constexpr int NT = kLastThreads, NW = NT / 64;
+  constexpr int PER = CHS / NT;
+  __shared__ uint64_t picked[kMaxK];
+  const int tid = threadIdx.x;
+  const int64_t row = blockIdx.x;
+  const int per = kSpan >> (lg + 2);  // groups per span
+  const int glog = lg + 2;            // log2 of the scores per group
+  const uint32_t* __restrict__ grow = groups + row * spans * per;
+  const float* __restrict__ vrow = vals + row * n;
+
+  {
+    __shared__ uint64_t list[kFastCap];
+    __shared__ uint32_t wave_t[NW], n_list, n_groups, n_sel, bound;
+    __shared__ uint32_t gsel[kFastCap];
+    __shared__ uint64_t sel[kFastCap + kRankPad + 8];
+    __shared__ uint32_t sel_bits[kFastCap];
+    const int lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // appends the lanes with `take` to a list; returns the lane's slot
+    auto slot = [&](uint32_t* count, bool take) -> uint32_t {
+      const uint64_t mask = __ballot(take);
+      uint32_t base = 0u;
+      if (mask != 0ull) {
+        if (lane == 0) base = atomicAdd(count, (uint32_t)__popcll(mask));
+        base = (uint32_t)__builtin_amdgcn_readlane((int)base, 0);
+      }
+      return base + __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+    };
+    // the maxima of the first level, spread over the waves (wave c % 16 holds maximum c)
+    constexpr int P1 = (CH1 > CHS ? CH1 : CHS) / NT;
+    const uint32_t* __restrict__ top = spans_in ? spans_in + row * spans : grow;
+    const int count = (int)(spans_in ? spans : spans * per);
+    uint32_t x[P1];
+    uint32_t tm = 0u;
+#pragma unroll
+    for (int e = 0; e < P1; e++) {
+      const int c = e * NT + lane * NW + wid;
+      x[e] = c < count ? top[c] : 0u;
+      tm = x[e] > tm ? x[e] : tm;
+    }
+    if (tid == 0) n_list = n_groups = n_sel = 0u;
+    for (int i = tid; i < kFastCap + kRankPad + 8; i += NT) sel[i] = 0ull;
+    // a lower bound on the k-th maximum, as in topk_core's pre-filter
+    const uint32_t j = (uint32_t)((k + NW - 1) / NW);
+    uint32_t t = 0u;
+#pragma unroll
+    for (int b = 31; b >= 0; b--) {
+      const uint32_t c = t | (1u << b);
+      t = (uint32_t)__popcll(__ballot(tm >= c)) >= j ? c : t;
+    }
+    if (lane == 0) wave_t[wid] = t;
+    __syncthreads();
+    uint32_t T = wave_t[0];
+#pragma unroll
+    for (int w = 1; w < NW; w++) T = wave_t[w] < T ? wave_t[w] : T;
+    bool ok = T != 0u;  // uniform, as every decision below
+    if (ok) {
+#pragma unroll
+      for (int e = 0; e < P1; e++) {
+        if (e * NT >= count) break;
+        const int c = e * NT + lane * NW + wid;
+        const bool take = x[e] >= T;
+        const uint32_t at = slot(&n_list, take);
+        if (take && at < (uint32_t)kFastCap) list[at] = ((uint64_t)x[e] << 32) | (uint64_t)(0xffffffffu - (uint32_t)c);
+      }
+      __syncthreads();
+      const int m = (int)n_list;
+      ok = m <= kFastCap;
+      if (ok) {
+        // ranks by count, four or two lanes a key for a short list: the keys of rank < k are the k
+        // best, in order, and the last of them is the bound
+        const int lgS = m <= NT / 4 ? 2 : (m <= NT / 2 ? 1 : 0);
+        const int part = tid & ((1 << lgS) - 1);
+        for (int i = tid >> lgS; i < m; i += NT >> lgS) {  // one turn when lanes share keys
+          const uint64_t me = list[i];
+          uint32_t rank = 0u;
+#pragma unroll 8
+          for (int q = part; q < m; q += 1 << lgS) rank += list[q] > me ? 1u : 0u;
+          if (lgS > 0) rank += dpp_u32<0xB1>(rank);  // a key's lanes take the turn together
+          if (lgS > 1) rank += dpp_u32<0x4E>(rank);
+          if (part == 0 && rank < (uint32_t)k) {
+            picked[rank] = me;
+            if (rank == (uint32_t)k - 1u) bound = (uint32_t)(me >> 32);
+          }
+        }
+        __syncthreads();
+        T = bound;
+        uint32_t ng;
+        if (spans_in) {
+          uint32_t at[PER], y[PER];
+#pragma unroll
+          for (int e = 0; e < PER; e++) {
+            const int c = e * NT + tid;
+            const uint32_t span = c < k * per ? 0xffffffffu - (uint32_t)picked[c / per] : 0u;
+            at[e] = span * (uint32_t)per + (uint32_t)(c & (per - 1));
+            y[e] = c < k * per ? grow[at[e]] : 0u;
+          }
+#pragma unroll
+          for (int e = 0; e < PER; e++) {
+            const bool take = y[e] >= T;  // T > 0
+            const uint32_t p = slot(&n_groups, take);
+            if (take && p < (uint32_t)kFastCap) gsel[p] = at[e];
+          }
+          __syncthreads();
+          ng = n_groups;
+        } else {
+          if (tid < k) gsel[tid] = 0xffffffffu - (uint32_t)picked[tid];
+          __syncthreads();
+          ng = (uint32_t)k;
+        }
+        ok = ng <= (uint32_t)kFastCap && (int)(ng << glog) <= 4 * CHS;
+        if (ok) {
+          for (int c0 = 0; c0 < (int)(ng << glog); c0 += CHS) {
+            float y[PER];
+            uint32_t at[PER];
+#pragma unroll
+            for (int e = 0; e < PER; e++) {
+              const int c = c0 + e * NT + tid;
+              const bool in = c < (int)(ng << glog);
+              const uint64_t i64 = ((uint64_t)gsel[in ? c >> glog : 0] << glog) + (uint64_t)(c & ((1 << glog) - 1));
+              at[e] = in && i64 < (uint64_t)n ? (uint32_t)i64 : 0xffffffffu;
+              y[e] = vrow[at[e] != 0xffffffffu ? at[e] : 0u];
+            }
+#pragma unroll
+            for (int e = 0; e < PER; e++) {
+              const uint32_t o = order_key(y[e]);
+              const bool take = at[e] != 0xffffffffu && o >= T;
+              const uint32_t p = slot(&n_sel, take);
+              if (take && p < (uint32_t)kFastCap) {
+                sel[p] = ((uint64_t)o << 32) | (uint64_t)(0xffffffffu - at[e]);
+                sel_bits[p] = __builtin_bit_cast(uint32_t, y[e]);
+              }
+            }
+          }
+          __syncthreads();
+          const int ms = (int)n_sel;  // >= k: each of the k best maxima is one
+          if (ms <= kFastCap) {
+            topk_rank_out<true, NT>(sel, sel_bits, ms, (ms + 7) & ~7, nullptr, 0, out_vals, out_idx, k, row);
+            return;
+          }
+        }
+      }
+    }
+    __syncthreads();
+  }
+
+  uint64_t key[PER];
+  float v[PER] = {};
+  if (spans_in) {
+    uint64_t k1[CH1 / NT];
+    const float none[CH1 / NT] = {};
+#pragma unroll
+    for (int e = 0; e < CH1 / NT; e++) {
+      const int64_t c = e * NT + tid;
+      k1[e] = c < spans ? ((uint64_t)spans_in[row * spans + c] << 32) | (uint64_t)(0xffffffffu - (uint32_t)c) : 0ull;
+    }
+    topk_core<false, false, NT, CH1>(k1, none, nullptr, 0, spans, picked, 0, nullptr, nullptr, k, 0, 0);
+    __syncthreads();
+    uint32_t at[PER];
+#pragma unroll
+    for (int e = 0; e < PER; e++) {
+      const int c = e * NT + tid;
+      const uint32_t span = c < k * per ? 0xffffffffu - (uint32_t)picked[c / per] : 0u;
+      at[e] = span * (uint32_t)per + (uint32_t)(c & (per - 1));
+      key[e] = c < k * per ? (uint64_t)grow[at[e]] : 0ull;
+    }
+#pragma unroll
+    for (int e = 0; e < PER; e++) key[e] = key[e] != 0ull ? (key[e] << 32) | (uint64_t)(0xffffffffu - at[e]) : 0ull;
+    __syncthreads();  // picked is read; the next selection writes it
+  } else {
+#pragma unroll
+    for (int e = 0; e < PER; e++) {
+      const int64_t c = e * NT + tid;
+      const uint32_t x = c < spans * per ? grow[c] : 0u;
+      key[e] = x != 0u ? ((uint64_t)x << 32) | (uint64_t)(0xffffffffu - (uint32_t)c) : 0ull;
+    }
+  }
+  topk_core<false, false, NT, CHS>(key, v, nullptr, 0, CHS, picked, 0, nullptr, nullptr, k, 0, 0);
+  __syncthreads();
+  uint32_t at[PER];
+#pragma unroll
+  for (int e = 0; e < PER; e++) {
+    const int c = e * NT + tid;
+    const uint64_t pk = c < k << (lg + 2) ? picked[c >> (lg + 2)] : 0ull;
+    // a padding key (fewer than k groups) names no group
+    const uint64_t i = (uint64_t)(0xffffffffu - (uint32_t)pk) * (uint64_t)(4 << lg) + (uint64_t)(c & ((4 << lg) - 1));
+    at[e] = pk != 0ull && i < (uint64_t)n ? (uint32_t)i : 0xffffffffu;
+    v[e] = vrow[at[e] != 0xffffffffu ? at[e] : 0u];
+  }
+#pragma unroll
+  for (int e = 0; e < PER; e++)
+    key[e] = at[e] != 0xffffffffu ? ((uint64_t)order_key(v[e]) << 32) | (uint64_t)(0xffffffffu - at[e]) : 0ull;
+  topk_core<true, true, NT, CHS>(key, v, vals, n, n, nullptr, 0, out_vals, out_idx, k, row, 0);
 }
 
 }  // namespace tms
