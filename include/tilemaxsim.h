@@ -333,6 +333,17 @@ int tms_maxsim_residual_checked(const void* Qs, int64_t nQ, int64_t nq, int64_t 
                                 int64_t* verdict, void* stream);
 
 /*
+ * PQ codes (`count` of code_bytes = 1, 2 or 4 bytes; 2 and 4 signed) checked to lie in [0, K):
+ * tms_codes_check launches the check, tms_codes_verdict waits for its verdict and returns
+ * TMS_ERR_BOUNDS when a code does not; scoring calls may be launched in between. `verdict`
+ * as for the *_checked calls: every successful tms_codes_check is followed by one
+ * tms_codes_verdict before the words are used again. No reference counterpart (the reference
+ * gathers out of range).
+ */
+int tms_codes_check(const void* codes, int64_t count, int code_bytes, int64_t K, int64_t* verdict, void* stream);
+int tms_codes_verdict(const int64_t* verdict, void* stream);
+
+/*
  * Measurement helper, not part of the scoring path and with no counterpart in the
  * reference: reads `bytes` (a multiple of 8 KiB) of `buf` once with a read-only
  * streaming kernel and writes one XOR word per thread to `sink`

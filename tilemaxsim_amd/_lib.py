@@ -73,6 +73,8 @@ SIGNATURES = {
                                   _c_void_p, _c_void_p, _c_void_p],
     "tms_maxsim_packed_checked": [_c_void_p, _i64, _i64, _c_void_p, _i64, _c_void_p, _i64, _int, _int, _c_void_p,
                                   _c_void_p, _c_void_p, _c_void_p, _c_void_p],
+    "tms_codes_check": [_c_void_p, _i64, _int, _i64, _c_void_p, _c_void_p],
+    "tms_codes_verdict": [_c_void_p, _c_void_p],
     "tms_maxsim_residual_checked": [_c_void_p, _i64, _i64, _i64, _c_void_p, _i64, _c_void_p, _int, _c_void_p, _c_void_p,
                                     _i64, _c_void_p, _i64, _c_void_p, _i64, _int, _int, _c_void_p, _c_void_p, _c_void_p,
                                     _c_void_p],

@@ -52,18 +52,46 @@ class TileMaxSimPQ:
         _check.same_device(Q=Q, codebook=self.codebook)
         return _check.query_for(Q, self.codebook.dtype)
 
-    def _codes(self, codes: torch.Tensor, validate: bool) -> torch.Tensor:
+    def _codes(self, codes: torch.Tensor, validate: bool) -> tuple[torch.Tensor, bool]:
+        """The codes as the kernels take them, and whether their range is still to be checked
+        (by :meth:`_checked`, beside the scoring kernels)."""
         if codes.dtype.is_floating_point or codes.dtype == torch.bool:
             raise TypeError(f"codes must be an integer tensor, got {codes.dtype}")
         _check.on_gpu("codes", codes)
         _check.same_device(codes=codes, codebook=self.codebook)
-        if validate and codes.numel() > 0 and (codes.dtype != torch.uint8 or self.K < 256):
-            lo, hi = int(codes.min()), int(codes.max())
-            if lo < 0 or hi >= self.K:
-                raise ValueError(f"codes must lie in [0, K={self.K}), found [{lo}, {hi}]")
+        check = validate and codes.numel() > 0 and (codes.dtype != torch.uint8 or self.K < 256)
         if codes.dtype not in _CODE_FLAGS:
+            if check:
+                self._refuse(codes)  # as they are, before they are converted
+                check = False
             codes = codes.to(torch.int32)
-        return codes.contiguous()
+        return codes.contiguous(), check
+
+    def _refuse(self, codes: torch.Tensor) -> None:
+        lo, hi = int(codes.min()), int(codes.max())
+        if lo < 0 or hi >= self.K:
+            raise ValueError(f"codes must lie in [0, K={self.K}), found [{lo}, {hi}]")
+
+    def _checked(self, codes: torch.Tensor, score):
+        """``score()``, with the codes' range checked by a kernel in front of it; only the
+        check's verdict is waited for."""
+        lib = _lib.load()
+        verdict, stream = _lib.verdict_ptr(), _lib.stream_of(codes)
+        with _lib.on_device(codes.device):
+            _lib.check(lib.tms_codes_check(codes.data_ptr(), codes.numel(), _CODE_BYTES[codes.dtype], self.K, verdict,
+                                           stream))
+        error = None
+        try:
+            scores = score()
+        except BaseException as e:  # the verdict's words are this call's until it is read
+            error = e
+        status = lib.tms_codes_verdict(verdict, stream)
+        if status == _lib.TMS_ERR_BOUNDS:
+            self._refuse(codes)
+        if error is not None:
+            raise error
+        _lib.check(status)
+        return scores
 
     def _table(self, Q: torch.Tensor, qcode: int) -> torch.Tensor:
         Nq = Q.shape[0]
@@ -95,8 +123,8 @@ class TileMaxSimPQ:
                 width), or any other integer dtype (converted to int32), values < K.
             method: "auto" (MFMA kernel when the shape allows it, else the table path),
                 "mfma" or "lut".
-            validate: check that codes lie in [0, K) (one device-to-host copy; skipped
-                for uint8 codes when K >= 256, where every byte is valid).
+            validate: check that codes lie in [0, K) (a kernel whose verdict is waited for;
+                skipped for uint8 codes when K >= 256, where every byte is valid).
 
         Returns:
             (B,) float32 MaxSim scores; a document with Nd == 0 scores -inf.
@@ -109,7 +137,13 @@ class TileMaxSimPQ:
         if method not in ("auto", "mfma", "lut"):
             raise ValueError(f"method must be 'auto', 'mfma' or 'lut', got {method!r}")
         Q, qcode = self._query(Q)
-        codes = self._codes(codes, validate)
+        codes, check = self._codes(codes, validate)
+        if not check:
+            return self._score(Q, qcode, codes, method)
+        return self._checked(codes, lambda: self._score(Q, qcode, codes, method))
+
+    def _score(self, Q: torch.Tensor, qcode: int, codes: torch.Tensor, method: str) -> torch.Tensor:
+        B, Nd, _ = codes.shape
         Nq = Q.shape[0]
         scores = torch.empty(B, dtype=torch.float32, device=Q.device)
         if B == 0:
@@ -152,7 +186,13 @@ class TileMaxSimPQ:
         _check.on_gpu("Qs", Qs)
         _check.same_device(Qs=Qs, codebook=self.codebook)
         Qs, qcode = _check.query_for(Qs, self.codebook.dtype)
-        codes = self._codes(codes, validate)
+        codes, check = self._codes(codes, validate)
+        if not check:
+            return self._score_queries(Qs, qcode, codes)
+        return self._checked(codes, lambda: self._score_queries(Qs, qcode, codes))
+
+    def _score_queries(self, Qs: torch.Tensor, qcode: int, codes: torch.Tensor) -> torch.Tensor:
+        B, Nd, _ = codes.shape
         nQ, Nq = Qs.shape[0], Qs.shape[1]
         scores = torch.empty(nQ, B, dtype=torch.float32, device=Qs.device)
         if B == 0 or nQ == 0:
