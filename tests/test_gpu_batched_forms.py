@@ -96,3 +96,24 @@ def test_pq(cuda, M, K, dsub, nQ, nq, B):
     for q in {0, nQ // 2, nQ - 1}:
         ref, lim = bar.with_bound(orc.maxsim_f64, Qs[q].float().numpy(), D)
         bar.assert_scores(got[q][pick], ref, lim, f"query {q}")
+
+
+@pytest.mark.parametrize("d,nbits", [(128, 2), (96, 1), (64, 4), (32, 2)])
+@pytest.mark.parametrize("nQ,nq", [f for f in FORMS if f[1] <= 96])
+def test_residual_bits(cuda, nQ, nq, d, nbits):
+    """A query's scores over a residual index are the same bits in every form."""
+    import torch
+    import tilemaxsim_amd as tms
+    rng = np.random.default_rng(nQ * 17 + nq + d)
+    lens = rng.integers(0, 60, 140)
+    offsets = torch.from_numpy(np.concatenate([[0], np.cumsum(lens)])).cuda()
+    T = int(offsets[-1])
+    index = (torch.from_numpy(rng.integers(0, 50, T).astype(np.int32)).cuda(),
+             torch.from_numpy(rng.integers(0, 256, (T, d * nbits // 8)).astype(np.uint8)).cuda(),
+             torch.from_numpy(_emb(rng, 50, d)).half().cuda(),
+             torch.linspace(-0.1, 0.1, 1 << nbits).half().cuda(), nbits, offsets)
+    Qs = torch.from_numpy(_emb(rng, nQ, nq, d)).half().cuda()
+    got = tms.flashmaxsim_score_residual_batched(Qs, *index)
+    for q in {0, nQ // 2, nQ - 1}:
+        two = tms.flashmaxsim_score_residual_batched(torch.stack([Qs[q], Qs[0]]), *index)[0]
+        assert torch.equal(got[q].view(torch.int32), two.view(torch.int32)), f"query {q}"

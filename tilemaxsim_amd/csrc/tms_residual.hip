@@ -25,6 +25,7 @@
 // rounding x to fp16 first (differences ~1e-4 relative on unit-norm data).
 #include <string.h>
 
+#include "tms_batched_kernel.h"
 #include "tms_check.h"
 
 namespace tms {
@@ -52,7 +53,7 @@ struct ResArgs {
   int64_t B, ndocs, T, ncent;
   PadLen pad;
   int32_t nq, nbq, blk0, d, rb, docs_per_wave;
-  int32_t nblk, blk_end;  // batched kernel: blocks per wave, one past the launch's last block
+  int32_t nblk_l, nblk_x, blk_end;  // batched: blocks of each wave 0-3 and 4-7, one past the launch's last
   int32_t wpd;            // fused kernel: waves per document (1: each wave walks whole documents)
 };
 
@@ -491,11 +492,12 @@ __global__ void __launch_bounds__(256) residual_maxsim_kernel(ResArgs a) {
 }
 
 // ---------------------------------------------------------------------------------
-// Batched queries over residual-compressed documents. One workgroup of eight waves per
-// CU walks a run of documents in 16-token tiles, every wave the same tiles. A tile is
+// Batched queries over residual-compressed documents. A workgroup of one of the dense
+// batched kernel's forms (tms_batched_kernel.h: four waves, or eight, of NB query blocks each)
+// walks a run of documents in 16-token tiles, every wave the same tiles. A tile is
 // decoded once: wave w < KS decodes k-step w (lane (r, g): chunk 4 w + g of token r, the
 // MFMA A-operand layout), the KS partial |v|^2 of each token meet in LDS, and the
-// normalised x = fp16(v * (1 / fp16(|v|))) goes to an LDS ring from which all eight
+// normalised x = fp16(v * (1 / fp16(|v|))) goes to an LDS ring from which all the
 // waves score the tile against the query blocks they hold, as the dense batched kernel
 // does. Step i opens with one LDS-only barrier and then: reads tile i+1's fragments;
 // (decoding waves) issues the ids of tile i+7 and the centroid chunks / residual bytes of
@@ -503,30 +505,33 @@ __global__ void __launch_bounds__(256) residual_maxsim_kernel(ResArgs a) {
 // barrier) and decodes tile i+3 (its partial norms to LDS); scores tile i. The decoding
 // work precedes the wave's own MFMAs, so it overlaps the MFMAs of the scoring-only wave
 // that shares its SIMD instead of stalling the barrier after them.
-constexpr int kResBatchedWaves = 8;
+// With few queries the decode outweighs the scoring, and the workgroups of four waves on one
+// CU overlap each other's: 4, 8, 16, 24, 32 and 34 queries over 50,000 documents (5M tokens, 2
+// bits) take 388, 502, 772, 1242, 1399 and 1772 us, against 691, 694, 1143, 1405, 1418 and
+// 2737 with eight waves of 1, 2 or 4 blocks for every pass.
+constexpr int kResSlots = 3;  // slots of every pipeline buffer: x tiles, partial norms, bodies, ids
+struct ResShared {
+  uint8_t lut[4096];
+  u32x4 ring[kResSlots][4][64];
+  f32x4 nrm[kResSlots][16];  // partial |v|^2 of token r from decoding wave w, at [slot][r][w]
+};
 
-template <int KS, int NBITS, int NB>
-__global__ void __launch_bounds__(64 * kResBatchedWaves, 1) residual_batched_kernel(ResArgs a) {
-  constexpr int NS = 3;  // slots of every pipeline buffer: x tiles, partial norms, bodies, ids
-  __shared__ __attribute__((aligned(16))) uint8_t lut[4096];
-  __shared__ u32x4 ring[NS][4][64];
-  __shared__ f32x4 nrm[NS][16];  // partial |v|^2 of token r from decoding wave w, at [slot][r][w]
-  build_lut<NBITS>(lut, a.weights);
-
+template <int KS, int NBITS, int NB, bool DEC>
+__device__ __forceinline__ void residual_batched_body(const ResArgs& a, ResShared& sh, int wid, int my_blk0,
+                                                      int my_nblk) {
+  constexpr int NS = kResSlots;
+  uint8_t* lut = sh.lut;
+  u32x4(&ring)[NS][4][64] = sh.ring;
+  f32x4(&nrm)[NS][16] = sh.nrm;
   const int lane = threadIdx.x & 63;
   const int r = lane & 15, g = lane >> 4;
-  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // scalar: `decoder` branches stay uniform
-  const bool decoder = wid < KS;
   const float NEG_INF = -__builtin_inff();
 
   const int64_t b_begin = wave_uniform((int64_t)blockIdx.x * a.docs_per_wave);
   const int64_t b_end = (b_begin + a.docs_per_wave < a.B) ? b_begin + a.docs_per_wave : a.B;
   const int64_t ndocs = b_end - b_begin;  // >= 1: the host launches no empty workgroup
 
-  // Query blocks: wave w holds blocks blk0 + w * nblk + j (whole queries).
-  const int my_blk0 = a.blk0 + wid * a.nblk;
-  int my_nblk = a.blk_end - my_blk0;  // <= 0 for a wave with no query
-  if (my_nblk > a.nblk) my_nblk = a.nblk;
+  // Query blocks: the wave holds blocks my_blk0 .. my_blk0 + my_nblk - 1 (whole queries).
   u32x4 qf[NB][KS][2];
   bool qv[NB][2];
 #pragma unroll
@@ -616,11 +621,10 @@ __global__ void __launch_bounds__(64 * kResBatchedWaves, 1) residual_batched_ker
   wc.t0 = 0;
   seek(wc, b_begin, true);
 
-  // The pipeline, instantiated twice: decoding waves (loads, decode, ring writes) and
-  // scoring-only waves, so each copy's loads are straight-line code whose outstanding
-  // count the compiler tracks exactly (a load under a branch would make it wait for all).
-  auto pipeline = [&](auto dec_tag) {
-    constexpr bool DEC = decltype(dec_tag)::value == 1;
+  // Decoding waves (loads, decode, ring writes) and scoring-only waves are separate
+  // instantiations, so each copy's loads are straight-line code whose outstanding count the
+  // compiler tracks exactly (a load under a branch would make it wait for all).
+  auto pipeline = [&]() {
     wb = wc;
     wi = wc;
     __syncthreads();  // the byte table is built
@@ -763,10 +767,7 @@ __global__ void __launch_bounds__(64 * kResBatchedWaves, 1) residual_batched_ker
       if (step(RingSlot<5>{})) break;
     }
   };
-  if (wc.b < b_end) {
-    if (decoder) pipeline(RingSlot<1>{});
-    else pipeline(RingSlot<0>{});
-  }
+  if (wc.b < b_end) pipeline();
 
   // coalesced store: lane i writes document b_begin + i for each of the wave's queries
   if (my_nblk > 0 && lane < ndocs) {
@@ -786,6 +787,20 @@ __global__ void __launch_bounds__(64 * kResBatchedWaves, 1) residual_batched_ker
       }
     }
   }
+}
+
+template <int KS, int NBITS, int NBL, int NBX, int W>
+__global__ void __launch_bounds__(64 * W, W == 8 || NBX > 2 ? 2 : (NBX == 2 ? 3 : 4)) residual_batched_kernel(ResArgs a) {
+  __shared__ __attribute__((aligned(16))) ResShared sh;
+  build_lut<NBITS>(sh.lut, a.weights);  // a barrier before the first decode
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int my_blk0 = a.blk0 + (wid < 4 ? wid * a.nblk_l : 4 * a.nblk_l + (wid - 4) * a.nblk_x);
+  int my_nblk = a.blk_end - my_blk0;  // <= 0 for a wave with no query
+  const int most = wid < 4 ? a.nblk_l : a.nblk_x;
+  if (my_nblk > most) my_nblk = most;
+  if (wid < KS) residual_batched_body<KS, NBITS, NBL, true>(a, sh, wid, my_blk0, my_nblk);
+  else if (W == 4 || wid < 4) residual_batched_body<KS, NBITS, NBL, false>(a, sh, wid, my_blk0, my_nblk);
+  else residual_batched_body<KS, NBITS, NBX, false>(a, sh, wid, my_blk0, my_nblk);
 }
 
 // ---------------------------------------------------------------------------------
@@ -852,9 +867,6 @@ static int check_format(const char* fn, int64_t d, int nbits, int64_t ncent, con
 #ifndef TMS_RES_QLDS
 #define TMS_RES_QLDS 1  // query fragments in LDS
 #endif
-#ifndef TMS_RES_BATCHED_TOKENS
-#define TMS_RES_BATCHED_TOKENS 4096  // document tokens one batched workgroup walks (whole documents)
-#endif
 // One residual load per token when the lane's run of KS*nbits bytes is a power of two and
 // the residuals pointer is aligned to it (rows are 4*KS*nbits bytes, so every run is).
 template <int KS, int NBITS, bool SPLIT>
@@ -885,22 +897,26 @@ static int launch_fused_ks(const ResArgs& a, int nbits, int64_t grid, hipStream_
   return check_launch("residual_maxsim_kernel");
 }
 
-template <int KS, int NB>
-static int launch_batched_nb(const ResArgs& a, int nbits, int64_t grid, hipStream_t st) {
-  const dim3 blk(64 * kResBatchedWaves);
-  if (nbits == 1) hipLaunchKernelGGL((residual_batched_kernel<KS, 1, NB>), dim3((unsigned)grid), blk, 0, st, a);
-  else if (nbits == 2) hipLaunchKernelGGL((residual_batched_kernel<KS, 2, NB>), dim3((unsigned)grid), blk, 0, st, a);
-  else hipLaunchKernelGGL((residual_batched_kernel<KS, 4, NB>), dim3((unsigned)grid), blk, 0, st, a);
-  return check_launch("residual_batched_kernel");
-}
-constexpr int kResMaxBlocksPerWave = 4;
-template <int KS>
-static int launch_batched_ks(const ResArgs& a, int nbits, int nb, int64_t grid, hipStream_t st) {
-  switch (nb) {
-    case 1: return launch_batched_nb<KS, 1>(a, nbits, grid, st);
-    case 2: return launch_batched_nb<KS, 2>(a, nbits, grid, st);
-    default: return launch_batched_nb<KS, kResMaxBlocksPerWave>(a, nbits, grid, st);
+template <int KS, int NBITS>
+static void launch_batched_form(const ResArgs& a, int f, int64_t grid, hipStream_t st) {
+  const dim3 g((unsigned)grid);
+  switch (f) {  // kBatchedForms
+    case 0: hipLaunchKernelGGL((residual_batched_kernel<KS, NBITS, 1, 1, 4>), g, dim3(256), 0, st, a); break;
+    case 1: hipLaunchKernelGGL((residual_batched_kernel<KS, NBITS, 2, 2, 4>), g, dim3(256), 0, st, a); break;
+    case 2: hipLaunchKernelGGL((residual_batched_kernel<KS, NBITS, 3, 3, 4>), g, dim3(256), 0, st, a); break;
+    case 3: hipLaunchKernelGGL((residual_batched_kernel<KS, NBITS, 4, 4, 4>), g, dim3(256), 0, st, a); break;
+    case 4: hipLaunchKernelGGL((residual_batched_kernel<KS, NBITS, 2, 3, 8>), g, dim3(512), 0, st, a); break;
+    case 5: hipLaunchKernelGGL((residual_batched_kernel<KS, NBITS, 3, 3, 8>), g, dim3(512), 0, st, a); break;
+    case 6: hipLaunchKernelGGL((residual_batched_kernel<KS, NBITS, 3, 4, 8>), g, dim3(512), 0, st, a); break;
+    default: hipLaunchKernelGGL((residual_batched_kernel<KS, NBITS, 4, 4, 8>), g, dim3(512), 0, st, a); break;
   }
+}
+template <int KS>
+static int launch_batched_ks(const ResArgs& a, int nbits, int f, int64_t grid, hipStream_t st) {
+  if (nbits == 1) launch_batched_form<KS, 1>(a, f, grid, st);
+  else if (nbits == 2) launch_batched_form<KS, 2>(a, f, grid, st);
+  else launch_batched_form<KS, 4>(a, f, grid, st);
+  return check_launch("residual_batched_kernel");
 }
 
 // Arguments shared by the two MaxSim entry points; returns TMS_OK with `a` filled, or an
@@ -1001,7 +1017,7 @@ static int residual_many(const char* fn, const void* Qs, int64_t nQ, int64_t nq,
                        offsets, ndocs, pids, B, pad, out, st, a);
   if (rc) return rc < 0 ? TMS_OK : rc;
   const int64_t nblocks = nQ * (int64_t)a.nbq;
-  if (a.nbq > kResMaxBlocksPerWave || nblocks < 2) {  // one query at a time
+  if (a.nbq > kMaxBlocksPerWave || nblocks < 2) {  // one query at a time
     for (int64_t qi = 0; qi < nQ; qi++) {
       rc = residual_one(fn, (const uint8_t*)Qs + qi * nq * d * 2, nq, d, centroids, ncent, bucket_weights, nbits,
                                codes, residuals, total_tokens, offsets, ndocs, pids, B, pad, out + qi * B, stream);
@@ -1010,34 +1026,28 @@ static int residual_many(const char* fn, const void* Qs, int64_t nQ, int64_t nq,
     return TMS_OK;
   }
   if (nblocks > ((int64_t)1 << 30)) return fail(TMS_ERR_UNSUPPORTED, "%s: too many queries", fn);
-  // Blocks per wave: the smallest of 1, 2, 4 whose launch covers every block in one pass
-  // (a wave computes all of its slots, used or not), else 4. A wave holds whole queries.
-  int nb = kResMaxBlocksPerWave;
-  for (int c = 1; c < kResMaxBlocksPerWave; c *= 2)
-    if (c >= a.nbq && nblocks <= (int64_t)kResBatchedWaves * ((c / a.nbq) * a.nbq)) {
-      nb = c;
-      break;
-    }
-  a.nblk = (nb / a.nbq) * a.nbq;
-  // about TMS_RES_BATCHED_TOKENS tokens per workgroup (whole documents, at most 64), at
-  // least four rounds of one workgroup per CU
+  // passes as the dense batched call's (batched_run)
+  constexpr int nf = (int)(sizeof(kBatchedForms) / sizeof(BatchedForm));
   const int64_t hint = ndocs > 0 ? total_tokens / ndocs : 1;
-  int64_t dpw = hint > 0 ? TMS_RES_BATCHED_TOKENS / hint : 1;
-  if (dpw > 1 && B / dpw < (int64_t)256 * 4) dpw = B / ((int64_t)256 * 4);
-  if (dpw < 1) dpw = 1;
-  if (dpw > 64) dpw = 64;
-  a.docs_per_wave = (int32_t)dpw;
-  const int64_t grid = (B + dpw - 1) / dpw;
-  if (grid > 0x7fffffff) return fail(TMS_ERR_UNSUPPORTED, "%s: too many documents", fn);
-  const int64_t per_launch = (int64_t)kResBatchedWaves * a.nblk;
-  for (int64_t b0 = 0; b0 < nblocks; b0 += per_launch) {
-    a.blk0 = (int32_t)b0;
-    a.blk_end = (int32_t)(nblocks - b0 < per_launch ? nblocks : b0 + per_launch);
+  const int64_t most = form_blocks(kBatchedForms[nf - 1], a.nbq) / a.nbq;  // queries per pass
+  for (int64_t q0 = 0; q0 < nQ; q0 += most) {
+    const int64_t q1 = q0 + most < nQ ? q0 + most : nQ;
+    int f = 0;
+    while (f < nf - 1 && form_blocks(kBatchedForms[f], a.nbq) < (q1 - q0) * a.nbq) f++;
+    a.blk0 = (int32_t)(q0 * a.nbq);
+    a.blk_end = (int32_t)(q1 * a.nbq);
+    a.nblk_l = kBatchedForms[f].NBL / a.nbq * a.nbq;
+    a.nblk_x = kBatchedForms[f].NBX / a.nbq * a.nbq;
+    const int per_cu = kBatchedForms[f].W == 8 || kBatchedForms[f].NBX > 2 ? (kBatchedForms[f].W == 8 ? 1 : 2)
+                                                                         : (kBatchedForms[f].NBX == 2 ? 3 : 4);
+    a.docs_per_wave = (int32_t)batched_docs_per_wg(B, hint, true, 256 * per_cu);
+    const int64_t grid = (B + a.docs_per_wave - 1) / a.docs_per_wave;
+    if (grid > 0x7fffffff) return fail(TMS_ERR_UNSUPPORTED, "%s: too many documents", fn);
     switch (d / 32) {
-      case 1: rc = launch_batched_ks<1>(a, nbits, nb, grid, st); break;
-      case 2: rc = launch_batched_ks<2>(a, nbits, nb, grid, st); break;
-      case 3: rc = launch_batched_ks<3>(a, nbits, nb, grid, st); break;
-      default: rc = launch_batched_ks<4>(a, nbits, nb, grid, st); break;
+      case 1: rc = launch_batched_ks<1>(a, nbits, f, grid, st); break;
+      case 2: rc = launch_batched_ks<2>(a, nbits, f, grid, st); break;
+      case 3: rc = launch_batched_ks<3>(a, nbits, f, grid, st); break;
+      default: rc = launch_batched_ks<4>(a, nbits, f, grid, st); break;
     }
     if (rc) return rc;
   }
