@@ -164,7 +164,7 @@ static int dense_entry(const char* fn, const void* Q, int64_t nQ, int64_t nq, in
     return run_stream(Q, nQ, nq, d, D, B, 0, offsets, nullptr, total_tokens, pad, dtype, out, st);
   // masked documents of up to 1,024 tokens (64 tiles, one lane each): the stream kernel walks
   // the tiles that hold a real token (2,000 x 180 tokens: 15 us against 22 for the general
-  // kernel; 20,000: 93 against 183); longer ones: the general kernel
+  // kernel; 20,000: 91 against 183); longer ones: the general kernel
   if (mode == MODE_MASKED && qreg && nd > 0 && nd <= kMaskedStreamMaxTokens)
     return run_stream(Q, nQ, nq, d, D, B, nd, nullptr, mask, 0, pad, dtype, out, st);
   if (dtype == TMS_DTYPE_F16) return run_dense<TMS_DTYPE_F16, TMS_DTYPE_F16>(a, nQ, mode, aligned, st);

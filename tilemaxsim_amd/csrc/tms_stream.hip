@@ -75,7 +75,7 @@ enum { ST_FIXED = 0, ST_VARLEN = 1, ST_MASKED = 2 };
 // of such a tile reads the tile's first real row instead (a duplicate cannot change a max):
 // masked tokens are neither fetched nor scored. A document without a real token takes R
 // tiles of row 0 whose maxima are dropped. Bound by HBM on the real tokens: 20,000 x 180
-// with a mean of 106 real tokens (0.55 GB) takes 93 us (5.9 TB/s of them), against 183 us
+// with a mean of 106 real tokens (0.55 GB) takes 91 us (6.0 TB/s of them), against 183 us
 // for the general kernel, which fetches every token and drains its loads at each tile.
 //
 // ST_VARLEN: documents at offsets (T >= 1 rows). Lane j of a wave holds its document j's first
@@ -377,6 +377,10 @@ __global__ void __launch_bounds__(256, 1) stream_maxsim_kernel(StreamArgs a) {
 #ifndef TMS_STREAM_PFD
 #define TMS_STREAM_PFD 2  // tiles in flight ahead of the one being scored (single-query path)
 #endif
+// Masked: one. A document's tiles with a real token are padded to a multiple of ahead + 1, and
+// those repeats cost more than the second load in flight gains (20,000 x 180, 106 real: 91.3
+// us a call against 93.1; 5,000, replayed: 32.9 against 34.7).
+constexpr int kMaskedPFD = 1;
 #ifndef TMS_STREAM_MIN_WAVES
 #define TMS_STREAM_MIN_WAVES (256 * 16 * 2)  // fewer documents per wave below this many waves
 #endif
@@ -387,7 +391,7 @@ __global__ void __launch_bounds__(256, 1) stream_maxsim_kernel(StreamArgs a) {
 template <int DT, int KS, int NB>
 static int stream_launch(const StreamArgs& a, int64_t grid, hipStream_t st) {
   if (a.mask)
-    hipLaunchKernelGGL((stream_maxsim_kernel<DT, KS, NB, TMS_STREAM_PFD, ST_MASKED>), dim3((unsigned)grid), dim3(256),
+    hipLaunchKernelGGL((stream_maxsim_kernel<DT, KS, NB, kMaskedPFD, ST_MASKED>), dim3((unsigned)grid), dim3(256),
                        0, st, a);
   else if (a.offsets)
     hipLaunchKernelGGL((stream_maxsim_kernel<DT, KS, NB, TMS_STREAM_PFD, ST_VARLEN>), dim3((unsigned)grid), dim3(256),
