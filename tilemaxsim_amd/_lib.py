@@ -158,6 +158,9 @@ def check_bounds(status: int, msg: str) -> None:
     check(status)
 
 
+DTYPE_CODES = {torch.float16: TMS_DTYPE_F16, torch.bfloat16: TMS_DTYPE_BF16, torch.float32: TMS_DTYPE_F32}
+
+
 def dtype_code(dt: torch.dtype) -> int:
     if dt == torch.float16:
         return TMS_DTYPE_F16
@@ -197,6 +200,16 @@ def on_device(dev: torch.device):
     if dev.index is None or dev.index == torch.cuda.current_device():
         return _CURRENT
     return torch.cuda.device(dev)
+
+
+def launch(dev: torch.device, fn, *args) -> int:
+    """``fn(*args, stream)`` on ``dev`` and torch's current stream there; its status. The
+    usual case, ``dev`` being current, costs no context."""
+    cur = torch.cuda.current_device()
+    if _raw_stream is not None and (dev.index == cur or dev.index is None):
+        return fn(*args, _raw_stream(cur))
+    with on_device(dev):
+        return fn(*args, torch.cuda.current_stream(dev).cuda_stream)
 
 
 def ptr(t: torch.Tensor | None) -> int | None:

@@ -80,12 +80,14 @@ def flash_maxsim_multi_doc(Q: torch.Tensor, D_flat: torch.Tensor, doc_offsets: t
     T, d = D_flat.shape
     Nq = Q.shape[0]
     assert Q.dim() == 2 and Q.shape[1] == d, f"flash_maxsim_multi_doc: Q width {Q.shape[1]} != D width {d}"
-    _check.embedding_dtype("D_flat", D_flat)
-    _check.contiguous("D_flat", D_flat)
-    _check.on_gpu("Q", Q)
-    _check.on_gpu("D_flat", D_flat)
-    _check.same_device(Q=Q, D_flat=D_flat)
-    Q, code = _check.query_for(Q, D_flat.dtype)
+    code = _check.plain_code(Q, D_flat)
+    if code is None:
+        _check.embedding_dtype("D_flat", D_flat)
+        _check.contiguous("D_flat", D_flat)
+        _check.on_gpu("Q", Q)
+        _check.on_gpu("D_flat", D_flat)
+        _check.same_device(Q=Q, D_flat=D_flat)
+        Q, code = _check.query_for(Q, D_flat.dtype)
     offsets = doc_offsets.to(device=Q.device, dtype=torch.int64).contiguous()
     num_docs = offsets.shape[0] - 1
     scores = torch.empty(num_docs, dtype=torch.float32, device=Q.device)
@@ -181,13 +183,15 @@ def maxsim_score(Q: torch.Tensor, D: torch.Tensor, D_mask: torch.Tensor | None =
     if tuple(D_mask.shape) != (B, Nd):
         raise ValueError(f"maxsim_score: D_mask must be (B, Nd) = {(B, Nd)}, got {tuple(D_mask.shape)}")
     assert Q.shape[1] == d, f"maxsim_score: Q width {Q.shape[1]} != D width {d}"
-    _check.embedding_dtype("D", D)
-    _check.contiguous("D", D)
-    _check.on_gpu("Q", Q)
-    _check.on_gpu("D", D)
-    _check.on_gpu("D_mask", D_mask)
-    _check.same_device(Q=Q, D=D, D_mask=D_mask)
-    Q, code = _check.query_for(Q, D.dtype)
+    code = _check.plain_code(Q, D)
+    if code is None or D_mask.device != D.device:
+        _check.embedding_dtype("D", D)
+        _check.contiguous("D", D)
+        _check.on_gpu("Q", Q)
+        _check.on_gpu("D", D)
+        _check.on_gpu("D_mask", D_mask)
+        _check.same_device(Q=Q, D=D, D_mask=D_mask)
+        Q, code = _check.query_for(Q, D.dtype)
     mask = D_mask
     if mask.dtype in (torch.bool, torch.int8):  # one byte per token: read as is (non-zero = real)
         mask = mask.view(torch.uint8)
@@ -197,8 +201,8 @@ def maxsim_score(Q: torch.Tensor, D: torch.Tensor, D_mask: torch.Tensor | None =
     scores = torch.empty(B, dtype=torch.float32, device=Q.device)
     if B == 0:
         return scores
-    lib = _lib.load()
-    with _lib.on_device(Q.device):
-        _lib.check(lib.tms_maxsim_masked(Q.data_ptr(), Q.shape[0], d, D.data_ptr(), mask.data_ptr(), B, Nd,
-                                         code, scores.data_ptr(), _lib.stream_of(Q)))
+    status = _lib.launch(D.device, _lib.load().tms_maxsim_masked, Q.data_ptr(), Q.shape[0], d, D.data_ptr(),
+                         mask.data_ptr(), B, Nd, code, scores.data_ptr())
+    if status:
+        _lib.check(status)
     return scores

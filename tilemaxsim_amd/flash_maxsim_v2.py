@@ -13,6 +13,16 @@ from . import _check, _lib
 
 
 def _dense(Q: torch.Tensor, D: torch.Tensor, fn: str) -> torch.Tensor:
+    code = _check.plain_code(Q, D)
+    if code is not None and D.dim() == 3 and Q.dim() == 2 and Q.shape[1] == D.shape[2]:
+        B, Nd, d = D.shape
+        scores = torch.empty(B, dtype=torch.float32, device=D.device)
+        if B > 0:
+            status = _lib.launch(D.device, _lib.load().tms_maxsim_dense, Q.data_ptr(), Q.shape[0], d, D.data_ptr(), B, Nd,
+                                 code, scores.data_ptr())
+            if status:
+                _lib.check(status)
+        return scores
     _check.tensor("Q", Q)
     _check.tensor("D", D)
     if D.dim() != 3:

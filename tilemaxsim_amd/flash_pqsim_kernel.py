@@ -149,17 +149,16 @@ class TileMaxSimPQ:
         if B == 0:
             return scores
         lib = _lib.load()
+        if method != "lut":
+            # the C entry point refuses shapes the MFMA kernel does not take before any
+            # device work; "auto" then scores through the table
+            status = _lib.launch(Q.device, lib.tms_pq_score, Q.data_ptr(), Nq, self.codebook.data_ptr(), self.M, self.K,
+                                 self.dsub, qcode | _CODE_FLAGS[codes.dtype], codes.data_ptr(), B, Nd, scores.data_ptr())
+            if status == _lib.TMS_OK or method == "mfma" or status != _lib.TMS_ERR_UNSUPPORTED:
+                _lib.check(status)
+                return scores
         with _lib.on_device(Q.device):
             stream = _lib.stream_of(Q)
-            if method != "lut":
-                # the C entry point refuses shapes the MFMA kernel does not take before any
-                # device work; "auto" then scores through the table
-                status = lib.tms_pq_score(Q.data_ptr(), Nq, self.codebook.data_ptr(), self.M, self.K, self.dsub,
-                                          qcode | _CODE_FLAGS[codes.dtype], codes.data_ptr(), B, Nd,
-                                          scores.data_ptr(), stream)
-                if status == _lib.TMS_OK or method == "mfma" or status != _lib.TMS_ERR_UNSUPPORTED:
-                    _lib.check(status)
-                    return scores
             table = self._table(Q, qcode)
             _lib.check(lib.tms_pq_score_lut_ex(table.data_ptr(), Nq, self.M, self.K, codes.data_ptr(),
                                                _CODE_BYTES[codes.dtype], B, Nd, scores.data_ptr(), stream))
