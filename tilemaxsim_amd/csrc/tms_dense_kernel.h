@@ -41,6 +41,11 @@
 
 namespace tms {
 
+template <bool V>
+struct Flag {
+  static constexpr bool value = V;
+};
+
 enum { MODE_FIXED = 0, MODE_VARLEN = 1, MODE_MASKED = 2 };
 
 struct DenseArgs {
@@ -58,6 +63,7 @@ struct DenseArgs {
   int32_t docs_per_wave;
   PadLen pad;              // varlen: score as if zero-padded to this many tokens (0 = off)
   int32_t mask4;           // masked: nd % 4 == 0 and a 4-byte aligned mask (word loads)
+  int32_t wpd;             // fixed: waves per document (1: each wave walks docs_per_wave whole documents)
 };
 
 // Elements 8c .. 8c+7 of row `row` (16 bytes; 32 for fp32), zero outside [0, d).
@@ -117,8 +123,12 @@ struct Cursor {
 // KS_REG == 0: Q fragments in LDS, k-groups of 4 steps (128 dims), any d.
 // KS_REG < 0: Q fragments read from memory (L2) with each tile's loads, for widths whose
 // fragments do not fit the LDS (one query block per launch).
-template <int DT, int QDT, int MODE, int NQB, int KS_REG, bool FULL, bool ALIGNED, int NSUB, int PFD, int NT>
+// SPLIT (fixed-length documents, small calls): part p of a document scores its tiles p,
+// p + wpd, ...; the parts' per-column maxima meet in LDS and part 0 sums them in the order of
+// the one-wave walk, whose bits they give.
+template <int DT, int QDT, int MODE, int NQB, int KS_REG, bool FULL, bool ALIGNED, int NSUB, int PFD, int NT, bool SPLIT>
 __global__ void __launch_bounds__(NT, 1) dense_maxsim_kernel(DenseArgs a) {
+  static_assert(!SPLIT || MODE == MODE_FIXED, "only fixed-length documents are split");
   constexpr bool QREG = KS_REG > 0;
   constexpr bool QGLB = KS_REG < 0;
   constexpr int KS = QREG ? KS_REG : 4;
@@ -252,12 +262,21 @@ __global__ void __launch_bounds__(NT, 1) dense_maxsim_kernel(DenseArgs a) {
     }
   }
 
+  const int wpd = SPLIT ? a.wpd : 1;
+  const int part = SPLIT ? wid % wpd : 0;
   const int64_t wave = (int64_t)blockIdx.x * (blockDim.x >> 6) + wid;
-  const int64_t b_begin = wave * a.docs_per_wave;
-  if (b_begin >= a.B || my_nblk <= 0) return;
-  const int64_t b_end = (b_begin + a.docs_per_wave < a.B) ? b_begin + a.docs_per_wave : a.B;
+  const int64_t b_begin = SPLIT ? (int64_t)blockIdx.x * ((NT / 64) / wpd) + wid / wpd : wave * a.docs_per_wave;
+  if (my_nblk <= 0 || (!SPLIT && b_begin >= a.B)) return;  // (parts of a document meet at a barrier)
+  const int64_t docs = SPLIT ? 1 : a.docs_per_wave;
+  const int64_t b_end = b_begin >= a.B ? b_begin : ((b_begin + docs < a.B) ? b_begin + docs : a.B);
 
   const float NEG_INF = -__builtin_inff();
+  __shared__ float red[SPLIT ? NT / 64 : 1][NQB][2][16];  // each part's per-column maxima
+  if constexpr (SPLIT) {  // a part without a tile keeps these
+    if (g == 0)
+#pragma unroll
+      for (int j = 0; j < NQB; j++) red[wid][j][0][r] = red[wid][j][1][r] = NEG_INF;
+  }
 
   // ---- per-query output ------------------------------------------------------
   // Block sums are added per query; a query whose first block precedes this wave's
@@ -331,8 +350,9 @@ __global__ void __launch_bounds__(NT, 1) dense_maxsim_kernel(DenseArgs a) {
         c.b = b;
         c.base = base;
         c.len = len;
-        c.t0 = 0;
+        c.t0 = SPLIT ? part * TT : 0;
         c.kg = 0;
+        if (SPLIT && c.t0 >= len) c.b = b_end;  // a part with no tile of the document
         return;
       }
       // an empty document zero-padded to pad_len > 0 tokens has every max equal to 0
@@ -347,7 +367,7 @@ __global__ void __launch_bounds__(NT, 1) dense_maxsim_kernel(DenseArgs a) {
       return;
     }
     c.kg = 0;
-    c.t0 += TT;
+    c.t0 += TT * wpd;
     if (c.t0 >= c.len) seek(c, c.b + 1);
   };
 
@@ -467,7 +487,9 @@ __global__ void __launch_bounds__(NT, 1) dense_maxsim_kernel(DenseArgs a) {
       for (int j = 0; j < NQB; j++) acc[sub][j][0] = acc[sub][j][1] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
 
-  auto finish_doc = [&](int64_t b, int64_t len) {
+  // COMBINE (after the parts' barrier): rmax holds part 0's maxima, already over the rows
+  auto finish = [&](int64_t b, int64_t len, auto combine) {
+    constexpr bool COMBINE = decltype(combine)::value;
     // zero padding up to pad_len adds dot products equal to 0 to a shorter document
     const bool padded = (MODE == MODE_VARLEN) && len < pad_len;
     float blk[NQB];
@@ -477,8 +499,16 @@ __global__ void __launch_bounds__(NT, 1) dense_maxsim_kernel(DenseArgs a) {
 #pragma unroll
       for (int h = 0; h < 2; h++) {
         float m = rmax[j][h];
-        m = fmaxf(m, __shfl_xor(m, 16));
-        m = fmaxf(m, __shfl_xor(m, 32));
+        if constexpr (COMBINE) {
+          for (int p = 1; p < wpd; p++) m = fmaxf(m, red[wid + p][j][h][r]);
+        } else {
+          m = fmaxf(m, __shfl_xor(m, 16));
+          m = fmaxf(m, __shfl_xor(m, 32));
+        }
+        if constexpr (SPLIT && !COMBINE) {
+          if (g == 0) red[wid][j][h][r] = m;
+          continue;
+        }
         if constexpr (QSCALE) m *= qinv[j][h];  // exact: a power of two (-inf stays -inf)
         if (padded) m = fmaxf(m, 0.f);
         bool valid;
@@ -492,8 +522,9 @@ __global__ void __launch_bounds__(NT, 1) dense_maxsim_kernel(DenseArgs a) {
       blk[j] = s;
       rmax[j][0] = rmax[j][1] = NEG_INF;
     }
-    write_doc(b, blk);
+    if (!SPLIT || COMBINE) write_doc(b, blk);
   };
+  auto finish_doc = [&](int64_t b, int64_t len) { finish(b, len, Flag<false>{}); };
 
   auto compute_tile = [&](const Buf& buf, const Cursor& c) {
     Raw lf[LINES ? NSUB : 1][LINES ? KS : 1];  // LINES: the fragments of the tile's loads
@@ -564,7 +595,7 @@ __global__ void __launch_bounds__(NT, 1) dense_maxsim_kernel(DenseArgs a) {
 #pragma unroll
           for (int h = 0; h < 2; h++) fold(rmax[j][h], acc1[sub][h], MODE == MODE_MASKED ? buf.m[sub] : 0u);
       }
-      if (c.t0 + TT >= c.len) finish_doc(c.b, c.len);
+      if (c.t0 + TT * wpd >= c.len) finish_doc(c.b, c.len);
       return;
     }
 #pragma unroll
@@ -618,13 +649,15 @@ __global__ void __launch_bounds__(NT, 1) dense_maxsim_kernel(DenseArgs a) {
             fold(rmax[j][h], acc[sub][j][h], MODE == MODE_MASKED ? buf.m[sub] : 0u);
             acc[sub][j][h] = f32x4{0.f, 0.f, 0.f, 0.f};
           }
-      if (c.t0 + TT >= c.len) finish_doc(c.b, c.len);
+      if (c.t0 + TT * wpd >= c.len) finish_doc(c.b, c.len);
     }
   };
 
   // ---- pipelined main loop -----------------------------------------------------
   // A ring of PFD + 1 tile buffers: the loads of the next PFD tiles are in flight
   // while a tile is scored. The ring is unrolled so every buffer index is static.
+  // A lambda, so that its exits still reach the parts' barrier.
+  [&]() {
   Cursor next;
   seek(next, b_begin);
   if (next.b >= b_end) return;
@@ -652,6 +685,17 @@ __global__ void __launch_bounds__(NT, 1) dense_maxsim_kernel(DenseArgs a) {
       compute_tile(ring[k], at[k]);
     }
   }
+  }();
+  if constexpr (SPLIT) {
+    __syncthreads();
+    if (part == 0 && b_begin < b_end) {
+#pragma unroll
+      for (int j = 0; j < NQB; j++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) rmax[j][h] = red[wid][j][h][r];
+      finish(b_begin, a.nd, Flag<true>{});
+    }
+  }
 }
 
 #ifndef TMS_DENSE_NSUB
@@ -669,10 +713,17 @@ constexpr int kNSub = TMS_DENSE_NSUB;
 #endif
 constexpr int kMaxQldsBytes = 64 * 1024;
 constexpr int kMaxDim = 1 << 16;  // widest embedding the dense entry points take
-constexpr size_t kStaticLds = 256;  // the kernel's static LDS (per-token query scales) beside the fragments
+constexpr size_t kStaticLds = 256;  // an unsplit launch's static LDS (per-token query scales) beside the fragments
 #ifndef TMS_DENSE_PFD
 #define TMS_DENSE_PFD 1  // tiles in flight ahead of the one being scored
 #endif
+
+// Waves a call of split documents may launch: two per SIMD, or one and a half with the query
+// in VGPRs (fp32, d <= 128). A small call is bound by each wave's walk of its tiles, a larger one
+// by the read: d = 512 fp16, 231 tokens, 100 / 500 / 1,000 documents 40 / 46 / 50 us whole,
+// 16 / 25 / 43 split, 1,500 72 / 77; fp32 d = 128, 150 tokens, 100 / 500 documents 14.2 / 16.4 us
+// whole, 7.9 / 11.2 split, 1,000 17.7 / 18.2.
+constexpr int64_t kSplitWaves = 2048, kSplitWavesReg = 1536;
 
 // LDS bytes of the query fragments of one launch (split queries: hi and lo terms).
 static inline size_t qlds_bytes(int dtype, int qdtype, int nqb, int nstep) {
@@ -708,7 +759,20 @@ static int launch_nt(const DenseArgs& a, int64_t waves, size_t lds, hipStream_t 
       return fail(TMS_ERR_UNSUPPORTED, "dense_maxsim_kernel: query fragments need %zu bytes of LDS, the device has %d",
                   lds, cap);
   }
-  hipLaunchKernelGGL((dense_maxsim_kernel<DT, QDT, MODE, NQB, KS_REG, FULL, ALIGNED, NS, TMS_DENSE_PFD, NT>),
+  if constexpr (MODE == MODE_FIXED && NT == 256 && KS_REG >= 0) {
+    // documents split over two or four waves, at most one wave per tile
+    DenseArgs s = a;
+    s.wpd = 1;
+    const int64_t tiles = (a.nd + 16 * NS - 1) / (16 * NS);
+    while (s.wpd < 4 && 2 * s.wpd <= tiles && 2 * s.wpd * a.B <= (KS_REG > 0 ? kSplitWavesReg : kSplitWaves))
+      s.wpd *= 2;
+    if (s.wpd > 1) {
+      hipLaunchKernelGGL((dense_maxsim_kernel<DT, QDT, MODE, NQB, KS_REG, FULL, ALIGNED, NS, TMS_DENSE_PFD, NT, true>),
+                         dim3((unsigned)((a.B * s.wpd + 3) / 4)), dim3(NT), lds, st, s);
+      return check_launch("dense_maxsim_kernel");
+    }
+  }
+  hipLaunchKernelGGL((dense_maxsim_kernel<DT, QDT, MODE, NQB, KS_REG, FULL, ALIGNED, NS, TMS_DENSE_PFD, NT, false>),
                      dim3((unsigned)grid), dim3(NT), lds, st, a);
   return check_launch("dense_maxsim_kernel");
 }
