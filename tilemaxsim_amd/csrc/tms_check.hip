@@ -238,6 +238,8 @@ static int wait_verdict(const char* fn, const int64_t* verdict, int parts, hipSt
     }
     const hipError_t e = hipStreamQuery(st);
     if (e == hipErrorNotReady) {
+      // no error: it must not surface in a later launch's check
+      if (hipPeekAtLastError() == hipErrorNotReady) (void)hipGetLastError();
       const timespec nap = {0, 20000};
       nanosleep(&nap, nullptr);
       continue;
