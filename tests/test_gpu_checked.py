@@ -199,3 +199,34 @@ def test_capture_is_refused(cuda):
         got = tms.flash_maxsim_multi_doc(Q, D, offsets, validate=False)
     g.replay()
     assert _same(got, want)
+
+
+def test_residual_padding_length_under_capture(cuda):
+    """Without the check nothing is waited for, and a replay finds the padding's length itself."""
+    import torch
+    import tilemaxsim_amd as tms
+    g = torch.Generator(device="cuda").manual_seed(3)
+    lens = torch.randint(1, 9, (300,), generator=g, device="cuda")
+    offsets = torch.cat([lens.new_zeros(1), lens.cumsum(0)])
+    T = int(offsets[-1])
+    cent = torch.nn.functional.normalize(torch.randn(64, 64, generator=g, device="cuda"), dim=-1).half()
+    index = (torch.randint(0, 64, (T,), generator=g, device="cuda", dtype=torch.int32),
+             torch.randint(0, 256, (T, 16), generator=g, device="cuda", dtype=torch.uint8), cent,
+             torch.tensor([-.05, -.01, .01, .05], device="cuda").half(), 2, offsets)
+    Q = torch.nn.functional.normalize(torch.randn(32, 64, generator=g, device="cuda"), dim=-1).half()
+    order = torch.argsort(lens)
+    pids = order[:100].clone()
+
+    def call():
+        return tms.flashmaxsim_score_residual(Q, *index, pids, validate=False)
+
+    call()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = call()
+    for lo in (0, 100, 200, 50):  # candidates of other longest lengths
+        pids.copy_(order[lo:lo + 100])
+        graph.replay()
+        torch.cuda.synchronize()
+        assert _same(out, call())
