@@ -759,9 +759,9 @@ class TopK:
     """Top-100 of every row of C2's score matrix (64 queries x 1M documents, MaxSim-like
     scores 10 + 0.5 N(0, 1), fp32) with tms_topk: the step the reference takes with
     torch.topk after scoring (src/cycle3_experiments.py:215). HIP events time each whole
-    call (every level of the tournament); the extra rows time other row shapes the same
+    call (the group maxima and the selection); the extra rows time other row shapes the same
     way, each checked against torch.topk on the GPU."""
-    kernel = "topk_level_kernel"
+    kernel = "topk_group_max_kernel"
     dtype = "fp32"
     SHAPES = [(32, 5_000_000, 100), (1, 1000, 100), (1, 256, 100), (1, 128, 100)]
 
