@@ -1,0 +1,54 @@
+"""CPU tests of the bounds checks' host side: where a verdict is waited for, the words it is
+written to, and which stores count as a call's own."""
+import contextlib
+
+import pytest
+import torch
+
+from tilemaxsim_amd import _lib
+from tilemaxsim_amd.flash_pqsim_kernel import TileMaxSimPQ
+
+
+def test_codes_verdict_is_waited_for_on_the_codes_device(monkeypatch):
+    """The check's launch, the scoring call and the verdict's wait all run with the codes'
+    device current: a default stream handle names the current device's stream."""
+    inside, calls = [], []
+
+    @contextlib.contextmanager
+    def on_device(dev):
+        inside.append(dev)
+        yield
+        inside.pop()
+
+    class Lib:
+        def tms_codes_check(self, *args):
+            calls.append(("check", list(inside)))
+            return _lib.TMS_OK
+
+        def tms_codes_verdict(self, verdict, stream):
+            calls.append(("verdict", list(inside)))
+            return _lib.TMS_OK
+
+    monkeypatch.setattr(_lib, "load", Lib)
+    monkeypatch.setattr(_lib, "on_device", on_device)
+    monkeypatch.setattr(_lib, "stream_of", lambda t: 0)
+    monkeypatch.setattr(_lib, "verdict_ptr", lambda: 64)
+    pq = TileMaxSimPQ.__new__(TileMaxSimPQ)
+    pq.K = 16
+    codes = torch.zeros(4, dtype=torch.int32)
+
+    def score():
+        calls.append(("score", list(inside)))
+        return "scores"
+
+    assert pq._checked(codes, score) == "scores"
+    assert calls == [(step, [codes.device]) for step in ("check", "score", "verdict")]
+    # a scoring call that raises: its verdict is still read there, and the error is passed on
+    calls.clear()
+
+    def fails():
+        raise MemoryError("no room for the scores")
+
+    with pytest.raises(MemoryError):
+        pq._checked(codes, fails)
+    assert calls == [(step, [codes.device]) for step in ("check", "verdict")] and not inside

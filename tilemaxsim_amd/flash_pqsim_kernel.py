@@ -76,16 +76,16 @@ class TileMaxSimPQ:
         """``score()``, with the codes' range checked by a kernel in front of it; only the
         check's verdict is waited for."""
         lib = _lib.load()
-        verdict, stream = _lib.verdict_ptr(), _lib.stream_of(codes)
-        with _lib.on_device(codes.device):
+        error = None
+        with _lib.on_device(codes.device):  # to the verdict's wait: a default stream is the current device's
+            verdict, stream = _lib.verdict_ptr(), _lib.stream_of(codes)
             _lib.check(lib.tms_codes_check(codes.data_ptr(), codes.numel(), _CODE_BYTES[codes.dtype], self.K, verdict,
                                            stream))
-        error = None
-        try:
-            scores = score()
-        except BaseException as e:  # the verdict's words are this call's until it is read
-            error = e
-        status = lib.tms_codes_verdict(verdict, stream)
+            try:
+                scores = score()
+            except BaseException as e:  # the verdict's words are this call's until it is read
+                error = e
+            status = lib.tms_codes_verdict(verdict, stream)
         if status == _lib.TMS_ERR_BOUNDS:
             self._refuse(codes)
         if error is not None:
