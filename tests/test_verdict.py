@@ -52,3 +52,22 @@ def test_codes_verdict_is_waited_for_on_the_codes_device(monkeypatch):
     with pytest.raises(MemoryError):
         pq._checked(codes, fails)
     assert calls == [(step, [codes.device]) for step in ("check", "verdict")] and not inside
+
+
+def test_verdict_words_do_not_follow_the_default_device(monkeypatch):
+    """The words are host memory under any default device (pinning itself needs a GPU and is
+    left out here; torch refuses to pin a tensor of another device)."""
+    zeros = torch.zeros
+
+    def host_zeros(*args, pin_memory=False, **kw):
+        words = zeros(*args, **kw)
+        assert pin_memory and words.device.type == "cpu"
+        return words
+
+    monkeypatch.setattr(torch, "zeros", host_zeros)
+    monkeypatch.delattr(_lib._thread, "verdict", raising=False)
+    try:
+        with torch.device("meta"):
+            assert _lib.verdict_ptr() != 0
+    finally:
+        vars(_lib._thread).pop("verdict", None)  # made without pinning

@@ -147,7 +147,7 @@ def verdict_ptr() -> int:
     shared; they go back to torch's pinned-memory pool when the thread ends."""
     v = getattr(_thread, "verdict", None)
     if v is None:
-        v = _thread.verdict = torch.zeros(TMS_CHECK_PARTS, dtype=torch.int64, pin_memory=True)
+        v = _thread.verdict = torch.zeros(TMS_CHECK_PARTS, dtype=torch.int64, device="cpu", pin_memory=True)
     return v.data_ptr()
 
 
