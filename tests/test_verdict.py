@@ -58,6 +58,8 @@ def test_verdict_words_do_not_follow_the_default_device(monkeypatch):
     """The words are host memory under any default device (pinning itself needs a GPU and is
     left out here; torch refuses to pin a tensor of another device)."""
     zeros = torch.zeros
+    with torch.device("meta"):
+        assert zeros(1).device.type == "meta"  # torch lists its constructors at first use, before the patch below
 
     def host_zeros(*args, pin_memory=False, **kw):
         words = zeros(*args, **kw)
