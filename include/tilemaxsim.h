@@ -310,8 +310,8 @@ int tms_maxsim_residual_batched(const void* Qs, int64_t nQ, int64_t nq, int64_t 
  * [0, ndocs); the scores of such a call are not to be used. zero_pad != 0 scores as if
  * zero-padded to the longest scored document, whose length the check finds. B >= 1.
  *   parts    device memory, TMS_CHECK_PARTS int64, any content; may be NULL without zero_pad
- *   verdict  pinned host memory (hipHostMalloc), TMS_CHECK_PARTS int64, used by one call at a
- *            time; NULL: nothing is waited for or refused (invalid documents score NaN). With
+ *   verdict  pinned host memory (hipHostMalloc), TMS_CHECK_PARTS int64, zeroed once and then
+ *            left to these calls, one at a time; NULL: nothing is waited for or refused (invalid documents score NaN). With
  *            a verdict the stream must not be under capture (TMS_ERR_HIP).
  * tms_maxsim_packed_checked takes lengths (1 <= B <= TMS_PACKED_SCAN_MAX) and writes their
  * offsets (B + 1). tms_maxsim_residual_checked scores as tms_maxsim_residual (nQ = 1), or as

@@ -1,12 +1,30 @@
 """CPU tests of the bounds checks' host side: where a verdict is waited for, the words it is
 written to, and which stores count as a call's own."""
 import contextlib
+import os
+import shutil
+import subprocess
 
 import pytest
 import torch
 
 from tilemaxsim_amd import _lib
 from tilemaxsim_amd.flash_pqsim_kernel import TileMaxSimPQ
+
+REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+def test_words_of_an_earlier_check_are_not_taken_for_this_one(tmp_path):
+    """tests/verdict_words.cpp against the polling code that the library uses."""
+    gxx = shutil.which("g++")
+    if gxx is None:
+        pytest.skip("g++ not available")
+    exe = str(tmp_path / "verdict_words")
+    build = subprocess.run([gxx, "-std=c++17", "-O1", "-Wall", "-Werror", "-I", os.path.join(REPO, "tilemaxsim_amd", "csrc"),
+                            os.path.join(REPO, "tests", "verdict_words.cpp"), "-o", exe], capture_output=True, text=True)
+    assert build.returncode == 0, build.stderr
+    run = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert run.returncode == 0 and run.stdout == "ok\n", (run.returncode, run.stdout, run.stderr)
 
 
 def test_codes_verdict_is_waited_for_on_the_codes_device(monkeypatch):

@@ -143,8 +143,8 @@ _thread = threading.local()
 
 def verdict_ptr() -> int:
     """Address of the calling thread's verdict words (pinned host memory). A ``*_checked``
-    call waits for its own verdicts before it returns, so a thread's words are never
-    shared; they go back to torch's pinned-memory pool when the thread ends."""
+    call reads its own verdicts, or lets its stream drain, before it returns; they go back to
+    torch's pinned-memory pool when the thread ends."""
     v = getattr(_thread, "verdict", None)
     if v is None:
         v = _thread.verdict = torch.zeros(TMS_CHECK_PARTS, dtype=torch.int64, device="cpu", pin_memory=True)

@@ -7,7 +7,10 @@
 // against 79, from a residual index of 100,000 documents 24 against 157.
 #include <time.h>
 
+#include <atomic>
+
 #include "tms_check.h"
+#include "tms_verdict.h"
 
 namespace tms {
 
@@ -26,8 +29,12 @@ __device__ __forceinline__ int64_t wave_max64(int64_t m) {
 }
 
 // The workgroup's maximum length and verdict: parts[blockIdx.x] (when given) for the scoring
-// kernel, and 1 (fine) or 2 into verdict[blockIdx.x], host memory, which the host waits for.
-__device__ __forceinline__ void publish(int64_t mx, bool bad, int64_t* parts, int64_t* verdict) {
+// kernel, and the outcome with the check's tag into verdict[blockIdx.x], host memory, which the
+// host waits for.
+__device__ __forceinline__ void store_verdict(int64_t* word, int64_t tag, bool bad) {
+  __hip_atomic_store(word, tag | (bad ? kVerdictBad : kVerdictFine), __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__device__ __forceinline__ void publish(int64_t mx, bool bad, int64_t* parts, int64_t* verdict, int64_t tag) {
   __shared__ int64_t wmax[kCheckWaves];
   __shared__ uint32_t wbad[kCheckWaves];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -43,9 +50,7 @@ __device__ __forceinline__ void publish(int64_t mx, bool bad, int64_t* parts, in
   const uint64_t all = __ballot(lane < kCheckWaves && wbad[lane] != 0u);
   if (lane == 0) {
     if (parts) parts[blockIdx.x] = mx;
-    if (verdict)
-      __hip_atomic_store(verdict + blockIdx.x, all != 0 ? (int64_t)2 : (int64_t)1, __ATOMIC_RELEASE,
-                         __HIP_MEMORY_SCOPE_SYSTEM);
+    if (verdict) store_verdict(verdict + blockIdx.x, tag, all != 0);
   }
 }
 
@@ -54,7 +59,8 @@ __device__ __forceinline__ void publish(int64_t mx, bool bad, int64_t* parts, in
 // (2M documents), by launch and one memory round trip at a few thousand.
 __global__ void __launch_bounds__(kCheckThreads) docs_check_kernel(const int64_t* __restrict__ offsets, int64_t ndocs,
                                                                    const int64_t* __restrict__ pids, int64_t B,
-                                                                   int64_t T, int64_t* parts, int64_t* verdict) {
+                                                                   int64_t T, int64_t* parts, int64_t* verdict,
+                                                                   int64_t tag) {
   const int64_t first = (int64_t)blockIdx.x * kCheckThreads + threadIdx.x;
   const int64_t stride = (int64_t)gridDim.x * kCheckThreads;
   bool bad = false;
@@ -78,14 +84,14 @@ __global__ void __launch_bounds__(kCheckThreads) docs_check_kernel(const int64_t
       }
     }
   }
-  publish(mx, bad, parts, verdict);
+  publish(mx, bad, parts, verdict, tag);
 }
 
 // Lengths to offsets (B + 1) in one workgroup, with the checks of docs_check_kernel: each
 // wave scans its 64 lengths of every 1,024, then the waves' sums are scanned.
 __global__ void __launch_bounds__(kCheckThreads) lengths_scan_kernel(const int64_t* __restrict__ lengths, int64_t B,
                                                                      int64_t T, int64_t* __restrict__ offsets,
-                                                                     int64_t* parts, int64_t* verdict) {
+                                                                     int64_t* parts, int64_t* verdict, int64_t tag) {
   __shared__ int64_t sums[kScanTiles * kCheckWaves];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   int64_t len[kScanTiles], incl[kScanTiles];
@@ -143,7 +149,7 @@ __global__ void __launch_bounds__(kCheckThreads) lengths_scan_kernel(const int64
       bad |= e < (int64_t)((uint64_t)e - (uint64_t)len[t]) || (i == B - 1 && e > T);
     }
   }
-  publish(mx, bad, parts, verdict);
+  publish(mx, bad, parts, verdict, tag);
 }
 
 // Codes below K: every code as unsigned, compared with `limit` (K, or 2^(bits - 1) for signed
@@ -172,7 +178,8 @@ __device__ __forceinline__ bool codes_over(const u32x4& x, uint32_t limit) {
 }
 template <int CB>
 __global__ void __launch_bounds__(kCheckThreads) codes_check_kernel(const uint8_t* __restrict__ codes, int64_t count,
-                                                                    uint32_t limit, bool marked, int64_t* verdict) {
+                                                                    uint32_t limit, bool marked, int64_t* verdict,
+                                                                    int64_t tag) {
   const int64_t bytes = count * CB;
   int64_t head = (int64_t)((16u - ((uintptr_t)codes & 15u)) & 15u);
   if (head > bytes) head = bytes;
@@ -203,15 +210,13 @@ __global__ void __launch_bounds__(kCheckThreads) codes_check_kernel(const uint8_
     }
   }
   if (!marked) {
-    publish(0, bad, nullptr, verdict);
+    publish(0, bad, nullptr, verdict, tag);
   } else if (__ballot(bad) != 0ull && (threadIdx.x & 63) == 0) {
-    __hip_atomic_store(verdict + 1, (int64_t)2, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    store_verdict(verdict + 1, tag, true);
   }
 }
 // After a grid of more workgroups than there are verdict words: the words it wrote are final.
-__global__ void check_done_kernel(int64_t* verdict) {
-  __hip_atomic_store(verdict, (int64_t)1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-}
+__global__ void check_done_kernel(int64_t* verdict, int64_t tag) { store_verdict(verdict, tag, false); }
 
 static int check_parts(int64_t items) {
   const int64_t g = (items + kCheckItems - 1) / kCheckItems;
@@ -221,57 +226,59 @@ static int check_parts(int64_t items) {
 // Waits until the check's workgroups have written their verdicts: a spin on host memory,
 // which sees them a microsecond or two after the kernel's stores, then short sleeps. Ends
 // also when the stream has drained or failed without them.
-static int wait_verdict(const char* fn, const int64_t* verdict, int parts, hipStream_t st) {
-  bool bad = false;
-  int seen = 0;
-  for (int64_t spin = 0;; spin++) {
-    while (seen < parts) {
-      const int64_t v = __atomic_load_n(verdict + seen, __ATOMIC_ACQUIRE);
-      if (v == 0) break;
-      bad |= v == 2;
-      seen++;
-    }
-    if (seen == parts) return bad ? TMS_ERR_BOUNDS : TMS_OK;
-    if (spin < 20000) {
-      __builtin_ia32_pause();
-      continue;
-    }
-    const hipError_t e = hipStreamQuery(st);
-    if (e == hipErrorNotReady) {
-      // no error: it must not surface in a later launch's check
-      if (hipPeekAtLastError() == hipErrorNotReady) (void)hipGetLastError();
-      const timespec nap = {0, 20000};
-      nanosleep(&nap, nullptr);
-      continue;
-    }
-    while (seen < parts && __atomic_load_n(verdict + seen, __ATOMIC_ACQUIRE) != 0) {
-      bad |= __atomic_load_n(verdict + seen, __ATOMIC_ACQUIRE) == 2;
-      seen++;
-    }
-    if (e == hipSuccess && seen == parts) return bad ? TMS_ERR_BOUNDS : TMS_OK;
-    return fail(TMS_ERR_HIP, "%s: the bounds check did not finish: %s", fn, hipGetErrorString(e));
-  }
+static int wait_verdict(const char* fn, const int64_t* verdict, int64_t tag, int parts, hipStream_t st) {
+  VerdictPoll poll{verdict, parts, tag};
+  hipError_t e = hipSuccess;
+  const VerdictState s = await_verdict(
+      poll, 20000,
+      [&]() {
+        e = hipStreamQuery(st);
+        // neither outcome may surface in a later launch's check: not ready is no error, and a
+        // failure is reported here
+        if (e != hipSuccess && hipPeekAtLastError() == e) (void)hipGetLastError();
+        return e == hipErrorNotReady ? STREAM_BUSY : (e == hipSuccess ? STREAM_DRAINED : STREAM_FAILED);
+      },
+      []() {
+        const timespec nap = {0, 20000};
+        nanosleep(&nap, nullptr);
+      });
+  if (s != VERDICT_PENDING) return s == VERDICT_BAD ? TMS_ERR_BOUNDS : TMS_OK;
+  if (e != hipSuccess) (void)hipStreamSynchronize(st);  // the words may go back to their pool after this call
+  return fail(TMS_ERR_HIP, "%s: the bounds check did not finish: %s", fn, hipGetErrorString(e));
 }
 
-// Refuses a stream under capture (the host cannot wait for a verdict there) and clears the
-// verdicts. The buffers are the calling thread's: every call waits for its own verdicts
-// before it returns, so no kernel writes them later.
-static int open_verdict(const char* fn, int64_t* verdict, hipStream_t st) {
+// Refuses a stream under capture (the host cannot wait for a verdict there) and gives the
+// check its tag.
+static int open_verdict(const char* fn, const int64_t* verdict, hipStream_t st, int64_t& tag) {
+  static std::atomic<int64_t> sequence{0};
+  tag = 0;
   if (!verdict) return TMS_OK;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   const hipError_t e = hipStreamIsCapturing(st, &cap);
-  if (e != hipSuccess || cap != hipStreamCaptureStatusNone)
+  if (e != hipSuccess) {
+    if (hipPeekAtLastError() == e) (void)hipGetLastError();  // reported here, not by a later launch's check
+    return fail(TMS_ERR_HIP, "%s: whether the stream is under capture: %s", fn, hipGetErrorString(e));
+  }
+  if (cap != hipStreamCaptureStatusNone)
     return fail(TMS_ERR_HIP, "%s: the bounds check waits for the GPU and cannot run under stream capture", fn);
-  for (int i = 0; i < TMS_CHECK_PARTS; i++) __atomic_store_n(verdict + i, (int64_t)0, __ATOMIC_RELEASE);
+  tag = verdict_tag(sequence.fetch_add(1, std::memory_order_relaxed) + 1);
   return TMS_OK;
 }
 
+// The launch check of a check kernel. The error it finds may be an older call's and the kernel
+// be on its way: its stores are let land before the caller has the words back.
+static int check_launched(const char* what, const int64_t* verdict, hipStream_t st) {
+  const int rc = check_launch(what);
+  if (rc && verdict) (void)hipStreamSynchronize(st);
+  return rc;
+}
+
 // The check's outcome first (as when it ran before the scoring call), then the scoring's.
-static int close_verdict(const char* fn, const int64_t* verdict, int parts, hipStream_t st, int scored) {
+static int close_verdict(const char* fn, const int64_t* verdict, int64_t tag, int parts, hipStream_t st, int scored) {
   if (!verdict) return scored;
   char why[512];
   keep_error(why, sizeof(why));
-  const int rc = wait_verdict(fn, verdict, parts, st);
+  const int rc = wait_verdict(fn, verdict, tag, parts, st);
   if (rc == TMS_ERR_BOUNDS) return fail(rc, "%s: document bounds or ids out of range", fn);
   if (rc) return rc;
   if (scored) set_error("%s", why);
@@ -291,16 +298,17 @@ int tms_maxsim_varlen_checked(const void* Qs, int64_t nQ, int64_t nq, int64_t d,
   if (B < 1 || !offsets) return fail(TMS_ERR_INVALID, "%s: at least one document and its offsets", fn);
   if (zero_pad && !parts) return fail(TMS_ERR_INVALID, "%s: parts is NULL", fn);
   hipStream_t st = (hipStream_t)stream;
-  int rc = open_verdict(fn, verdict, st);
+  int64_t tag;
+  int rc = open_verdict(fn, verdict, st, tag);
   if (rc) return rc;
   const int g = check_parts(B);
   hipLaunchKernelGGL(docs_check_kernel, dim3(g), dim3(kCheckThreads), 0, st, offsets, B, nullptr, B, total_tokens,
-                     zero_pad ? parts : nullptr, verdict);
-  rc = check_launch("docs_check_kernel");
+                     zero_pad ? parts : nullptr, verdict, tag);
+  rc = check_launched("docs_check_kernel", verdict, st);
   if (rc) return rc;
   rc = varlen_scores(fn, Qs, nQ, nq, d, D_flat, total_tokens, offsets, B, zero_pad ? PadLen{0, parts, g} : PadLen{0, nullptr, 0},
                      dtype, out, stream);
-  return close_verdict(fn, verdict, g, st, rc);
+  return close_verdict(fn, verdict, tag, g, st, rc);
 }
 
 int tms_maxsim_packed_checked(const void* Q, int64_t nq, int64_t d, const void* D_packed, int64_t total_tokens,
@@ -311,15 +319,16 @@ int tms_maxsim_packed_checked(const void* Q, int64_t nq, int64_t d, const void* 
   if (B > TMS_PACKED_SCAN_MAX) return fail(TMS_ERR_UNSUPPORTED, "%s: more than %d documents", fn, TMS_PACKED_SCAN_MAX);
   if (zero_pad && !parts) return fail(TMS_ERR_INVALID, "%s: parts is NULL", fn);
   hipStream_t st = (hipStream_t)stream;
-  int rc = open_verdict(fn, verdict, st);
+  int64_t tag;
+  int rc = open_verdict(fn, verdict, st, tag);
   if (rc) return rc;
   hipLaunchKernelGGL(lengths_scan_kernel, dim3(1), dim3(kCheckThreads), 0, st, lengths, B, total_tokens, offsets,
-                     zero_pad ? parts : nullptr, verdict);
-  rc = check_launch("lengths_scan_kernel");
+                     zero_pad ? parts : nullptr, verdict, tag);
+  rc = check_launched("lengths_scan_kernel", verdict, st);
   if (rc) return rc;
   rc = varlen_scores(fn, Q, 1, nq, d, D_packed, total_tokens, offsets, B, zero_pad ? PadLen{0, parts, 1} : PadLen{0, nullptr, 0},
                      dtype, out, stream);
-  return close_verdict(fn, verdict, 1, st, rc);
+  return close_verdict(fn, verdict, tag, 1, st, rc);
 }
 
 int tms_maxsim_residual_checked(const void* Qs, int64_t nQ, int64_t nq, int64_t d, const void* centroids,
@@ -333,20 +342,21 @@ int tms_maxsim_residual_checked(const void* Qs, int64_t nQ, int64_t nq, int64_t 
                                       (long long)ndocs);
   if (zero_pad && !parts) return fail(TMS_ERR_INVALID, "%s: parts is NULL", fn);
   hipStream_t st = (hipStream_t)stream;
-  int rc = open_verdict(fn, verdict, st);
+  int64_t tag;
+  int rc = open_verdict(fn, verdict, st, tag);
   if (rc) return rc;
   const int g = check_parts(ndocs > B ? ndocs : B);
   hipLaunchKernelGGL(docs_check_kernel, dim3(g), dim3(kCheckThreads), 0, st, offsets, ndocs, pids, B, total_tokens,
-                     zero_pad ? parts : nullptr, verdict);
-  rc = check_launch("docs_check_kernel");
+                     zero_pad ? parts : nullptr, verdict, tag);
+  rc = check_launched("docs_check_kernel", verdict, st);
   if (rc) return rc;
   rc = residual_scores(fn, Qs, nQ, nq, d, centroids, ncent, bucket_weights, nbits, codes, residuals, total_tokens, offsets,
                        ndocs, pids, B, zero_pad ? PadLen{0, parts, g} : PadLen{0, nullptr, 0}, batched != 0, out, stream);
-  return close_verdict(fn, verdict, g, st, rc);
+  return close_verdict(fn, verdict, tag, g, st, rc);
 }
 
-// verdict[TMS_CHECK_PARTS - 1] is the host's: the words to wait for, or 0 for a marked grid
-// (word 0 says that it is done, word 1 that a code was out of range).
+// verdict[TMS_CHECK_PARTS - 1] is the host's: the check's tag with the words to wait for, 0 of
+// them for a marked grid (word 0 says that it is done, word 1 that a code was out of range).
 int tms_codes_check(const void* codes, int64_t count, int code_bytes, int64_t K, int64_t* verdict, void* stream) {
   const char* fn = "tms_codes_check";
   if (count < 1 || K < 0 || !codes || !verdict) return fail(TMS_ERR_INVALID, "%s: bad size or NULL pointer", fn);
@@ -354,12 +364,13 @@ int tms_codes_check(const void* codes, int64_t count, int code_bytes, int64_t K,
     return fail(TMS_ERR_INVALID, "%s: code_bytes must be 1, 2 or 4, got %d", fn, code_bytes);
   if ((uintptr_t)codes % code_bytes) return fail(TMS_ERR_INVALID, "%s: misaligned codes", fn);
   hipStream_t st = (hipStream_t)stream;
-  const int rc = open_verdict(fn, verdict, st);
+  int64_t tag;
+  int rc = open_verdict(fn, verdict, st, tag);
   if (rc) return rc;
   const int64_t top = code_bytes == 1 ? 256 : (code_bytes == 2 ? 32768 : (int64_t)1 << 31);
-  verdict[TMS_CHECK_PARTS - 1] = 1;
+  verdict[TMS_CHECK_PARTS - 1] = tag | 1;
   if (K >= top && code_bytes == 1) {  // every byte is a code
-    verdict[0] = 1;
+    verdict[0] = tag | kVerdictFine;
     return TMS_OK;
   }
   const uint32_t limit = (uint32_t)(K < top ? K : top);
@@ -368,24 +379,26 @@ int tms_codes_check(const void* codes, int64_t count, int code_bytes, int64_t K,
   const bool marked = bytes > ((int64_t)32 << 20);
   const int64_t most = marked ? 512 : TMS_CHECK_PARTS - 1;
   const int g = (int)(want < most ? want : most);
-  verdict[TMS_CHECK_PARTS - 1] = marked ? 0 : g;
+  verdict[TMS_CHECK_PARTS - 1] = tag | (marked ? 0 : g);
   const uint8_t* p = (const uint8_t*)codes;
   if (code_bytes == 1)
-    hipLaunchKernelGGL(codes_check_kernel<1>, dim3(g), dim3(kCheckThreads), 0, st, p, count, limit, marked, verdict);
+    hipLaunchKernelGGL(codes_check_kernel<1>, dim3(g), dim3(kCheckThreads), 0, st, p, count, limit, marked, verdict, tag);
   else if (code_bytes == 2)
-    hipLaunchKernelGGL(codes_check_kernel<2>, dim3(g), dim3(kCheckThreads), 0, st, p, count, limit, marked, verdict);
+    hipLaunchKernelGGL(codes_check_kernel<2>, dim3(g), dim3(kCheckThreads), 0, st, p, count, limit, marked, verdict, tag);
   else
-    hipLaunchKernelGGL(codes_check_kernel<4>, dim3(g), dim3(kCheckThreads), 0, st, p, count, limit, marked, verdict);
-  if (marked) hipLaunchKernelGGL(check_done_kernel, dim3(1), dim3(1), 0, st, verdict);
-  return check_launch("codes_check_kernel");
+    hipLaunchKernelGGL(codes_check_kernel<4>, dim3(g), dim3(kCheckThreads), 0, st, p, count, limit, marked, verdict, tag);
+  if (marked) hipLaunchKernelGGL(check_done_kernel, dim3(1), dim3(1), 0, st, verdict, tag);
+  return check_launched("codes_check_kernel", verdict, st);
 }
 
 int tms_codes_verdict(const int64_t* verdict, void* stream) {
   const char* fn = "tms_codes_verdict";
   if (!verdict) return fail(TMS_ERR_INVALID, "%s: NULL pointer", fn);
-  const int parts = (int)verdict[TMS_CHECK_PARTS - 1];
-  int rc = wait_verdict(fn, verdict, parts > 0 ? parts : 1, (hipStream_t)stream);
-  if (rc == TMS_OK && parts == 0 && __atomic_load_n(verdict + 1, __ATOMIC_ACQUIRE) != 0) rc = TMS_ERR_BOUNDS;
+  const int64_t mark = verdict[TMS_CHECK_PARTS - 1], tag = mark & ~(int64_t)0xff;
+  const int parts = (int)(mark & 0xff);
+  int rc = wait_verdict(fn, verdict, tag, parts > 0 ? parts : 1, (hipStream_t)stream);
+  if (rc == TMS_OK && parts == 0 && __atomic_load_n(verdict + 1, __ATOMIC_ACQUIRE) == (tag | kVerdictBad))
+    rc = TMS_ERR_BOUNDS;
   return rc == TMS_ERR_BOUNDS ? fail(rc, "%s: codes out of range", fn) : rc;
 }
 
