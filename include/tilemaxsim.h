@@ -309,7 +309,9 @@ int tms_maxsim_residual_batched(const void* Qs, int64_t nQ, int64_t nq, int64_t 
  * returns TMS_ERR_BOUNDS when offsets decrease or leave [0, total_tokens], or a pid leaves
  * [0, ndocs); the scores of such a call are not to be used. zero_pad != 0 scores as if
  * zero-padded to the longest scored document, whose length the check finds. B >= 1.
- *   parts    device memory, TMS_CHECK_PARTS int64, any content; may be NULL without zero_pad
+ *   parts    device memory, TMS_CHECK_PARTS int64, any content: what the check tells the
+ *            scoring kernels, which leave a refused call unscored (NaN). May be NULL without
+ *            zero_pad; a verdict is then waited for before the scoring starts
  *   verdict  pinned host memory (hipHostMalloc), TMS_CHECK_PARTS int64, zeroed once and then
  *            left to these calls, one at a time; NULL: nothing is waited for or refused (invalid documents score NaN). With
  *            a verdict the stream must not be under capture (TMS_ERR_HIP).

@@ -193,6 +193,7 @@ __device__ __forceinline__ void batched_body(const BatchedArgs& a, BatchedRing<S
     }
 
   // lane j holds document b_begin + j's first row and length (-1: invalid offsets)
+  const int64_t pad = pad_part(a.pad, lane);
   int64_t dbase = 0;
   int32_t dlen = -1;
   if (lane < ndocs) {
@@ -203,7 +204,8 @@ __device__ __forceinline__ void batched_body(const BatchedArgs& a, BatchedRing<S
       dlen = (int32_t)(e0 - s0);
     }
   }
-  const int64_t pad_len = pad_length(a.pad, lane);
+  if (refused(pad)) dlen = -1;
+  const int64_t pad_len = pad_length(a.pad, pad);
   float pend[NB];  // lane j: scores of document b_begin + j
 #pragma unroll
   for (int j = 0; j < NB; j++) pend[j] = NEG_INF;

@@ -2,7 +2,7 @@
 // return the verdict: one small kernel before the scoring kernel on the same stream, in
 // place of a chain of elementwise passes and host copies. The check also leaves the longest
 // scored document's length on the device, where the scoring kernel reads it (the
-// zero-padding semantics need it), so the host waits only for the check's verdict while the
+// zero-padding semantics need it), and there too whether the call is refused, so the host waits only for the check's verdict while the
 // scoring kernel runs: PLAID's last stage over 1,024 packed documents takes 20 us a call
 // against 79, from a residual index of 100,000 documents 24 against 157.
 #include <time.h>
@@ -29,7 +29,7 @@ __device__ __forceinline__ int64_t wave_max64(int64_t m) {
 }
 
 // The workgroup's maximum length and verdict: parts[blockIdx.x] (when given) for the scoring
-// kernel, and the outcome with the check's tag into verdict[blockIdx.x], host memory, which the
+// kernel, -1 there if the call is refused (it has a verdict, and it is bad), and the outcome with the check's tag into verdict[blockIdx.x], host memory, which the
 // host waits for.
 __device__ __forceinline__ void store_verdict(int64_t* word, int64_t tag, bool bad) {
   __hip_atomic_store(word, tag | (bad ? kVerdictBad : kVerdictFine), __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -49,7 +49,7 @@ __device__ __forceinline__ void publish(int64_t mx, bool bad, int64_t* parts, in
   mx = wave_max64(lane < kCheckWaves ? wmax[lane] : 0);
   const uint64_t all = __ballot(lane < kCheckWaves && wbad[lane] != 0u);
   if (lane == 0) {
-    if (parts) parts[blockIdx.x] = mx;
+    if (parts) parts[blockIdx.x] = verdict && all != 0 ? -1 : mx;
     if (verdict) store_verdict(verdict + blockIdx.x, tag, all != 0);
   }
 }
@@ -59,8 +59,8 @@ __device__ __forceinline__ void publish(int64_t mx, bool bad, int64_t* parts, in
 // (2M documents), by launch and one memory round trip at a few thousand.
 __global__ void __launch_bounds__(kCheckThreads) docs_check_kernel(const int64_t* __restrict__ offsets, int64_t ndocs,
                                                                    const int64_t* __restrict__ pids, int64_t B,
-                                                                   int64_t T, int64_t* parts, int64_t* verdict,
-                                                                   int64_t tag) {
+                                                                   int64_t T, bool longest, int64_t* parts,
+                                                                   int64_t* verdict, int64_t tag) {
   const int64_t first = (int64_t)blockIdx.x * kCheckThreads + threadIdx.x;
   const int64_t stride = (int64_t)gridDim.x * kCheckThreads;
   bool bad = false;
@@ -84,14 +84,15 @@ __global__ void __launch_bounds__(kCheckThreads) docs_check_kernel(const int64_t
       }
     }
   }
-  publish(mx, bad, parts, verdict, tag);
+  publish(longest ? mx : 0, bad, parts, verdict, tag);
 }
 
 // Lengths to offsets (B + 1) in one workgroup, with the checks of docs_check_kernel: each
 // wave scans its 64 lengths of every 1,024, then the waves' sums are scanned.
 __global__ void __launch_bounds__(kCheckThreads) lengths_scan_kernel(const int64_t* __restrict__ lengths, int64_t B,
                                                                      int64_t T, int64_t* __restrict__ offsets,
-                                                                     int64_t* parts, int64_t* verdict, int64_t tag) {
+                                                                     bool longest, int64_t* parts, int64_t* verdict,
+                                                                     int64_t tag) {
   __shared__ int64_t sums[kScanTiles * kCheckWaves];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   int64_t len[kScanTiles], incl[kScanTiles];
@@ -149,7 +150,7 @@ __global__ void __launch_bounds__(kCheckThreads) lengths_scan_kernel(const int64
       bad |= e < (int64_t)((uint64_t)e - (uint64_t)len[t]) || (i == B - 1 && e > T);
     }
   }
-  publish(mx, bad, parts, verdict, tag);
+  publish(longest ? mx : 0, bad, parts, verdict, tag);
 }
 
 // Codes below K: every code as unsigned, compared with `limit` (K, or 2^(bits - 1) for signed
@@ -273,14 +274,17 @@ static int check_launched(const char* what, const int64_t* verdict, hipStream_t 
   return rc;
 }
 
+static int refuse(const char* fn, int rc) {
+  return rc == TMS_ERR_BOUNDS ? fail(rc, "%s: document bounds or ids out of range", fn) : rc;
+}
+
 // The check's outcome first (as when it ran before the scoring call), then the scoring's.
 static int close_verdict(const char* fn, const int64_t* verdict, int64_t tag, int parts, hipStream_t st, int scored) {
   if (!verdict) return scored;
   char why[512];
   keep_error(why, sizeof(why));
   const int rc = wait_verdict(fn, verdict, tag, parts, st);
-  if (rc == TMS_ERR_BOUNDS) return fail(rc, "%s: document bounds or ids out of range", fn);
-  if (rc) return rc;
+  if (rc) return refuse(fn, rc);
   if (scored) set_error("%s", why);
   return scored;
 }
@@ -303,11 +307,11 @@ int tms_maxsim_varlen_checked(const void* Qs, int64_t nQ, int64_t nq, int64_t d,
   if (rc) return rc;
   const int g = check_parts(B);
   hipLaunchKernelGGL(docs_check_kernel, dim3(g), dim3(kCheckThreads), 0, st, offsets, B, nullptr, B, total_tokens,
-                     zero_pad ? parts : nullptr, verdict, tag);
+                     zero_pad != 0, parts, verdict, tag);
   rc = check_launched("docs_check_kernel", verdict, st);
   if (rc) return rc;
-  rc = varlen_scores(fn, Qs, nQ, nq, d, D_flat, total_tokens, offsets, B, zero_pad ? PadLen{0, parts, g} : PadLen{0, nullptr, 0},
-                     dtype, out, stream);
+  if (verdict && !parts && (rc = wait_verdict(fn, verdict, tag, g, st))) return refuse(fn, rc);
+  rc = varlen_scores(fn, Qs, nQ, nq, d, D_flat, total_tokens, offsets, B, PadLen{0, parts, g}, dtype, out, stream);
   return close_verdict(fn, verdict, tag, g, st, rc);
 }
 
@@ -323,11 +327,11 @@ int tms_maxsim_packed_checked(const void* Q, int64_t nq, int64_t d, const void* 
   int rc = open_verdict(fn, verdict, st, tag);
   if (rc) return rc;
   hipLaunchKernelGGL(lengths_scan_kernel, dim3(1), dim3(kCheckThreads), 0, st, lengths, B, total_tokens, offsets,
-                     zero_pad ? parts : nullptr, verdict, tag);
+                     zero_pad != 0, parts, verdict, tag);
   rc = check_launched("lengths_scan_kernel", verdict, st);
   if (rc) return rc;
-  rc = varlen_scores(fn, Q, 1, nq, d, D_packed, total_tokens, offsets, B, zero_pad ? PadLen{0, parts, 1} : PadLen{0, nullptr, 0},
-                     dtype, out, stream);
+  if (verdict && !parts && (rc = wait_verdict(fn, verdict, tag, 1, st))) return refuse(fn, rc);
+  rc = varlen_scores(fn, Q, 1, nq, d, D_packed, total_tokens, offsets, B, PadLen{0, parts, 1}, dtype, out, stream);
   return close_verdict(fn, verdict, tag, 1, st, rc);
 }
 
@@ -347,11 +351,12 @@ int tms_maxsim_residual_checked(const void* Qs, int64_t nQ, int64_t nq, int64_t 
   if (rc) return rc;
   const int g = check_parts(ndocs > B ? ndocs : B);
   hipLaunchKernelGGL(docs_check_kernel, dim3(g), dim3(kCheckThreads), 0, st, offsets, ndocs, pids, B, total_tokens,
-                     zero_pad ? parts : nullptr, verdict, tag);
+                     zero_pad != 0, parts, verdict, tag);
   rc = check_launched("docs_check_kernel", verdict, st);
   if (rc) return rc;
+  if (verdict && !parts && (rc = wait_verdict(fn, verdict, tag, g, st))) return refuse(fn, rc);
   rc = residual_scores(fn, Qs, nQ, nq, d, centroids, ncent, bucket_weights, nbits, codes, residuals, total_tokens, offsets,
-                       ndocs, pids, B, zero_pad ? PadLen{0, parts, g} : PadLen{0, nullptr, 0}, batched != 0, out, stream);
+                       ndocs, pids, B, PadLen{0, parts, g}, batched != 0, out, stream);
   return close_verdict(fn, verdict, tag, g, st, rc);
 }
 

@@ -263,15 +263,21 @@ struct DocEnd {
 };
 
 // The zero-padding length of a call (0: none): a number, or the largest of up to 64 numbers
-// that an earlier kernel on the stream left in device memory.
+// that a check kernel earlier on the stream left in device memory, one a workgroup; a negative
+// one says that the call is refused.
 struct PadLen {
   int64_t len;
   const int64_t* parts;
   int32_t nparts;
 };
-__device__ __forceinline__ int64_t pad_length(const PadLen& p, int lane) {
+// A lane's one of the numbers: read ahead of a wave's other first loads and used by the two
+// functions below after them, so that the wave waits for memory once.
+__device__ __forceinline__ int64_t pad_part(const PadLen& p, int lane) {
+  return p.parts != nullptr && lane < p.nparts ? p.parts[lane] : 0;
+}
+__device__ __forceinline__ int64_t pad_length(const PadLen& p, int64_t part) {
   if (p.parts == nullptr) return p.len;  // uniform
-  int64_t m = lane < p.nparts ? p.parts[lane] : 0;
+  int64_t m = part;
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) {
     const int64_t x = __shfl_xor(m, o);
@@ -279,6 +285,10 @@ __device__ __forceinline__ int64_t pad_length(const PadLen& p, int lane) {
   }
   return wave_uniform(m);
 }
+// Whether the check in front of this kernel refused the call. Its documents are then all taken
+// as invalid: one at a time they may be in range and still far longer together than the
+// corpus (offsets out of order), work that the caller would wait behind.
+__device__ __forceinline__ bool refused(int64_t part) { return __ballot(part < 0) != 0ull; }
 
 // Per-thread last-error text behind tms_last_error().
 void set_error(const char* fmt, ...);

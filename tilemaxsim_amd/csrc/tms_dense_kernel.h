@@ -168,7 +168,9 @@ __global__ void __launch_bounds__(NT, 1) dense_maxsim_kernel(DenseArgs a) {
     else return load_chunk<QDT, ALIGNED>(a.Q, row, 4 * S + gg, a.d, a.nchunk);
   };
 
-  const int64_t pad_len = MODE == MODE_VARLEN ? pad_length(a.pad, lane) : 0;
+  const int64_t pad = MODE == MODE_VARLEN ? pad_part(a.pad, lane) : 0;
+  const int64_t pad_len = MODE == MODE_VARLEN ? pad_length(a.pad, pad) : 0;
+  const bool refuse = MODE == MODE_VARLEN && refused(pad);
 
   // Query blocks of this launch: [my_blk0, my_blk0 + my_nblk).
   const int my_blk0 = a.blk0, my_nblk = a.nblk;
@@ -327,7 +329,7 @@ __global__ void __launch_bounds__(NT, 1) dense_maxsim_kernel(DenseArgs a) {
     bad = false;
     if constexpr (MODE == MODE_VARLEN) {
       int64_t s = a.offsets[b], e = a.offsets[b + 1];
-      if (s < 0 || e < s || e > a.total_tokens) {
+      if (refuse || s < 0 || e < s || e > a.total_tokens) {
         bad = true;
         base = 0;
         return 0;

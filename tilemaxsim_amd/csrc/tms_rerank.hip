@@ -79,14 +79,14 @@ __device__ __forceinline__ void rerank_body(const RerankArgs& a) {
     qtmp[i] = v ? *(const u32x4*)(a.Q + (row * a.d + 8 * (4 * s + (fl >> 4))) * 2) : u32x4{0u, 0u, 0u, 0u};
   }
 
-  const int64_t pad_len = MODE == RR_VARLEN ? pad_length(a.pad, lane) : 0;
+  const int64_t pad = MODE == RR_VARLEN ? pad_part(a.pad, lane) : 0;
   // the document's rows [base, base + len); invalid offsets mark it bad
   int64_t base = 0, len = 0;
   bool bad = false;
   if (live) {
     if constexpr (MODE == RR_VARLEN) {
       const int64_t s = a.offsets[b], e = a.offsets[b + 1];
-      bad = s < 0 || e < s || e > a.T;
+      bad = s < 0 || e < s || e > a.T || refused(pad);
       base = bad ? 0 : s;
       len = bad ? 0 : e - s;
     } else {
@@ -94,6 +94,7 @@ __device__ __forceinline__ void rerank_body(const RerankArgs& a) {
       len = a.nd;
     }
   }
+  const int64_t pad_len = MODE == RR_VARLEN ? pad_length(a.pad, pad) : 0;
   base = wave_uniform(base);
   len = wave_uniform(len);
   const int64_t ntile = (len + 15) / 16;

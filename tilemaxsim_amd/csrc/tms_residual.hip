@@ -272,7 +272,7 @@ __global__ void __launch_bounds__(256) residual_maxsim_kernel(ResArgs a) {
   // The wave's documents (at most 64) are read once, lane j holding document
   // b_begin + j: base row and length (-1 for an invalid pid or offsets). The walk
   // below takes them with readlane, so crossing a document never waits for memory.
-  const int64_t pad_len = pad_length(a.pad, lane);
+  const int64_t pad = pad_part(a.pad, lane);
   int64_t dbase = 0;
   int32_t dlen = -1;
   if (b_begin + lane < b_end) {
@@ -285,6 +285,8 @@ __global__ void __launch_bounds__(256) residual_maxsim_kernel(ResArgs a) {
       }
     }
   }
+  if (refused(pad)) dlen = -1;
+  const int64_t pad_len = pad_length(a.pad, pad);
   auto bounds = [&](int64_t b, int64_t& base) -> int64_t {
     const int j = (int)(b - b_begin);
     const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)dbase, j);
@@ -552,7 +554,7 @@ __device__ __forceinline__ void residual_batched_body(const ResArgs& a, ResShare
 
   // The workgroup's documents (at most 64): lane j holds document b_begin + j's first
   // index row and length (-1 for an invalid pid or offsets).
-  const int64_t pad_len = pad_length(a.pad, lane);
+  const int64_t pad = pad_part(a.pad, lane);
   int64_t dbase = 0;
   int32_t dlen = -1;
   if (lane < ndocs) {
@@ -565,6 +567,8 @@ __device__ __forceinline__ void residual_batched_body(const ResArgs& a, ResShare
       }
     }
   }
+  if (refused(pad)) dlen = -1;
+  const int64_t pad_len = pad_length(a.pad, pad);
   // Per-document scores of the wave's blocks: lane j holds document b_begin + j.
   float pend[NB];
 #pragma unroll

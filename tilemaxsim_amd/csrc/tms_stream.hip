@@ -127,6 +127,7 @@ __global__ void __launch_bounds__(256, 1) stream_maxsim_kernel(StreamArgs a) {
   // length (-1: invalid offsets).
   int64_t dbase = 0;
   int32_t dlen = 0;
+  const int64_t pad = VARLEN ? pad_part(a.pad, lane) : 0;
   if constexpr (VARLEN) {
     dlen = -1;
     if (lane < ndocs) {
@@ -136,6 +137,10 @@ __global__ void __launch_bounds__(256, 1) stream_maxsim_kernel(StreamArgs a) {
         dlen = (int32_t)(e0 - s0);
         dbase = dlen > 0 ? s0 : 0;
       }
+    }
+    if (refused(pad)) {
+      dlen = -1;
+      dbase = 0;
     }
   }
   // MASKED: the bits of the lane's tile, and which of the wave's tiles hold a real token
@@ -151,7 +156,7 @@ __global__ void __launch_bounds__(256, 1) stream_maxsim_kernel(StreamArgs a) {
   auto doc_live = [&](int64_t dd) -> uint64_t {  // MASKED: bit t: tile t holds a real token
     return (mlive >> (dd * mtiles)) & (~0ull >> (64 - mtiles));
   };
-  const int64_t pad_len = VARLEN ? pad_length(a.pad, lane) : 0;
+  const int64_t pad_len = VARLEN ? pad_length(a.pad, pad) : 0;
   auto doc_len = [&](int64_t dd) -> int64_t {
     if constexpr (VARLEN) return (int32_t)__builtin_amdgcn_readlane((uint32_t)dlen, (int)dd);
     else return a.nd;

@@ -96,9 +96,10 @@ def flash_maxsim_multi_doc(Q: torch.Tensor, D_flat: torch.Tensor, doc_offsets: t
     lib = _lib.load()
     with _lib.on_device(Q.device):
         if validate:  # the check runs on the device before the scoring kernel; its verdict is waited for
+            parts = torch.empty(_lib.TMS_CHECK_PARTS, dtype=torch.int64, device=Q.device)
             _lib.check_bounds(
                 lib.tms_maxsim_varlen_checked(Q.data_ptr(), 1, Nq, d, D_flat.data_ptr(), T, offsets.data_ptr(), num_docs, 0,
-                                              code, scores.data_ptr(), None, _lib.verdict_ptr(), _lib.stream_of(Q)),
+                                              code, scores.data_ptr(), parts.data_ptr(), _lib.verdict_ptr(), _lib.stream_of(Q)),
                 "flash_maxsim_multi_doc: doc_offsets must be non-decreasing within [0, total_tokens]")
             return scores
         _lib.check(lib.tms_maxsim_varlen(Q.data_ptr(), Nq, d, D_flat.data_ptr(), T, offsets.data_ptr(), num_docs,
@@ -134,10 +135,10 @@ def _varlen_batched(fn: str, Qs: torch.Tensor, D_flat: torch.Tensor, doc_offsets
     lib = _lib.load()
     with _lib.on_device(Qs.device):
         if validate or zero_pad:
-            parts = torch.empty(_lib.TMS_CHECK_PARTS, dtype=torch.int64, device=Qs.device) if zero_pad else None
+            parts = torch.empty(_lib.TMS_CHECK_PARTS, dtype=torch.int64, device=Qs.device)
             _lib.check_bounds(
                 lib.tms_maxsim_varlen_checked(Qs.data_ptr(), nQ, Nq, d, D_flat.data_ptr(), T, offsets.data_ptr(), B,
-                                              int(zero_pad), code, out.data_ptr(), _lib.ptr(parts), _lib.verdict_ptr(),
+                                              int(zero_pad), code, out.data_ptr(), parts.data_ptr(), _lib.verdict_ptr(),
                                               _lib.stream_of(Qs)),
                 f"{fn}: doc_offsets must be non-decreasing within [0, total_tokens]")
             return out

@@ -105,7 +105,7 @@ def _score(fn: str, Qs, nQ: int, Nq: int, d: int, batched: bool, index, offsets,
     waited for."""
     codes, residuals, centroids, bucket_weights, nbits = index
     zeros = padding == "zeros"
-    parts = torch.empty(_lib.TMS_CHECK_PARTS, dtype=torch.int64, device=out.device) if zeros else None
+    parts = torch.empty(_lib.TMS_CHECK_PARTS, dtype=torch.int64, device=out.device) if validate or zeros else None
     lib = _lib.load()
     with _lib.on_device(out.device):
         args = (Nq, d, centroids.data_ptr(), centroids.shape[0], bucket_weights.data_ptr(), nbits, codes.data_ptr(),
