@@ -38,6 +38,7 @@
 #include <string.h>
 
 #include "tms_common.h"
+#include "tms_rules.h"
 
 namespace tms {
 
@@ -720,13 +721,6 @@ constexpr size_t kStaticLds = 256;  // an unsplit launch's static LDS (per-token
 #define TMS_DENSE_PFD 1  // tiles in flight ahead of the one being scored
 #endif
 
-// Waves a call of split documents may launch: two per SIMD, or one and a half with the query
-// in VGPRs (fp32, d <= 128). A small call is bound by each wave's walk of its tiles, a larger one
-// by the read: d = 512 fp16, 231 tokens, 100 / 500 / 1,000 documents 40 / 46 / 50 us whole,
-// 16 / 25 / 43 split, 1,500 72 / 77; fp32 d = 128, 150 tokens, 100 / 500 documents 14.2 / 16.4 us
-// whole, 7.9 / 11.2 split, 1,000 17.7 / 18.2.
-constexpr int64_t kSplitWaves = 2048, kSplitWavesReg = 1536;
-
 // LDS bytes of the query fragments of one launch (split queries: hi and lo terms).
 static inline size_t qlds_bytes(int dtype, int qdtype, int nqb, int nstep) {
   const bool split = dtype == TMS_DTYPE_F32 || qdtype == TMS_DTYPE_F32;
@@ -762,12 +756,9 @@ static int launch_nt(const DenseArgs& a, int64_t waves, size_t lds, hipStream_t 
                   lds, cap);
   }
   if constexpr (MODE == MODE_FIXED && NT == 256 && KS_REG >= 0) {
-    // documents split over two or four waves, at most one wave per tile
+    // small calls: documents split over two or four waves
     DenseArgs s = a;
-    s.wpd = 1;
-    const int64_t tiles = (a.nd + 16 * NS - 1) / (16 * NS);
-    while (s.wpd < 4 && 2 * s.wpd <= tiles && 2 * s.wpd * a.B <= (KS_REG > 0 ? kSplitWavesReg : kSplitWaves))
-      s.wpd *= 2;
+    s.wpd = dense_split_waves(a.B, (a.nd + 16 * NS - 1) / (16 * NS), lds, NQB, KS_REG);
     if (s.wpd > 1) {
       hipLaunchKernelGGL((dense_maxsim_kernel<DT, QDT, MODE, NQB, KS_REG, FULL, ALIGNED, NS, TMS_DENSE_PFD, NT, true>),
                          dim3((unsigned)((a.B * s.wpd + 3) / 4)), dim3(NT), lds, st, s);
