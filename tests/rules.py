@@ -26,6 +26,9 @@ def lib():
         out = ctypes.CDLL(so)
     i64, integer = ctypes.c_int64, ctypes.c_int
     out.dense_split_waves.argtypes = [i64, i64, ctypes.c_size_t, integer, integer]
+    out.topk_group_lanes.argtypes = [i64, i64, integer]
+    out.topk_workspace.argtypes = [i64, i64, integer]
+    out.topk_workspace.restype = i64
     return out
 
 

@@ -34,3 +34,36 @@ def test_dense_split_bounds():
     ("float32", "float32", 64, 32, 400, 768, 2), ("float32", "float32", 128, 64, 1000, 768, 1)])
 def test_dense_split_stays_where_it_is_faster(qdt, ddt, d, nq, nd, B, want):
     assert rules.dense_split(qdt, ddt, d, nq, B, nd) == want
+
+
+def test_topk_groups_fit():
+    """k groups fit the selection, the maxima the workspace, the spans their stage."""
+    lanes, workspace = rules.lib().topk_group_lanes, rules.lib().topk_workspace
+    taken = 0
+    for rows, n, k in itertools.product((1, 3, 256, 257, 513, 65535), (8, 4096, 4097, 5000, 24_000, 33_000, 131_073, 1 << 20, 4_200_000,
+                                                                      1 << 24, (1 << 24) + 1, (1 << 32) - 1),
+                                        (1, 7, 8, 9, 64, 100, 128, 129, 200, 300, 321, 512, 513, 1024)):
+        lg = lanes(rows, n, k)
+        if lg == 0:
+            continue
+        taken += 1
+        keys, spans, per = (4096 if k <= 128 else 16384), -(-n // 1024), 1024 >> (lg + 2)
+        assert 3 <= lg <= 6 and (4 << lg) * k <= keys and n > 4096
+        direct = spans * per <= keys
+        assert direct or (k <= spans <= 16384 and per * k <= keys)
+        assert 4 * rows * spans * (per + (not direct)) <= workspace(rows, n, k)
+    assert taken > 100
+
+
+@pytest.mark.parametrize("rows,n,k,groups", [
+    # more rows than run at once: short ones take the tournament
+    (4096, 8192, 100, False), (10_000, 5000, 10, False), (4096, 5000, 128, False), (2048, 16_384, 200, False),
+    (1000, 8192, 100, False), (257, 8192, 100, False), (256, 8192, 100, True), (2048, 40_000, 100, True), (512, 24_000, 100, True),
+    # few groups for their k, and the tournament's slow last chunk
+    (1, 5000, 128, False), (1, 6500, 128, True), (1, 4200, 128, True), (1, 5000, 100, True), (1, 16_384, 256, False),
+    (1, 24_000, 200, True), (300, 20_000, 200, False),
+    # large k needs much to save
+    (1, 300_000, 512, False), (16, 100_000, 460, False), (64, 100_000, 512, True), (1, 1_000_000, 512, True),
+    (32, 1_000_000, 100, True)])
+def test_topk_groups_stay_where_they_are_faster(rows, n, k, groups):
+    assert (rules.lib().topk_group_lanes(rows, n, k) > 0) == groups

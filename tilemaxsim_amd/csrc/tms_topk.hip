@@ -8,28 +8,7 @@
 
 namespace tms {
 
-static int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
-
-// Keys per row after each level, starting from n; stops when a row fits one chunk.
-static int64_t level_sizes(int64_t n, int k, int64_t* sizes, int max_levels) {
-  int64_t lv = 0;
-  while (n > kChunk && lv < max_levels) {
-    n = ceil_div(n, kChunk) * k;
-    sizes[lv++] = n;
-  }
-  return lv;
-}
-
-int64_t topk_workspace_bytes(int64_t nrows, int64_t n, int k) {
-  int64_t sizes[64];
-  const int64_t lv = level_sizes(n, k, sizes, 64);
-  int64_t a = 0, b = 0;  // ping-pong buffers: even levels in a, odd in b
-  for (int64_t i = 0; i < lv; i++) {
-    if (i % 2 == 0) a = sizes[i] > a ? sizes[i] : a;
-    else b = sizes[i] > b ? sizes[i] : b;
-  }
-  return (a + b) * nrows * (int64_t)sizeof(uint64_t);
-}
+int64_t topk_workspace_bytes(int64_t nrows, int64_t n, int k) { return topk_workspace(nrows, n, k); }
 
 }  // namespace tms
 
@@ -70,26 +49,6 @@ int topk_checks(const char* fn, const float* scores, int64_t nrows, int64_t n, i
   return TMS_OK;
 }
 
-// Group maxima (tms_topk_kernel.h): the groups' size for k, or 0 where the tournament takes
-// the row. k groups of a span's or of g scores have to fit the selection's keys (4,096 up to
-// k = 128, 16,384 up to 512), the spans its first stage, and the maxima the workspace the
-// tournament would use (which leaves it k < 8 and a few k above a power of two). Rows of few
-// groups for their k stay too: their maxima bound little (5,000 scores, k = 200: 17 us, by
-// groups 51).
-constexpr int64_t kGroupMaxSpans = 16384;
-static int group_lanes_log2(int64_t nrows, int64_t n, int k) {
-  const int64_t keys = k <= kFilterMaxK ? 4096 : 16384;
-  if (n <= kChunk || k > keys / 32 || (k > kFilterMaxK && n < (int64_t)64 * k)) return 0;
-  int lg = 3;
-  // the largest group of which k fit, with twice k groups in the row
-  while (lg < 6 && ((int64_t)8 << lg) * k <= keys && n >= 2 * ((int64_t)8 << lg) * k) lg++;
-  const int64_t spans = ceil_div(n, kSpan), per = kSpan >> (lg + 2);
-  const bool direct = spans * per <= keys;
-  if (!direct && (spans > kGroupMaxSpans || per * k > keys || spans < k)) return 0;
-  const int64_t need = nrows * spans * (per + (direct ? 0 : 1)) * (int64_t)sizeof(uint32_t);
-  return need <= topk_workspace_bytes(nrows, n, k) ? lg : 0;
-}
-
 template <int CH1, int CHS>
 static void group_last(int64_t nrows, hipStream_t st, const float* scores, int64_t n, int64_t spans, int lg,
                        const uint32_t* groups, const uint32_t* spans_in, float* out_values, int64_t* out_indices, int k) {
@@ -99,7 +58,7 @@ static void group_last(int64_t nrows, hipStream_t st, const float* scores, int64
 
 static int group_run(const float* scores, int64_t nrows, int64_t n, int k, int lg, uint32_t* ws, float* out_values,
                      int64_t* out_indices, hipStream_t st) {
-  const int64_t keys = k <= kFilterMaxK ? 4096 : 16384;
+  const int64_t keys = topk_group_keys(k);
   const int64_t spans = ceil_div(n, kSpan), per = kSpan >> (lg + 2), total = nrows * spans;
   uint32_t* groups = ws;
   uint32_t* spans_out = spans * per <= keys ? nullptr : ws + total * per;
@@ -131,10 +90,10 @@ static int group_run(const float* scores, int64_t nrows, int64_t n, int k, int l
 // The levels of one call; `workspace` holds topk_workspace_bytes(nrows, n, k) bytes.
 int topk_run(const float* scores, int64_t nrows, int64_t n, int64_t k, void* workspace, float* out_values,
              int64_t* out_indices, hipStream_t st) {
-  if (const int lg = group_lanes_log2(nrows, n, (int)k))
+  if (const int lg = topk_group_lanes(nrows, n, (int)k))
     return group_run(scores, nrows, n, (int)k, lg, (uint32_t*)workspace, out_values, out_indices, st);
   int64_t sizes[64];
-  const int64_t lv = level_sizes(n, (int)k, sizes, 64);
+  const int64_t lv = topk_level_sizes(n, (int)k, sizes, 64);
   int64_t amax = 0;
   for (int64_t i = 0; i < lv; i += 2) amax = sizes[i] > amax ? sizes[i] : amax;
   uint64_t* bufs[2] = {(uint64_t*)workspace, (uint64_t*)workspace + amax * nrows};

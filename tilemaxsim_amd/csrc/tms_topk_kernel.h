@@ -25,10 +25,10 @@
 // into its own copy of the histogram.
 #pragma once
 #include "tms_common.h"
+#include "tms_rules.h"
 
 namespace tms {
 
-constexpr int kChunk = 4096;  // keys sorted per workgroup (32 KiB of LDS)
 // Threads per workgroup: a level that shrinks many chunks at once runs 4 waves per chunk
 // (16 keys per thread); the last level, one chunk per row and nothing else running
 // beside it, runs 16 waves (4 keys per thread, four waves per SIMD to overlap its serial
@@ -40,13 +40,11 @@ constexpr int kMaxK = kChunk / 4;
 // Rows (or last levels) of at most kShortRow keys: one chunk of that size over four
 // waves, one per SIMD, so the serial steps (scans, reductions) are not repeated by four
 // waves on every SIMD.
-constexpr int kShortRow = 1024;
 constexpr int kShortThreads = 256;
 constexpr int kRankSortMaxK = 256;  // the last level orders up to this many keys by rank, more by a bitonic sort
 // Levels that pass k keys on, at k <= kFilterMaxK, first drop the keys below a bound on
 // the chunk's k-th key and select among the rest, gathered in LDS, when at most
 // kCandCap of them remain.
-constexpr int kFilterMaxK = 128;
 constexpr int kCandCap = 1024;
 
 // Order-preserving image of a float's bits, never 0 (0 is the padding key). Positive
@@ -605,7 +603,6 @@ __global__ void __launch_bounds__(NT) topk_level_kernel(const float* __restrict_
 // their groups, then the scores of those groups, from at most CHS keys at a time, and reads
 // g k scores again instead of sorting every chunk. The first pass is bound by the read of the
 // scores; the tournament's first level was bound by its issue (VALUBusy 71-81 %).
-constexpr int kSpan = 1024;
 constexpr int kGroupWaves = 4;  // waves per workgroup of the first pass
 
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // rows start at any score
