@@ -75,6 +75,41 @@ def test_long_rows(cuda, n):
     _check(_fill("rising", 1, n, n), [100, 300])
 
 
+@pytest.mark.parametrize("n,k,groups,kept", [
+    (40_000, 100, 100, c) for c in (100, 767, 768, 769, 3000)] + [
+    (100_000, 300, 300, c) for c in (1023, 1024, 1025, 5000)] + [
+    # by spans: the groups that reach the bound in one load of the selection, in two, and in too many
+    (1_000_000, 100, 100, c) for c in (700, 2000)] + [
+    (1_000_000, 100, 200, c) for c in (700, 5000)] + [(1_000_000, 100, 600, 15_000), (1_000_000, 400, 1200, 20_000)])
+def test_scores_that_reach_the_bound(cuda, n, k, groups, kept):
+    """``kept`` scores reach the k-th largest maximum, in ``groups`` groups of 32 (as many a
+    span in the k best spans, where spans come first): on both sides of the count that is
+    ordered by rank, and of what the last selection holds."""
+    import torch
+    import rules
+    assert rules.lib().topk_group_lanes(2, n, k) == 3
+    g = torch.Generator(device="cuda").manual_seed(n + kept)
+    x = torch.randn(2, n, generator=g, device="cuda")
+    spans = n > 100_000
+    for row in range(2):
+        if spans:  # groups // k of each of k spans
+            span = torch.randperm(n // 1024, generator=g, device="cuda")[:k]
+            first = (span[:, None] * 1024 + 32 * torch.arange(groups // k, device="cuda")).reshape(-1)
+        else:
+            first = 32 * torch.randperm(n // 32, generator=g, device="cuda")[:groups]
+        first = first.cpu()
+        # one score of the first group is the bound, and in its span the largest; the others go over the rest
+        lead = 1 if not spans else groups // k
+        rest = (first[lead:, None] + torch.arange(32)).reshape(-1, 32)
+        order = torch.cat([rest[:, 0], rest[:, 1:].reshape(-1)[torch.randperm(rest.numel() - len(rest))]])
+        at = order[:kept - lead].cuda()
+        x[row, at] = 200.0 + torch.rand(len(at), generator=g, device="cuda")
+        x[row, first[:lead].cuda()] = 100.0
+    reach = torch.sort(x, dim=1, descending=True).values
+    assert bool((reach[:, kept - 1] == 100.0).all()) and bool((reach[:, kept] < 50.0).all())
+    _check(x, [k])
+
+
 def test_alignment_and_rows(cuda):
     """Rows that start at every offset of 16 bytes (odd row lengths), and many rows."""
     import torch

@@ -695,9 +695,11 @@ __global__ void __launch_bounds__(64 * kGroupWaves) topk_group_max_kernel(const 
 // First the fast way: the k-th largest maximum T is a bound on the k-th largest score, so
 // after one selection among the maxima only what reaches T is kept: the k best spans' groups,
 // those groups' scores (on continuous scores a few more than k), and the scores kept are
-// ordered by rank. Lists that outgrow kFastCap (sorted rows, ties) take the selection level
-// by level. 32 rows of 1M scores, k = 100: 32 us with the first pass, against 58 for the
-// tournament and 41 selecting level by level throughout.
+// ordered by rank. Where more are kept than ranks are cheap for (sorted rows, ties) the last
+// selection, or the last two, run over the groups or spans found so far: 1 row of 5,000 scores in
+// sorted runs of 100, k = 100, 16 us (59 by ranks of up to 2,048), 64 sorted rows of 8,192 18
+// (26 with all selections anew). 32 rows of 1M scores, k = 100: 32 us with the first pass,
+// against 58 for the tournament and 41 selecting level by level throughout.
 constexpr int kFastCap = 2048;
 template <int CH1, int CHS>
 __global__ void __launch_bounds__(kLastThreads) topk_group_last_kernel(const float* __restrict__ vals, int64_t n,
@@ -708,20 +710,35 @@ __global__ void __launch_bounds__(kLastThreads) topk_group_last_kernel(const flo
                                                                        int64_t* __restrict__ out_idx, int k) {
   constexpr int NT = kLastThreads, NW = NT / 64;
   constexpr int PER = CHS / NT;
+  constexpr int kRankCap = CHS <= 4096 ? 768 : 1024;  // scores ordered by rank, within one turn of the threads
   __shared__ uint64_t picked[kMaxK];
+  __shared__ uint32_t gsel[kFastCap];
+  enum { NOTHING, FIRST_MAXIMA, GROUPS } have = NOTHING;  // selected so far: picked (of `top`), or gsel and total
+  int total = 0;      // scores of the groups in gsel
+  uint32_t at[PER];   // their indices (past the row: 2^32 - 1) and values
+  float v[PER] = {};
   const int tid = threadIdx.x;
   const int64_t row = blockIdx.x;
   const int per = kSpan >> (lg + 2);  // groups per span
   const int glog = lg + 2;            // log2 of the scores per group
   const uint32_t* __restrict__ grow = groups + row * spans * per;
   const float* __restrict__ vrow = vals + row * n;
+  auto load_scores = [&](int c0) {  // scores [c0, c0 + CHS) of the total
+#pragma unroll
+    for (int e = 0; e < PER; e++) {
+      const int c = c0 + e * NT + tid;
+      const bool in = c < total;
+      const uint64_t i = ((uint64_t)gsel[in ? c >> glog : 0] << glog) + (uint64_t)(c & ((1 << glog) - 1));
+      at[e] = in && i < (uint64_t)n ? (uint32_t)i : 0xffffffffu;
+      v[e] = vrow[at[e] != 0xffffffffu ? at[e] : 0u];
+    }
+  };
 
   {
     __shared__ uint64_t list[kFastCap];
     __shared__ uint32_t wave_t[NW], n_list, n_groups, n_sel, bound;
-    __shared__ uint32_t gsel[kFastCap];
-    __shared__ uint64_t sel[kFastCap + kRankPad + 8];
-    __shared__ uint32_t sel_bits[kFastCap];
+    __shared__ uint64_t sel[kRankCap + kRankPad + 8];
+    __shared__ uint32_t sel_bits[kRankCap];
     const int lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
     // appends the lanes with `take` to a list; returns the lane's slot
     auto slot = [&](uint32_t* count, bool take) -> uint32_t {
@@ -746,7 +763,7 @@ __global__ void __launch_bounds__(kLastThreads) topk_group_last_kernel(const flo
       tm = x[e] > tm ? x[e] : tm;
     }
     if (tid == 0) n_list = n_groups = n_sel = 0u;
-    for (int i = tid; i < kFastCap + kRankPad + 8; i += NT) sel[i] = 0ull;
+    for (int i = tid; i < kRankCap + kRankPad + 8; i += NT) sel[i] = 0ull;
     // a lower bound on the k-th maximum, as in topk_core's pre-filter
     const uint32_t j = (uint32_t)((k + NW - 1) / NW);
     uint32_t t = 0u;
@@ -767,8 +784,8 @@ __global__ void __launch_bounds__(kLastThreads) topk_group_last_kernel(const flo
         if (e * NT >= count) break;
         const int c = e * NT + lane * NW + wid;
         const bool take = x[e] >= T;
-        const uint32_t at = slot(&n_list, take);
-        if (take && at < (uint32_t)kFastCap) list[at] = ((uint64_t)x[e] << 32) | (uint64_t)(0xffffffffu - (uint32_t)c);
+        const uint32_t p = slot(&n_list, take);
+        if (take && p < (uint32_t)kFastCap) list[p] = ((uint64_t)x[e] << 32) | (uint64_t)(0xffffffffu - (uint32_t)c);
       }
       __syncthreads();
       const int m = (int)n_list;
@@ -792,9 +809,10 @@ __global__ void __launch_bounds__(kLastThreads) topk_group_last_kernel(const flo
         }
         __syncthreads();
         T = bound;
+        have = FIRST_MAXIMA;
         uint32_t ng;
         if (spans_in) {
-          uint32_t at[PER], y[PER];
+          uint32_t y[PER];
 #pragma unroll
           for (int e = 0; e < PER; e++) {
             const int c = e * NT + tid;
@@ -817,31 +835,24 @@ __global__ void __launch_bounds__(kLastThreads) topk_group_last_kernel(const flo
         }
         ok = ng <= (uint32_t)kFastCap && (int)(ng << glog) <= 4 * CHS;
         if (ok) {
-          for (int c0 = 0; c0 < (int)(ng << glog); c0 += CHS) {
-            float y[PER];
-            uint32_t at[PER];
+          total = (int)(ng << glog);
+          for (int c0 = 0; c0 < total; c0 += CHS) {
+            load_scores(c0);
 #pragma unroll
             for (int e = 0; e < PER; e++) {
-              const int c = c0 + e * NT + tid;
-              const bool in = c < (int)(ng << glog);
-              const uint64_t i64 = ((uint64_t)gsel[in ? c >> glog : 0] << glog) + (uint64_t)(c & ((1 << glog) - 1));
-              at[e] = in && i64 < (uint64_t)n ? (uint32_t)i64 : 0xffffffffu;
-              y[e] = vrow[at[e] != 0xffffffffu ? at[e] : 0u];
-            }
-#pragma unroll
-            for (int e = 0; e < PER; e++) {
-              const uint32_t o = order_key(y[e]);
+              const uint32_t o = order_key(v[e]);
               const bool take = at[e] != 0xffffffffu && o >= T;
               const uint32_t p = slot(&n_sel, take);
-              if (take && p < (uint32_t)kFastCap) {
+              if (take && p < (uint32_t)kRankCap) {
                 sel[p] = ((uint64_t)o << 32) | (uint64_t)(0xffffffffu - at[e]);
-                sel_bits[p] = __builtin_bit_cast(uint32_t, y[e]);
+                sel_bits[p] = __builtin_bit_cast(uint32_t, v[e]);
               }
             }
           }
+          if (total <= CHS) have = GROUPS;
           __syncthreads();
           const int ms = (int)n_sel;  // >= k: each of the k best maxima is one
-          if (ms <= kFastCap) {
+          if (ms <= kRankCap) {
             topk_rank_out<true, NT>(sel, sel_bits, ms, (ms + 7) & ~7, nullptr, 0, out_vals, out_idx, k, row);
             return;
           }
@@ -852,47 +863,46 @@ __global__ void __launch_bounds__(kLastThreads) topk_group_last_kernel(const flo
   }
 
   uint64_t key[PER];
-  float v[PER] = {};
-  if (spans_in) {
-    uint64_t k1[CH1 / NT];
-    const float none[CH1 / NT] = {};
+  if (have != GROUPS) {
+    if (spans_in) {
+      if (have == NOTHING) {
+        uint64_t k1[CH1 / NT];
+        const float none[CH1 / NT] = {};
 #pragma unroll
-    for (int e = 0; e < CH1 / NT; e++) {
-      const int64_t c = e * NT + tid;
-      k1[e] = c < spans ? ((uint64_t)spans_in[row * spans + c] << 32) | (uint64_t)(0xffffffffu - (uint32_t)c) : 0ull;
+        for (int e = 0; e < CH1 / NT; e++) {
+          const int64_t c = e * NT + tid;
+          k1[e] = c < spans ? ((uint64_t)spans_in[row * spans + c] << 32) | (uint64_t)(0xffffffffu - (uint32_t)c) : 0ull;
+        }
+        topk_core<false, false, NT, CH1>(k1, none, nullptr, 0, spans, picked, 0, nullptr, nullptr, k, 0, 0);
+        __syncthreads();
+      }
+#pragma unroll
+      for (int e = 0; e < PER; e++) {
+        const int c = e * NT + tid;
+        const uint32_t span = c < k * per ? 0xffffffffu - (uint32_t)picked[c / per] : 0u;
+        at[e] = span * (uint32_t)per + (uint32_t)(c & (per - 1));
+        key[e] = c < k * per ? (uint64_t)grow[at[e]] : 0ull;
+      }
+#pragma unroll
+      for (int e = 0; e < PER; e++) key[e] = key[e] != 0ull ? (key[e] << 32) | (uint64_t)(0xffffffffu - at[e]) : 0ull;
+      __syncthreads();  // picked is read; the next selection writes it
+    } else {
+#pragma unroll
+      for (int e = 0; e < PER; e++) {
+        const int64_t c = e * NT + tid;
+        const uint32_t x = c < spans * per ? grow[c] : 0u;
+        key[e] = x != 0u ? ((uint64_t)x << 32) | (uint64_t)(0xffffffffu - (uint32_t)c) : 0ull;
+      }
     }
-    topk_core<false, false, NT, CH1>(k1, none, nullptr, 0, spans, picked, 0, nullptr, nullptr, k, 0, 0);
+    topk_core<false, false, NT, CHS>(key, v, nullptr, 0, CHS, picked, 0, nullptr, nullptr, k, 0, 0);
     __syncthreads();
-    uint32_t at[PER];
-#pragma unroll
-    for (int e = 0; e < PER; e++) {
-      const int c = e * NT + tid;
-      const uint32_t span = c < k * per ? 0xffffffffu - (uint32_t)picked[c / per] : 0u;
-      at[e] = span * (uint32_t)per + (uint32_t)(c & (per - 1));
-      key[e] = c < k * per ? (uint64_t)grow[at[e]] : 0ull;
-    }
-#pragma unroll
-    for (int e = 0; e < PER; e++) key[e] = key[e] != 0ull ? (key[e] << 32) | (uint64_t)(0xffffffffu - at[e]) : 0ull;
-    __syncthreads();  // picked is read; the next selection writes it
-  } else {
-#pragma unroll
-    for (int e = 0; e < PER; e++) {
-      const int64_t c = e * NT + tid;
-      const uint32_t x = c < spans * per ? grow[c] : 0u;
-      key[e] = x != 0u ? ((uint64_t)x << 32) | (uint64_t)(0xffffffffu - (uint32_t)c) : 0ull;
-    }
-  }
-  topk_core<false, false, NT, CHS>(key, v, nullptr, 0, CHS, picked, 0, nullptr, nullptr, k, 0, 0);
-  __syncthreads();
-  uint32_t at[PER];
-#pragma unroll
-  for (int e = 0; e < PER; e++) {
-    const int c = e * NT + tid;
-    const uint64_t pk = c < k << (lg + 2) ? picked[c >> (lg + 2)] : 0ull;
-    // a padding key (fewer than k groups) names no group
-    const uint64_t i = (uint64_t)(0xffffffffu - (uint32_t)pk) * (uint64_t)(4 << lg) + (uint64_t)(c & ((4 << lg) - 1));
-    at[e] = pk != 0ull && i < (uint64_t)n ? (uint32_t)i : 0xffffffffu;
-    v[e] = vrow[at[e] != 0xffffffffu ? at[e] : 0u];
+    // a padding key (fewer than k groups) names no group: its first score lies past the row
+    if (tid < k) gsel[tid] = picked[tid] != 0ull ? 0xffffffffu - (uint32_t)picked[tid] : 0xffffffffu;
+    __syncthreads();
+    total = k << glog;
+    load_scores(0);
+  } else if (PER > 4) {  // too many to have been kept in registers
+    load_scores(0);
   }
 #pragma unroll
   for (int e = 0; e < PER; e++)
