@@ -29,6 +29,7 @@ def lib():
     out.topk_group_lanes.argtypes = [i64, i64, integer]
     out.topk_workspace.argtypes = [i64, i64, integer]
     out.topk_workspace.restype = i64
+    out.pq_per_query.argtypes = [i64] * 6
     return out
 
 

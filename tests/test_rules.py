@@ -67,3 +67,14 @@ def test_topk_groups_fit():
     (32, 1_000_000, 100, True)])
 def test_topk_groups_stay_where_they_are_faster(rows, n, k, groups):
     assert (rules.lib().topk_group_lanes(rows, n, k) > 0) == groups
+
+
+@pytest.mark.parametrize("M,K,dsub,nQ,nq,tokens,alone", [
+    (16, 256, 8, 2, 32, 524_288, True), (16, 256, 8, 2, 32, 524_287, False), (16, 256, 8, 3, 32, 1_179_647, False),
+    (16, 256, 8, 3, 32, 1_179_648, True), (16, 64, 4, 3, 32, 1 << 21, False), (16, 64, 4, 3, 32, 3 << 20, True), (16, 256, 8, 6, 32, 10_240_000, True), (16, 256, 8, 7, 32, 25_600_000, False),
+    # codebooks whose shared pass costs few queries, or whose own kernel is slow
+    (64, 256, 2, 6, 32, 25_600_000, False), (64, 256, 2, 4, 32, 25_600_000, False), (64, 256, 2, 3, 32, 25_600_000, True),
+    (4, 256, 32, 6, 32, 25_600_000, False), (4, 256, 32, 4, 32, 25_600_000, True), (32, 64, 2, 6, 32, 25_600_000, False), (16, 64, 4, 6, 32, 10_240_000, False),
+    (16, 16, 8, 5, 32, 10_240_000, True), (16, 256, 8, 2, 64, 3_840_000, True), (16, 64, 4, 3, 64, 7_680_000, False)])
+def test_pq_queries_go_alone_where_it_is_faster(M, K, dsub, nQ, nq, tokens, alone):
+    assert bool(rules.lib().pq_per_query(nQ, -(-nq // 32), tokens, M, dsub, M * dsub * K * 2)) == alone

@@ -22,6 +22,7 @@
 #include <string.h>
 
 #include "tms_pq_kernel.h"
+#include "tms_rules.h"
 
 namespace tms {
 
@@ -545,14 +546,10 @@ int tms_pq_score_batched(const void* Qs, int64_t nQ, int64_t nq, const void* cod
   // The shared-tile kernel takes uint8 codes, a query of the codebook's type and a
   // codebook of at most 64 KiB beside its tile ring; other inputs, and queries of more
   // than 4 blocks, are scored one query at a time.
-  // Up to six blocks over many tokens go query by query too: the shared-tile workgroups then
-  // wait on each tile's gathers, 590 us a pass over 100,000 x 128 tokens where one query
-  // takes 108 by itself (7 queries: 712 against 756); with few tokens the launches weigh more
-  // (two queries over 1,000 documents: 11 us in one pass, 20 in two calls; four over 10,000:
-  // 65 against 82).
-  const int64_t blocks = nQ * nbq;
-  const bool per_query = blocks <= 6 && (int64_t)B * nd >= ((int64_t)1 << 17) * blocks * blocks;
-  const bool shared = flags == 0 && M * dsub * K * 2 <= 64 * 1024 && nbq <= 4 && blocks >= 2 && !per_query;
+  // A few queries over many tokens (pq_per_query) go that way, too.
+  const int64_t codebook_bytes = M * dsub * K * 2;
+  const bool shared = flags == 0 && codebook_bytes <= 64 * 1024 && nbq <= 4 && nQ * nbq >= 2 &&
+                      !pq_per_query(nQ, nbq, B * nd, M, dsub, codebook_bytes);
   if (!shared) {
     const int64_t qbytes = nq * M * dsub * ((flags & TMS_QUERY_F32) ? 4 : 2);
     for (int64_t q = 0; q < nQ; q++) {

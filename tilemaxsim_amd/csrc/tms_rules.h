@@ -35,6 +35,28 @@ inline int dense_split_waves(int64_t B, int64_t tiles, size_t lds, int nqb, int 
   return w;
 }
 
+// Whether a batched PQ call (nQ queries of nbq blocks, `tokens` of them, M codes of dsub
+// dimensions a token, a codebook of `lds` bytes) goes query by query. One pass of the
+// shared-tile workgroups waits on each tile's gathers whatever the queries are, so a few
+// queries over many tokens are faster one at a time, in their own kernel. With fewer tokens the
+// launches and each workgroup's codebook copy weigh more: blocks^2 x 131,072 tokens are enough for
+// two queries, or for five of a codebook that leaves a CU room for two shared-tile workgroups
+// (above 37 KiB, codewords of 8 to 32 bytes: `wide`), else twice that. A shared pass takes the
+// time of 5 to 6 queries there, of 3 to 4 where a query's own kernel gathers many short or few
+// long codewords (dsub = 2 of M = 32 or 64, dsub = 32), else of 4 to 5. 25.6M tokens, 2, 4 and
+// 6 queries, shared / one at a time: M = 16, K = 256, dsub = 8 1182 / 425, 1184 / 846, 1418 /
+// 1272; M = 16, K = 64, dsub = 4 467 / 268, 502 / 544, 692 / 815; M = 64, K = 256, dsub = 2 1418 /
+// 770, 1425 / 1547, 1676 / 2310.
+inline bool pq_per_query(int64_t nQ, int64_t nbq, int64_t tokens, int64_t M, int64_t dsub, int64_t lds) {
+  const int64_t blocks = nQ * nbq;
+  const bool wide = lds > 37 * 1024 && dsub >= 4 && dsub <= 16;
+  const int64_t unit = (int64_t)(nQ == 2 || (wide && nQ <= 5) ? 1 : 2) << 17;
+  if (blocks > 6 || tokens < unit * blocks * blocks) return false;
+  if (nQ <= 3) return true;
+  if (dsub == 2 && M > 16) return false;
+  return nQ <= (dsub > 16 ? 4 : 5) || wide;
+}
+
 // ---- top-k of fp32 rows (tms_topk_kernel.h) -----------------------------------------
 constexpr int kChunk = 4096;      // keys a tournament workgroup selects from
 constexpr int kFilterMaxK = 128;  // the largest k with a bound on the k-th key taken first
