@@ -183,6 +183,33 @@ def test_threads_and_streams(cuda):
     assert not wrong
 
 
+def test_default_device(cuda):
+    """Checked calls under a default device, in a thread that has made none before."""
+    import torch
+    import tilemaxsim_amd as tms
+    Q, D, lens, offsets = _docs(70, d=64)
+    pq = tms.TileMaxSimPQ(torch.randn(8, 16, 8, device="cuda").half())
+    codes = torch.randint(0, 16, (30, 20, 8), device="cuda", dtype=torch.int32)
+    calls = [lambda: tms.flash_maxsim_multi_doc(Q, D, offsets), lambda: tms.flashmaxsim_score_packed(Q, D, lens),
+             lambda: tms.flash_maxsim_multi_doc_batched(torch.stack([Q, Q, Q]), D, offsets),
+             lambda: pq.score_batch(Q, codes)]
+    want = [c() for c in calls]
+    got, bad = [], offsets.clone()
+    bad[3] = -1
+
+    def work():
+        for dev in ("cuda", "cpu"):
+            with torch.device(dev):
+                got.append([c() for c in calls])
+                with pytest.raises(ValueError):
+                    tms.flash_maxsim_multi_doc(Q, D, bad)
+
+    t = threading.Thread(target=work)
+    t.start()
+    t.join()
+    assert len(got) == 2 and all(_same(a, b) for g in got for a, b in zip(g, want))
+
+
 def test_capture_is_refused(cuda):
     import torch
     import tilemaxsim_amd as tms

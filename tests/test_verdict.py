@@ -91,3 +91,30 @@ def test_verdict_words_do_not_follow_the_default_device(monkeypatch):
             assert _lib.verdict_ptr() != 0
     finally:
         vars(_lib._thread).pop("verdict", None)  # made without pinning
+
+
+def test_parts_are_a_thread_s_own_and_follow_its_stream(monkeypatch):
+    """One buffer a thread, for the stream and device that it last used: calls of two threads,
+    or on two streams, never share one."""
+    import threading
+    dev = torch.device("cpu")
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    vars(_lib._thread).pop("parts", None)
+    first = _lib.parts_ptr(dev, 16)
+    assert first != 0 and _lib.parts_ptr(dev, 16) == first
+    held = _lib._thread.parts  # alive, so that its memory is not given out again
+    seen = []
+
+    def other():
+        seen.append((_lib.parts_ptr(dev, 16), _lib._thread.parts))
+
+    t = threading.Thread(target=other)
+    t.start()
+    t.join()
+    assert seen[0][0] != first and _lib.parts_ptr(dev, 16) == first
+    assert _lib.parts_ptr(dev, 32) != first and _lib._thread.parts is not held
+    assert _lib.parts_ptr(torch.device("meta"), 32) == 0  # another device: its own buffer
+    vars(_lib._thread).pop("parts", None)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    _lib.parts_ptr(dev, 48)  # under capture: nothing is kept
+    assert not hasattr(_lib._thread, "parts")

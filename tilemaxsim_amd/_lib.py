@@ -151,6 +151,21 @@ def verdict_ptr() -> int:
     return v.data_ptr()
 
 
+def parts_ptr(dev: torch.device, stream: int) -> int:
+    """Address of the words in which a check on ``stream`` (torch's current one on ``dev``) tells
+    the scoring kernels behind it what it found. A thread keeps one such buffer, for the
+    stream that it last used: an allocation is a tenth of a small call. Kernels on the stream
+    use it in turn, and it goes back to torch's allocator, under that stream, when the thread
+    turns to another one or ends. Not for a captured call, whose kernels outlive its turn."""
+    kept = getattr(_thread, "parts", None)
+    if kept is None or kept[0] != stream or kept[1] != dev:
+        words = torch.empty(TMS_CHECK_PARTS, dtype=torch.int64, device=dev)
+        kept = (stream, dev, words.data_ptr(), words)
+        if not torch.cuda.is_current_stream_capturing():  # a checked call there is refused; nothing of its pool is kept
+            _thread.parts = kept
+    return kept[2]
+
+
 def check_bounds(status: int, msg: str) -> None:
     """:func:`check`, with ``msg`` for the bounds a ``*_checked`` call refused."""
     if status == TMS_ERR_BOUNDS:

@@ -311,7 +311,7 @@ int tms_maxsim_varlen_checked(const void* Qs, int64_t nQ, int64_t nq, int64_t d,
   rc = check_launched("docs_check_kernel", verdict, st);
   if (rc) return rc;
   if (verdict && !parts && (rc = wait_verdict(fn, verdict, tag, g, st))) return refuse(fn, rc);
-  rc = varlen_scores(fn, Qs, nQ, nq, d, D_flat, total_tokens, offsets, B, PadLen{0, parts, g}, dtype, out, stream);
+  rc = varlen_scores(fn, Qs, nQ, nq, d, D_flat, total_tokens, offsets, B, PadLen{0, parts, g, zero_pad != 0}, dtype, out, stream);
   return close_verdict(fn, verdict, tag, g, st, rc);
 }
 
@@ -331,7 +331,7 @@ int tms_maxsim_packed_checked(const void* Q, int64_t nq, int64_t d, const void* 
   rc = check_launched("lengths_scan_kernel", verdict, st);
   if (rc) return rc;
   if (verdict && !parts && (rc = wait_verdict(fn, verdict, tag, 1, st))) return refuse(fn, rc);
-  rc = varlen_scores(fn, Q, 1, nq, d, D_packed, total_tokens, offsets, B, PadLen{0, parts, 1}, dtype, out, stream);
+  rc = varlen_scores(fn, Q, 1, nq, d, D_packed, total_tokens, offsets, B, PadLen{0, parts, 1, zero_pad != 0}, dtype, out, stream);
   return close_verdict(fn, verdict, tag, 1, st, rc);
 }
 
@@ -356,7 +356,7 @@ int tms_maxsim_residual_checked(const void* Qs, int64_t nQ, int64_t nq, int64_t 
   if (rc) return rc;
   if (verdict && !parts && (rc = wait_verdict(fn, verdict, tag, g, st))) return refuse(fn, rc);
   rc = residual_scores(fn, Qs, nQ, nq, d, centroids, ncent, bucket_weights, nbits, codes, residuals, total_tokens, offsets,
-                       ndocs, pids, B, PadLen{0, parts, g}, batched != 0, out, stream);
+                       ndocs, pids, B, PadLen{0, parts, g, zero_pad != 0}, batched != 0, out, stream);
   return close_verdict(fn, verdict, tag, g, st, rc);
 }
 

@@ -263,12 +263,13 @@ struct DocEnd {
 };
 
 // The zero-padding length of a call (0: none): a number, or the largest of up to 64 numbers
-// that a check kernel earlier on the stream left in device memory, one a workgroup; a negative
-// one says that the call is refused.
+// that a check kernel earlier on the stream left in device memory, one a workgroup (`longest`);
+// a negative one says that the call is refused.
 struct PadLen {
   int64_t len;
   const int64_t* parts;
   int32_t nparts;
+  int32_t longest;
 };
 // A lane's one of the numbers: read ahead of a wave's other first loads and used by the two
 // functions below after them, so that the wave waits for memory once.
@@ -276,7 +277,7 @@ __device__ __forceinline__ int64_t pad_part(const PadLen& p, int lane) {
   return p.parts != nullptr && lane < p.nparts ? p.parts[lane] : 0;
 }
 __device__ __forceinline__ int64_t pad_length(const PadLen& p, int64_t part) {
-  if (p.parts == nullptr) return p.len;  // uniform
+  if (p.longest == 0) return p.len;  // uniform
   int64_t m = part;
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) {

@@ -95,7 +95,7 @@ static int pick_docs_per_wave(int64_t B, int64_t tokens_per_doc_hint, bool f32, 
 
 static int dense_entry(const char* fn, const void* Q, int64_t nQ, int64_t nq, int64_t d, const void* D, int64_t B,
                        int64_t nd, int64_t total_tokens, const int64_t* offsets, const uint8_t* mask, int mode,
-                       int dtype, float* out, void* stream, PadLen pad = PadLen{0, nullptr, 0}) {
+                       int dtype, float* out, void* stream, PadLen pad = PadLen{0, nullptr, 0, 0}) {
   const bool q32 = (dtype & TMS_QUERY_F32) != 0;  // fp32 queries (implied for fp32 documents)
   dtype &= ~TMS_QUERY_F32;
   if (dtype != TMS_DTYPE_F16 && dtype != TMS_DTYPE_BF16 && dtype != TMS_DTYPE_F32)
@@ -207,14 +207,14 @@ int tms_maxsim_varlen(const void* Q, int64_t nq, int64_t d, const void* D_flat, 
 int tms_maxsim_varlen_padded(const void* Q, int64_t nq, int64_t d, const void* D_flat, int64_t total_tokens,
                              const int64_t* offsets, int64_t B, int64_t pad_len, int dtype, float* out, void* stream) {
   return tms::dense_entry("tms_maxsim_varlen_padded", Q, 1, nq, d, D_flat, B, 0, total_tokens, offsets, nullptr,
-                          tms::MODE_VARLEN, dtype, out, stream, tms::PadLen{pad_len, nullptr, 0});
+                          tms::MODE_VARLEN, dtype, out, stream, tms::PadLen{pad_len, nullptr, 0, 0});
 }
 
 int tms_maxsim_varlen_batched(const void* Qs, int64_t nQ, int64_t nq, int64_t d, const void* D_flat,
                               int64_t total_tokens, const int64_t* offsets, int64_t B, int64_t pad_len, int dtype,
                               float* out, void* stream) {
   return tms::dense_entry("tms_maxsim_varlen_batched", Qs, nQ, nq, d, D_flat, B, 0, total_tokens, offsets, nullptr,
-                          tms::MODE_VARLEN, dtype, out, stream, tms::PadLen{pad_len, nullptr, 0});
+                          tms::MODE_VARLEN, dtype, out, stream, tms::PadLen{pad_len, nullptr, 0, 0});
 }
 
 int tms_maxsim_dense_batched(const void* Qs, int64_t nQ, int64_t nq, int64_t d, const void* D, int64_t B, int64_t nd,

@@ -1109,7 +1109,7 @@ int tms_maxsim_residual(const void* Q, int64_t nq, int64_t d, const void* centro
                         int64_t total_tokens, const int64_t* offsets, int64_t ndocs, const int64_t* pids, int64_t B,
                         int64_t pad_len, float* out, void* stream) {
   return tms::residual_scores("tms_maxsim_residual", Q, 1, nq, d, centroids, ncent, bucket_weights, nbits, codes,
-                              residuals, total_tokens, offsets, ndocs, pids, B, tms::PadLen{pad_len, nullptr, 0}, false,
+                              residuals, total_tokens, offsets, ndocs, pids, B, tms::PadLen{pad_len, nullptr, 0, 0}, false,
                               out, stream);
 }
 
@@ -1119,7 +1119,7 @@ int tms_maxsim_residual_batched(const void* Qs, int64_t nQ, int64_t nq, int64_t 
                                 const int64_t* pids, int64_t B, int64_t pad_len, float* out, void* stream) {
   return tms::residual_scores("tms_maxsim_residual_batched", Qs, nQ, nq, d, centroids, ncent, bucket_weights, nbits,
                               codes, residuals, total_tokens, offsets, ndocs, pids, B,
-                              tms::PadLen{pad_len, nullptr, 0}, true, out, stream);
+                              tms::PadLen{pad_len, nullptr, 0, 0}, true, out, stream);
 }
 
 }  // extern "C"

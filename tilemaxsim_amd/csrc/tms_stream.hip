@@ -447,7 +447,7 @@ int run_stream(const void* Q, int64_t nQ, int64_t nq, int64_t d, const void* D, 
   a.d = (int32_t)d;
   const int64_t nblocks = nQ * (int64_t)a.nbq;
   if (!offsets && !mask && a.nbq <= 4 && (nblocks >= 4 || nQ == 3))  // batched: documents at implicit offsets b * nd
-    return run_varlen_batched(Q, nQ, nq, d, D, B * nd, nullptr, nd, B, PadLen{0, nullptr, 0}, dtype, out, st, false);
+    return run_varlen_batched(Q, nQ, nq, d, D, B * nd, nullptr, nd, B, PadLen{0, nullptr, 0, 0}, dtype, out, st, false);
   const int64_t hint = offsets ? (B > 0 ? T / B : 1) : nd;  // tokens per document
   int64_t dpw = hint > 0 ? TMS_STREAM_TOKENS_PER_WAVE / hint : 1;
   const int64_t min_waves = TMS_STREAM_MIN_WAVES;

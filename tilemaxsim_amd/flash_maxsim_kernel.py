@@ -96,10 +96,11 @@ def flash_maxsim_multi_doc(Q: torch.Tensor, D_flat: torch.Tensor, doc_offsets: t
     lib = _lib.load()
     with _lib.on_device(Q.device):
         if validate:  # the check runs on the device before the scoring kernel; its verdict is waited for
-            parts = torch.empty(_lib.TMS_CHECK_PARTS, dtype=torch.int64, device=Q.device)
+            stream = _lib.stream_of(Q)
             _lib.check_bounds(
                 lib.tms_maxsim_varlen_checked(Q.data_ptr(), 1, Nq, d, D_flat.data_ptr(), T, offsets.data_ptr(), num_docs, 0,
-                                              code, scores.data_ptr(), parts.data_ptr(), _lib.verdict_ptr(), _lib.stream_of(Q)),
+                                              code, scores.data_ptr(), _lib.parts_ptr(Q.device, stream), _lib.verdict_ptr(),
+                                              stream),
                 "flash_maxsim_multi_doc: doc_offsets must be non-decreasing within [0, total_tokens]")
             return scores
         _lib.check(lib.tms_maxsim_varlen(Q.data_ptr(), Nq, d, D_flat.data_ptr(), T, offsets.data_ptr(), num_docs,
@@ -135,11 +136,11 @@ def _varlen_batched(fn: str, Qs: torch.Tensor, D_flat: torch.Tensor, doc_offsets
     lib = _lib.load()
     with _lib.on_device(Qs.device):
         if validate or zero_pad:
-            parts = torch.empty(_lib.TMS_CHECK_PARTS, dtype=torch.int64, device=Qs.device)
+            stream = _lib.stream_of(Qs)
             _lib.check_bounds(
                 lib.tms_maxsim_varlen_checked(Qs.data_ptr(), nQ, Nq, d, D_flat.data_ptr(), T, offsets.data_ptr(), B,
-                                              int(zero_pad), code, out.data_ptr(), parts.data_ptr(), _lib.verdict_ptr(),
-                                              _lib.stream_of(Qs)),
+                                              int(zero_pad), code, out.data_ptr(), _lib.parts_ptr(Qs.device, stream),
+                                              _lib.verdict_ptr(), stream),
                 f"{fn}: doc_offsets must be non-decreasing within [0, total_tokens]")
             return out
         _lib.check(lib.tms_maxsim_varlen_batched(Qs.data_ptr(), nQ, Nq, d, D_flat.data_ptr(), T, offsets.data_ptr(), B,

@@ -81,21 +81,21 @@ def flashmaxsim_score_packed(Q: torch.Tensor, D_packed: torch.Tensor, D_lengths:
         return scores
     # the lengths' sums, their checks and the longest one (the zero padding's length) are
     # taken on the device, before the scoring kernel that uses them
-    parts = torch.empty(_lib.TMS_CHECK_PARTS, dtype=torch.int64, device=dev)
     scan = B <= _lib.TMS_PACKED_SCAN_MAX  # longer lists: torch's prefix sum
     lengths = D_lengths.to(device=dev, dtype=torch.int64).contiguous()
     offsets = torch.empty(B + 1, dtype=torch.int64, device=dev) if scan else lengths_to_offsets(lengths, dev)
     lib = _lib.load()
     with _lib.on_device(dev):
+        stream = _lib.stream_of(Q2)
+        parts, verdict = _lib.parts_ptr(dev, stream), _lib.verdict_ptr()
         if scan:
             status = lib.tms_maxsim_packed_checked(Q2.data_ptr(), Q2.shape[0], d, D_packed.data_ptr(), T,
                                                    lengths.data_ptr(), B, 1, _lib.TMS_DTYPE_F16, scores.data_ptr(),
-                                                   offsets.data_ptr(), parts.data_ptr(), _lib.verdict_ptr(),
-                                                   _lib.stream_of(Q2))
+                                                   offsets.data_ptr(), parts, verdict, stream)
         else:
             status = lib.tms_maxsim_varlen_checked(Q2.data_ptr(), 1, Q2.shape[0], d, D_packed.data_ptr(), T,
                                                    offsets.data_ptr(), B, 1, _lib.TMS_DTYPE_F16, scores.data_ptr(),
-                                                   parts.data_ptr(), _lib.verdict_ptr(), _lib.stream_of(Q2))
+                                                   parts, verdict, stream)
         _lib.check_bounds(status,
                           "flashmaxsim_score_packed: D_lengths must be >= 0 and sum to at most D_packed.shape[0]")
     return scores

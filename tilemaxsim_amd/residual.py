@@ -105,16 +105,20 @@ def _score(fn: str, Qs, nQ: int, Nq: int, d: int, batched: bool, index, offsets,
     waited for."""
     codes, residuals, centroids, bucket_weights, nbits = index
     zeros = padding == "zeros"
-    parts = torch.empty(_lib.TMS_CHECK_PARTS, dtype=torch.int64, device=out.device) if validate or zeros else None
     lib = _lib.load()
     with _lib.on_device(out.device):
         args = (Nq, d, centroids.data_ptr(), centroids.shape[0], bucket_weights.data_ptr(), nbits, codes.data_ptr(),
                 residuals.data_ptr(), codes.shape[0], offsets.data_ptr(), ndocs, _lib.ptr(pids), B)
         stream = _lib.stream_of(out)
         if validate or zeros:
+            if validate:
+                parts, verdict = _lib.parts_ptr(out.device, stream), _lib.verdict_ptr()
+            else:  # nothing is waited for: also a captured call's, whose words are its own
+                words = torch.empty(_lib.TMS_CHECK_PARTS, dtype=torch.int64, device=out.device)
+                parts, verdict = words.data_ptr(), None
             _lib.check_bounds(
-                lib.tms_maxsim_residual_checked(Qs.data_ptr(), nQ, *args, int(zeros), int(batched), out.data_ptr(),
-                                                _lib.ptr(parts), _lib.verdict_ptr() if validate else None, stream),
+                lib.tms_maxsim_residual_checked(Qs.data_ptr(), nQ, *args, int(zeros), int(batched), out.data_ptr(), parts,
+                                                verdict, stream),
                 f"{fn}: doc_offsets must be non-decreasing within [0, T] and pids within [0, ndocs)")
         elif batched:
             _lib.check(lib.tms_maxsim_residual_batched(Qs.data_ptr(), nQ, *args, 0, out.data_ptr(), stream))
