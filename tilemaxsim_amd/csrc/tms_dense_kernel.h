@@ -170,7 +170,13 @@ __global__ void __launch_bounds__(NT, 1) dense_maxsim_kernel(DenseArgs a) {
   };
 
   const int64_t pad = MODE == MODE_VARLEN ? pad_part(a.pad, lane) : 0;
-  const int64_t pad_len = MODE == MODE_VARLEN ? pad_length(a.pad, pad) : 0;
+  // fp32 rows with the query in memory fill the registers: found anew at each document's end there
+  constexpr bool PAD_ANEW = MODE == MODE_VARLEN && QGLB && DT == TMS_DTYPE_F32;
+  const int64_t pad_once = MODE == MODE_VARLEN && !PAD_ANEW ? pad_length(a.pad, pad) : 0;
+  auto padding = [&]() -> int64_t {
+    if constexpr (PAD_ANEW) return pad_length(a.pad, pad_part(a.pad, lane));
+    else return pad_once;
+  };
   const bool refuse = MODE == MODE_VARLEN && refused(pad);
 
   // Query blocks of this launch: [my_blk0, my_blk0 + my_nblk).
@@ -360,7 +366,7 @@ __global__ void __launch_bounds__(NT, 1) dense_maxsim_kernel(DenseArgs a) {
       }
       // an empty document zero-padded to pad_len > 0 tokens has every max equal to 0
       if (bad) write_bad(b);
-      else write_empty(b, pad_len > 0 ? 0.f : NEG_INF);
+      else write_empty(b, padding() > 0 ? 0.f : NEG_INF);
     }
     c.b = b_end;
   };
@@ -494,7 +500,7 @@ __global__ void __launch_bounds__(NT, 1) dense_maxsim_kernel(DenseArgs a) {
   auto finish = [&](int64_t b, int64_t len, auto combine) {
     constexpr bool COMBINE = decltype(combine)::value;
     // zero padding up to pad_len adds dot products equal to 0 to a shorter document
-    const bool padded = (MODE == MODE_VARLEN) && len < pad_len;
+    const bool padded = (MODE == MODE_VARLEN) && len < padding();
     float blk[NQB];
 #pragma unroll
     for (int j = 0; j < NQB; j++) {
