@@ -793,8 +793,11 @@ __device__ __forceinline__ void residual_batched_body(const ResArgs& a, ResShare
   }
 }
 
+// Waves per SIMD the registers are budgeted for, which for W = 4 are workgroups per CU.
+constexpr int residual_min_waves(int W, int NBX) { return W == 8 || NBX > 2 ? 2 : (NBX == 2 ? 3 : 4); }
+
 template <int KS, int NBITS, int NBL, int NBX, int W>
-__global__ void __launch_bounds__(64 * W, W == 8 || NBX > 2 ? 2 : (NBX == 2 ? 3 : 4)) residual_batched_kernel(ResArgs a) {
+__global__ void __launch_bounds__(64 * W, residual_min_waves(W, NBX)) residual_batched_kernel(ResArgs a) {
   __shared__ __attribute__((aligned(16))) ResShared sh;
   build_lut<NBITS>(sh.lut, a.weights);  // a barrier before the first decode
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1042,8 +1045,7 @@ static int residual_many(const char* fn, const void* Qs, int64_t nQ, int64_t nq,
     a.blk_end = (int32_t)(q1 * a.nbq);
     a.nblk_l = kBatchedForms[f].NBL / a.nbq * a.nbq;
     a.nblk_x = kBatchedForms[f].NBX / a.nbq * a.nbq;
-    const int per_cu = kBatchedForms[f].W == 8 || kBatchedForms[f].NBX > 2 ? (kBatchedForms[f].W == 8 ? 1 : 2)
-                                                                         : (kBatchedForms[f].NBX == 2 ? 3 : 4);
+    const int per_cu = kBatchedForms[f].W == 8 ? 1 : residual_min_waves(4, kBatchedForms[f].NBX);
     a.docs_per_wave = (int32_t)batched_docs_per_wg(B, hint, true, 256 * per_cu);
     const int64_t grid = (B + a.docs_per_wave - 1) / a.docs_per_wave;
     if (grid > 0x7fffffff) return fail(TMS_ERR_UNSUPPORTED, "%s: too many documents", fn);
