@@ -117,3 +117,26 @@ def test_residual_bits(cuda, nQ, nq, d, nbits):
     for q in {0, nQ // 2, nQ - 1}:
         two = tms.flashmaxsim_score_residual_batched(torch.stack([Qs[q], Qs[0]]), *index)[0]
         assert torch.equal(got[q].view(torch.int32), two.view(torch.int32)), f"query {q}"
+
+
+@pytest.mark.parametrize("dt", ["float16", "bfloat16", "float32"])
+@pytest.mark.parametrize("d", [128, 96, 64, 32])
+def test_few_documents(cuda, d, dt):
+    """Up to 256 documents the blocks go over eight waves: the bits of the call of 257, whose
+    blocks go over four, and (16-bit rows) of the one-query kernels."""
+    import torch
+    import tilemaxsim_amd as tms
+    rng = np.random.default_rng(d)
+    lens = rng.integers(0, 50, 257)
+    lens[0], lens[255] = 49, 0
+    offsets = torch.from_numpy(np.concatenate([[0], np.cumsum(lens)])).cuda()
+    D = torch.from_numpy(_emb(rng, int(lens.sum()), d)).to(getattr(torch, dt)).cuda()
+    for nQ, nq in ((5, 32), (8, 20), (9, 32), (13, 32), (16, 32), (17, 32), (3, 64), (4, 40), (8, 64), (2, 96), (5, 96)):
+        Qs = torch.from_numpy(_emb(rng, nQ, nq, d)).to(getattr(torch, dt)).cuda()
+        many = tms.flash_maxsim_multi_doc_batched(Qs, D, offsets)
+        for B in (256, 65, 1):
+            few = tms.flash_maxsim_multi_doc_batched(Qs, D, offsets[:B + 1])
+            assert torch.equal(few.view(torch.int32), many[:, :B].contiguous().view(torch.int32)), (nQ, nq, B)
+        if dt != "float32":
+            one = torch.stack([tms.flash_maxsim_multi_doc(q, D, offsets) for q in Qs])
+            assert torch.equal(many.view(torch.int32), one.view(torch.int32)), (nQ, nq)

@@ -17,6 +17,7 @@
 //  * W = 4 waves of NB = 1..4 blocks, two to four workgroups per CU, for up to 4 NB blocks;
 //  * W = 8 waves, one workgroup per CU, above that: NBL blocks in each of waves 0-3 and NBX
 //    in each of waves 4-7 (waves w and w + 4 share a SIMD), up to 4 (NBL + NBX) blocks.
+// Calls of few documents take W = 8 for 5 to 16 blocks as well (batched_spread).
 // 50,000 x 180 tokens, d = 128 fp16, for 4, 8, 16, 20, 24, 32 and 34 queries: 418, 583, 918,
 // 1250, 1408, 1761 and 2160 us (1.34 PFLOP/s at 32), against 605, 656, 1136, 1670, 1750, 1848
 // and 3523 with 8 waves of 1, 2 or 4 blocks for every pass.
@@ -24,6 +25,7 @@
 #include <string.h>
 
 #include "tms_common.h"
+#include "tms_rules.h"
 
 namespace tms {
 
@@ -422,6 +424,8 @@ struct BatchedForm {
 };
 constexpr BatchedForm kBatchedForms[] = {{4, 1, 1}, {4, 2, 2}, {4, 3, 3}, {4, 4, 4}, {8, 2, 3}, {8, 3, 3}, {8, 3, 4}, {8, 4, 4}};
 constexpr BatchedForm kBatchedFormsQ32[] = {{4, 1, 1}, {4, 2, 2}, {8, 1, 2}, {8, 2, 2}};  // twice the registers a block
+// For calls of few documents (batched_spread), the passes of 5 to 16 blocks.
+constexpr BatchedForm kBatchedSpreadForms[] = {{8, 1, 1}, {8, 2, 2}};
 
 // Blocks a form holds when every query takes nbq blocks (a wave holds whole queries).
 static inline int64_t form_blocks(const BatchedForm& f, int nbq) {
@@ -439,8 +443,13 @@ static int batched_ks(const BatchedArgs& a, int64_t grid, size_t lds, hipStream_
   }
   return check_launch("batched_tile_kernel");
 }
+// Form f of the list (Q32's for fp32 queries), or spread form -1 - f.
 template <int DT, class SRC>
 static int batched_form(int f, const BatchedArgs& a, int64_t grid, size_t lds, hipStream_t st) {
+  if constexpr (SRC::kDirect) {
+    if (f == -1) return batched_ks<DT, 1, 1, 8, SRC>(a, grid, lds, st);
+    if (f == -2) return batched_ks<DT, 2, 2, 8, SRC>(a, grid, lds, st);
+  }
   if constexpr (SRC::kQ32) {
     switch (f) {
       case 0: return batched_ks<DT, 1, 1, 4, SRC>(a, grid, lds, st);
@@ -498,11 +507,20 @@ static int batched_run(BatchedArgs a, int64_t nQ, int64_t tokens_per_doc, int dt
     const int64_t blocks = (q1 - q0) * a.nbq;
     int f = 0;
     while (f < nf - 1 && form_blocks(forms[f], a.nbq) < blocks) f++;
+    BatchedForm form = forms[f];
+    if (SRC::kDirect && batched_spread(a.B)) {
+      for (int i = 0; i < 2; i++)
+        if (form_blocks(kBatchedSpreadForms[i], a.nbq) >= blocks && kBatchedSpreadForms[i].NBX < form.NBX) {
+          form = kBatchedSpreadForms[i];
+          f = -1 - i;
+          break;
+        }
+    }
     a.blk0 = (int32_t)(q0 * a.nbq);
     a.blk_end = (int32_t)(q1 * a.nbq);
-    a.nblk_l = forms[f].NBL / a.nbq * a.nbq;
-    a.nblk_x = forms[f].NBX / a.nbq * a.nbq;
-    int64_t per_cu = forms[f].W == 8 ? 1 : batched_min_waves<SRC>(4, forms[f].NBX);
+    a.nblk_l = form.NBL / a.nbq * a.nbq;
+    a.nblk_x = form.NBX / a.nbq * a.nbq;
+    int64_t per_cu = form.W == 8 ? 1 : batched_min_waves<SRC>(4, form.NBX);
     const int64_t fit = (160 * 1024) / (int64_t)(sizeof(BatchedRing<SRC>) + lds);
     if (per_cu > fit) per_cu = fit;
     a.docs_per_wg = (int32_t)batched_docs_per_wg(a.B, tokens_per_doc, a.offsets != nullptr, 256 * per_cu);

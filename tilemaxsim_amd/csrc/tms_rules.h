@@ -35,6 +35,14 @@ inline int dense_split_waves(int64_t B, int64_t tiles, size_t lds, int nqb, int 
   return w;
 }
 
+// Whether batched queries over B documents spread their blocks over eight waves, one or two
+// blocks each (tms_batched_kernel.h), rather than over four of up to four. Up to one document
+// a CU, each workgroup has a CU to itself and walks its document as fast as one wave's step
+// goes; above, two to four workgroups of four waves a CU do more than one of eight. d = 128,
+// 1,000 tokens, 6 queries, over four / eight waves: 50 documents fp16 1 / 0.80, fp32 1 / 0.74; 256
+// documents 1 / 0.85 and 0.80; 300 documents 1 / 1.37 and 1.20.
+inline bool batched_spread(int64_t B) { return B <= 256; }
+
 // Whether a batched PQ call (nQ queries of nbq blocks, `tokens` of them, M codes of dsub
 // dimensions a token, a codebook of `lds` bytes) goes query by query. One pass of the
 // shared-tile workgroups waits on each tile's gathers whatever the queries are, so a few
