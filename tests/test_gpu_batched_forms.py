@@ -1,7 +1,8 @@
 """GPU parity of the shared-tile kernel's workgroup forms (``tms_batched_kernel.h``).
 
 A call of n query blocks takes passes of up to 32 blocks (16 for fp32 queries), each in the
-smallest form that holds it: 4 waves of 1-4 blocks, or 8 waves of 2-4. Cases sit on both
+smallest form that holds it: 4 waves of 1-4 blocks, or 8 waves of 2-4 (up to 256 documents
+also 8 waves of 1 or 2 for 5 to 16 blocks). Cases sit on both
 sides of every form's capacity, at queries of one to four blocks, with document counts on
 both sides of one workgroup and of a round of them. Dense scores must be the bits of the
 one-query kernels (the same products, and the same order of the sums over query tokens);
@@ -26,7 +27,7 @@ def _emb(rng, *shape):
     return x / np.linalg.norm(x, axis=-1, keepdims=True)
 
 
-@pytest.mark.parametrize("d,B", [(128, 130), (96, 1), (64, 65), (32, 1100)])
+@pytest.mark.parametrize("d,B", [(128, 130), (96, 1), (64, 65), (32, 1100), (128, 300), (96, 257), (64, 400)])
 @pytest.mark.parametrize("nQ,nq", FORMS)
 def test_dense_bits(cuda, nQ, nq, d, B):
     import torch
@@ -119,9 +120,10 @@ def test_residual_bits(cuda, nQ, nq, d, nbits):
         assert torch.equal(got[q].view(torch.int32), two.view(torch.int32)), f"query {q}"
 
 
-@pytest.mark.parametrize("dt", ["float16", "bfloat16", "float32"])
+@pytest.mark.parametrize("qdt,dt", [("float16", "float16"), ("bfloat16", "bfloat16"), ("float32", "float32"),
+                                    ("float32", "float16"), ("float32", "bfloat16")])
 @pytest.mark.parametrize("d", [128, 96, 64, 32])
-def test_few_documents(cuda, d, dt):
+def test_few_documents(cuda, d, qdt, dt):
     """Up to 256 documents the blocks go over eight waves: the bits of the call of 257, whose
     blocks go over four, and (16-bit rows) of the one-query kernels."""
     import torch
@@ -132,11 +134,11 @@ def test_few_documents(cuda, d, dt):
     offsets = torch.from_numpy(np.concatenate([[0], np.cumsum(lens)])).cuda()
     D = torch.from_numpy(_emb(rng, int(lens.sum()), d)).to(getattr(torch, dt)).cuda()
     for nQ, nq in ((5, 32), (8, 20), (9, 32), (13, 32), (16, 32), (17, 32), (3, 64), (4, 40), (8, 64), (2, 96), (5, 96)):
-        Qs = torch.from_numpy(_emb(rng, nQ, nq, d)).to(getattr(torch, dt)).cuda()
+        Qs = torch.from_numpy(_emb(rng, nQ, nq, d)).to(getattr(torch, qdt)).cuda()
         many = tms.flash_maxsim_multi_doc_batched(Qs, D, offsets)
         for B in (256, 65, 1):
             few = tms.flash_maxsim_multi_doc_batched(Qs, D, offsets[:B + 1])
             assert torch.equal(few.view(torch.int32), many[:, :B].contiguous().view(torch.int32)), (nQ, nq, B)
-        if dt != "float32":
+        if qdt != "float32":
             one = torch.stack([tms.flash_maxsim_multi_doc(q, D, offsets) for q in Qs])
             assert torch.equal(many.view(torch.int32), one.view(torch.int32)), (nQ, nq)
